@@ -78,6 +78,10 @@ int64_t dspark_attn_workspace_bytes(int n_req, int64_t key_rows_bound, int row_t
  *   [n_groups + 1] run ranges: run w holds records range[w] .. range[w+1]
  *   [n_req][4] request records: first partial slot, segment count,
  *       first query row, query length
+ * Requests with more than 8 query tokens (in a call whose max_q exceeds 8)
+ * are attended by workgroups of their own, one per (record, KV head, 32 query
+ * tokens): their records may stand in any run or, after the last run's
+ * records, in none (records with query length 0 are skipped).
  * The segments of a request must cover its keys exactly once, and a split
  * request's segments must use consecutive partial slots in key order (the
  * merge folds them in slot order).  Cuts at the same key positions give

@@ -315,7 +315,13 @@ __device__ __forceinline__ bool chunk_segment(const VarlenArgs& a, bool verify, 
   return true;
 }
 
-// The addressing of one segment for one (KV head, row tile); every field is
+// Requests with more query tokens than this are attended by the prefill
+// workgroups of a launch whose largest request exceeds it: from two
+// 16-row tiles on, one workgroup per tile would stream the keys once per 8
+// tokens.
+constexpr int DECODE_TOKENS = 8;
+
+// The addressing of one segment for one KV head; every field is
 // wave-uniform.  Key j of the request lives in part A (committed rows) for
 // j < a_len, else in part B (rows new to this call).
 struct SegView {
@@ -329,12 +335,14 @@ struct SegView {
   int kend;       // keys [k0, kend) are visible to some row of the tile
   int kfast;      // tiles below kfast need no clamping, source choice or mask
   int q0, ql, kl, pslot;
-  bool live;      // the tile has query rows (8t < ql)
+  bool live;      // the segment has query rows attended here
   bool ends;      // the segment holds the request's last key
 };
 
-template <bool VERIFY>
-__device__ __forceinline__ SegView seg_view(const VarlenArgs& a, const Segment& sg, int g, int t) {
+// MIXED: the launch also has requests that prefill workgroups attend; their
+// segments have no live rows here.
+template <bool VERIFY, bool MIXED>
+__device__ __forceinline__ SegView seg_view(const VarlenArgs& a, const Segment& sg, int g) {
   SegView v;
   // The segment is wave-uniform; say so, so that its fields and everything
   // derived from them stay in scalar registers.
@@ -345,8 +353,8 @@ __device__ __forceinline__ SegView seg_view(const VarlenArgs& a, const Segment& 
   v.k0 = __builtin_amdgcn_readfirstlane(sg.k0);
   const int k1 = __builtin_amdgcn_readfirstlane(sg.k1);
   v.pslot = __builtin_amdgcn_readfirstlane(sg.pslot);
-  v.live = 8 * t < v.ql;
-  v.ends = k1 == v.kl;
+  v.live = v.ql > 0 && (!MIXED || v.ql <= DECODE_TOKENS);
+  v.ends = k1 == v.kl && (!MIXED || v.live);
   if (VERIFY) {
     v.a_len = v.kl - v.ql;
     const size_t abase = (size_t)start * (size_t)a.slot_stride + (size_t)g * a.a_head_stride;
@@ -364,12 +372,12 @@ __device__ __forceinline__ SegView seg_view(const VarlenArgs& a, const Segment& 
     v.vB = v.vA;
     v.bbase = 0;
   }
-  const int last_tok = min(8 * t + 7, v.ql - 1);
+  const int last_tok = min(DECODE_TOKENS - 1, v.ql - 1);
   const int tile_lim = a.causal ? v.kl - v.ql + last_tok + 1 : v.kl;
   v.kend = v.live ? min(k1, tile_lim) : v.k0;
   // Keys below kfast come from part A and are visible to every row of this
   // tile (bottom-right causal: row tok sees keys <= kl - ql + tok).
-  v.kfast = min(min(v.kend, v.a_len), a.causal ? v.kl - v.ql + 8 * t + 1 : v.kl);
+  v.kfast = min(min(v.kend, v.a_len), a.causal ? v.kl - v.ql + 1 : v.kl);
   return v;
 }
 
@@ -426,23 +434,23 @@ __device__ __forceinline__ void load_slow(const VarlenArgs& a, const SegView& s,
 }
 
 // Q of this lane's row of segment s.
-__device__ __forceinline__ void load_q(const VarlenArgs& a, const SegView& s, int g, int t, bf16x8 (&qf)[4]) {
+__device__ __forceinline__ void load_q(const VarlenArgs& a, const SegView& s, int g, bf16x8 (&qf)[4]) {
   const int lane = threadIdx.x & 63;
   const int col = lane & 15;
   const int grp = lane >> 4;
-  const int tok = 8 * t + (col >> 1);
+  const int tok = col >> 1;
   const bool row_ok = tok < s.ql;
   const bf16* qp = a.q + (size_t)(s.q0 + (row_ok ? tok : 0)) * Q_ROW + (size_t)(2 * g + (col & 1)) * HD + 8 * grp;
   #pragma unroll
   for (int ks = 0; ks < 4; ++ks) qf[ks] = row_ok ? ld8(qp + 32 * ks) : zero8();
 }
 
-// One run of segments for one (KV head, row tile): wave w computes tiles
+// One run of segments for one KV head: wave w computes tiles
 // k0 + 32w, k0 + 32(w+4), ... of each segment.
 // fetch(n, sg) yields the run's n-th segment (false past the end); every
 // branch on it is uniform across the workgroup.
-template <bool VERIFY, typename Fetch>
-__device__ __forceinline__ void varlen_run(const VarlenArgs& a, unsigned char* smem, int g, int t, Fetch fetch) {
+template <bool VERIFY, bool MIXED, typename Fetch>
+__device__ __forceinline__ void varlen_run(const VarlenArgs& a, unsigned char* smem, int g, Fetch fetch) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int col = lane & 15;
@@ -456,14 +464,14 @@ __device__ __forceinline__ void varlen_run(const VarlenArgs& a, unsigned char* s
   }
   unsigned char* vs = smem + wave * KT * ROWB;
   unsigned char* kst = smem + (4 + wave) * KT * ROWB;
-  const int tok = 8 * t + (col >> 1);
+  const int tok = col >> 1;
 
   Segment sg;
   if (!fetch(0, sg)) return;
-  SegView cur = seg_view<VERIFY>(a, sg, g, t);
+  SegView cur = seg_view<VERIFY, MIXED>(a, sg, g);
   bf16x8 qf[4];
   for (int n = 0;; ++n) {
-    load_q(a, cur, g, t, qf);
+    load_q(a, cur, g, qf);
     Segment nsg;
     const bool more = fetch(n + 1, nsg);
 
@@ -516,11 +524,11 @@ __device__ __forceinline__ void varlen_run(const VarlenArgs& a, unsigned char* s
       load_slow(a, cur, kt, T);
       compute(T, kt, std::true_type{});
     }
-    // Fused stage: the workgroup holding the request's last segment (row
-    // tile 0) is the only reader of its new rows for KV head g, so it also
+    // Fused stage: the workgroup holding the request's last segment is
+    // the only reader of its new rows for KV head g, so it also
     // copies them into the scratch layer.  The first 256 16-byte pieces are
     // loaded here and stored after the merge, which hides their latency.
-    const bool stage = VERIFY && a.stage_k && cur.ends && t == 0;
+    const bool stage = VERIFY && a.stage_k && cur.ends;
     const int n_stage = 2 * cur.ql * 16;
     auto stage_off = [&](int i, bool& v_half) -> size_t {
       v_half = i >= cur.ql * 16;
@@ -567,10 +575,10 @@ __device__ __forceinline__ void varlen_run(const VarlenArgs& a, unsigned char* s
         #pragma unroll
         for (int i = 0; i < 8; ++i) acc[i] += sc * src[i];
       }
-      const int tok_r = 8 * t + (row >> 1);
+      const int tok_r = row >> 1;
       const int head_r = 2 * g + (row & 1);
       if (cur.pslot >= 0) {
-        const size_t p = (size_t)(cur.pslot * 8 + g) * a.tmax + t;
+        const size_t p = (size_t)(cur.pslot * 8 + g) * a.tmax;
         float* po = a.part_o + (p * 16 + row) * HD + d0;
         *reinterpret_cast<f32x4*>(po) = f32x4{acc[0], acc[1], acc[2], acc[3]};
         *reinterpret_cast<f32x4*>(po + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]};
@@ -595,7 +603,7 @@ __device__ __forceinline__ void varlen_run(const VarlenArgs& a, unsigned char* s
     }
     __syncthreads();   // the next segment reuses the V tiles and the merge buffer
     if (!more) break;
-    cur = seg_view<VERIFY>(a, nsg, g, t);
+    cur = seg_view<VERIFY, MIXED>(a, nsg, g);
   }
 }
 
@@ -633,13 +641,12 @@ __device__ __forceinline__ uint64_t tl_now() { return __builtin_amdgcn_s_memreal
 // Without a list, a persistent grid walks the fixed chunks (item, KV head)
 // with a stride of the grid size, so per-workgroup start-up is paid once
 // per CU slot.
-template <bool VERIFY>
-__global__ __launch_bounds__(256, 2) void varlen_attn_kernel(VarlenArgs a) {
-  __shared__ __attribute__((aligned(16))) unsigned char smem[VARLEN_SMEM];
-  const int slot = blockIdx.x >> 3;
-  const int g = a.work ? (slot & 7) : (blockIdx.x & 7);
+template <bool VERIFY, bool MIXED>
+__device__ __forceinline__ void varlen_workgroup(const VarlenArgs& a, unsigned char* smem, int wid, int grid) {
+  const int slot = wid >> 3;
+  const int g = a.work ? (slot & 7) : (wid & 7);
   if (a.work) {
-    const int run = ((slot >> 3) << 3) | (blockIdx.x & 7);
+    const int run = ((slot >> 3) << 3) | (wid & 7);
     const int32_t* range = a.work + WORK_INTS * a.n_work + run;
     const int b = min(max(range[0], 0), a.n_work);      // clamped: never past the records
     const int e = min(max(range[1], b), a.n_work);
@@ -647,7 +654,7 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_kernel(VarlenArgs a) {
     const uint64_t tl_start = tl_now();
     int tl_keys = 0;
 #endif
-    varlen_run<VERIFY>(a, smem, g, blockIdx.y, [&](int n, Segment& sg) {
+    varlen_run<VERIFY, MIXED>(a, smem, g, [&](int n, Segment& sg) {
       if (b + n >= e) return false;
       const int32_t* w = a.work + WORK_INTS * (b + n);
       sg = Segment{w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7]};
@@ -658,7 +665,6 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_kernel(VarlenArgs a) {
     });
 #ifdef DSPARK_TIMELINE
     const uint64_t tl_end = tl_now();
-    const int wid = blockIdx.x + gridDim.x * blockIdx.y;
     if (threadIdx.x == 0 && wid < TL_WGS) {
       uint32_t hw, xcc;
       asm volatile("s_getreg_b32 %0, hwreg(HW_REG_HW_ID)" : "=s"(hw));
@@ -672,10 +678,16 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_kernel(VarlenArgs a) {
 #endif
     return;
   }
-  varlen_run<VERIFY>(a, smem, g, blockIdx.y, [&](int n, Segment& sg) {
-    const int idx = blockIdx.x + n * gridDim.x;
+  varlen_run<VERIFY, MIXED>(a, smem, g, [&](int n, Segment& sg) {
+    const int idx = wid + n * grid;
     return idx < a.n_slots && chunk_segment(a, VERIFY, idx >> 3, sg);
   });
+}
+
+template <bool VERIFY>
+__global__ __launch_bounds__(256, 2) void varlen_attn_kernel(VarlenArgs a) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem[VARLEN_SMEM];
+  varlen_workgroup<VERIFY, false>(a, smem, blockIdx.x, gridDim.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -1534,6 +1546,431 @@ __global__ __launch_bounds__(DWAVES * WAVE) void draft_attn_kernel(DraftArgs a) 
 }
 
 // ---------------------------------------------------------------------------
+// varlen / verify, requests of more than DECODE_TOKENS query tokens (prompt
+// prefill and chunks of it)
+// ---------------------------------------------------------------------------
+// Workgroup (segment, KV head g, tile t) attends query tokens 32t .. 32t+31
+// of the segment's request over the segment's keys: 4 waves, each with a
+// 32-row tile of 16 tokens x 2 query heads (row n is token n/2, head 2g + n%2)
+// on the draft kernel's 32x32x16 MFMA layout.  Keys and values come through
+// LDS in stages of 64 keys that all waves read.  A tile of at most 16 / 32
+// tokens has RG = 1 / 2 row groups, and the 4/RG waves of a row group divide
+// the 32-key half stages among them round-robin; their states merge through
+// LDS at the end.  Everything a request's bits depend on (tiles, row groups,
+// key order) follows from its own lengths and cuts, never from the batch.
+constexpr int PF_WAVES = 4;
+constexpr int PF_SEGS_Y = 32768;                     // segments per grid plane
+constexpr int PF_TOKENS = 32;                        // query tokens per workgroup
+constexpr int PF_GROUP = 16;                         // query tokens per wave
+constexpr int PF_HALF = DSTEP * ROWB;                // bytes of a stage's K rows, or of its V rows
+constexpr int PF_V = 2 * PF_HALF;                    // two K slots, then two V slots
+constexpr int PF_STATE = (64 + 2) * WAVE * 4;        // bytes of one wave's state in the merge
+constexpr int PF_SMEM = PF_WAVES * PF_STATE;         // the merge space, over the stages
+static_assert(PF_SMEM >= PF_V + 2 * PF_HALF && 2 * PF_SMEM <= 160 * 1024, "two workgroups per CU");
+
+__device__ __forceinline__ void prefill_k(bf16x8 (&kf)[8], uint32_t ka) {
+  #pragma unroll
+  for (int ks = 0; ks < 8; ++ks) kf[ks] = lds_k_frag<false>(ka ^ (32u * ks));
+}
+
+// V^T of PV k-step t, dims 32D .. 32D+31, of the staged V rows at LDS address va.
+__device__ __forceinline__ bf16x8 prefill_v(uint32_t va, int t, int D) {
+  const bf16x4 lo = lds_tr4((va ^ (64u * D)) + 1024u * t);
+  const bf16x4 hi = lds_tr4((va ^ (64u * D) ^ CTX_V1_XOR) + CTX_V1_ADD + 1024u * t);
+  bf16x8 v;
+  #pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    v[i] = lo[i];
+    v[4 + i] = hi[i];
+  }
+  return v;
+}
+
+// Raw scores S^T = K Q^T of a 32-key tile.
+__device__ __forceinline__ f32x16 prefill_scores(const bf16x8 (&qf)[8], const bf16x8 (&kf)[8]) {
+  f32x16 x = {};
+  #pragma unroll
+  for (int ks = 0; ks < 8; ++ks) x = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks], qf[ks], x, 0, 0, 0);
+  return x;
+}
+
+// The running maximum (as pair_tile's, from raw scores); returns the maximum
+// the probabilities are taken against.
+__device__ __forceinline__ float prefill_max(PairState& st, const f32x16& x, float scale_log2) {
+  float mx = x[0];
+  #pragma unroll
+  for (int r = 1; r < 16; ++r) mx = fmaxf(mx, x[r]);
+  // lanes l and l^32 hold the same row
+  const auto both = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, mx), __builtin_bit_cast(uint32_t, mx),
+                                                     false, false);
+  mx = fmaxf(__builtin_bit_cast(float, (uint32_t)both[0]), __builtin_bit_cast(float, (uint32_t)both[1])) * scale_log2;
+  const bool raise = mx > st.m + RESCALE_SLACK;
+  if (__builtin_amdgcn_ballot_w64(raise)) {
+    const float alpha = raise ? fast_exp2(st.m - mx) : 1.0f;
+    st.l *= alpha;
+    #pragma unroll
+    for (int D = 0; D < 4; ++D) st.o[D] *= alpha;
+    st.m = raise ? mx : st.m;
+  }
+  return (st.m == -INFINITY) ? 0.f : st.m;
+}
+
+__device__ __forceinline__ void prefill_probs(PairState& st, const f32x16& x, float m_use, float scale_log2,
+                                              bf16x8 (&pb)[2]) {
+  float ps[2] = {0.f, 0.f};
+  #pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const float p = fast_exp2(__builtin_fmaf(x[r], scale_log2, -m_use));
+    ps[r & 1] += p;
+    pb[r >> 3][r & 7] = (bf16)p;
+  }
+  st.l += ps[0] + ps[1];
+}
+
+// A tile below every row's limit whose scores x are known: its probabilities
+// and output, and the scores of the next tile (K at LDS address ka), whose
+// MFMAs are spread among the exponentials.
+__device__ __forceinline__ f32x16 prefill_full_tile(PairState& st, const bf16x8 (&qf)[8], const f32x16& x, uint32_t ka,
+                                                    uint32_t va, float scale_log2) {
+  bf16x8 kf[8], vt[2][4];
+  prefill_k(kf, ka);
+  #pragma unroll
+  for (int t = 0; t < 2; ++t)
+    #pragma unroll
+    for (int D = 0; D < 4; ++D) vt[t][D] = prefill_v(va, t, D);
+  __builtin_amdgcn_sched_barrier(0);
+  const float m_use = prefill_max(st, x, scale_log2);
+  bf16x8 pb[2];
+  const f32x16 nx = prefill_scores(qf, kf);
+  prefill_probs(st, x, m_use, scale_log2, pb);
+  #pragma unroll
+  for (int t = 0; t < 2; ++t)
+    #pragma unroll
+    for (int D = 0; D < 4; ++D)
+      st.o[D] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vt[t][D], pb[t], st.o[D], 0, 0, 0);
+  #pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // a score MFMA,
+    __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);   // then two keys' worth of VALU
+  }
+  __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+  return nx;
+}
+
+// A tile that some rows see in part or not at all (`lim`: the lane's limit in
+// staged rows).  In PV the lane's rows below 16 take the V rows below lim0 and
+// the others those below lim1, every other V row counting as zero, in two
+// passes of which each row keeps its own: a probability of zero times an
+// infinite or NaN V row past a row's limit would otherwise reach the row.
+__device__ __forceinline__ void prefill_edge_tile(PairState& st, f32x16 x, uint32_t va, int lim, int lim0, int lim1,
+                                                  float scale_log2) {
+  #pragma unroll
+  for (int r = 0; r < 16; ++r)
+    if (acc_row(r, 0) >= lim) x[r] = -INFINITY;
+  const float m_use = prefill_max(st, x, scale_log2);
+  bf16x8 pb[2];
+  prefill_probs(st, x, m_use, scale_log2, pb);
+  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x & 63;
+  #pragma unroll 1
+  for (int half = 0; half < 2; ++half) {
+    const int lim_h = half ? lim1 : lim0;
+    const bool mine = ((lane >> 4) & 1) == half;
+    #pragma unroll
+    for (int D = 0; D < 4; ++D) {
+      f32x16 o = st.o[D];
+      #pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        u32x4_t keep;                       // bf16 pair masks of the V rows below lim_h
+        #pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int row = acc_row(8 * t + 2 * i, lane >> 5);      // and row + 1
+          keep[i] = row + 1 < lim_h ? 0xffffffffu : (row < lim_h ? 0xffffu : 0u);
+        }
+        const bf16x8 v = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4_t, prefill_v(va, t, D)) & keep);
+        o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v, pb[t], o, 0, 0, 0);
+      }
+      #pragma unroll
+      for (int e = 0; e < 16; ++e) st.o[D][e] = mine ? o[e] : st.o[D][e];
+    }
+  }
+}
+
+// Folds the KG states of a row group (`next` floats apart, each [16 quads of
+// four dims][lane][4], then max and sum per lane) and writes quads
+// 16 kg / KG .. of the lane's row: the output, or the FP32 partial in the
+// 8-token tiles the merge kernel reads.
+template <int KG>
+__device__ __forceinline__ void prefill_merge(const VarlenArgs& a, const float* group, int next, int kg, int q0, int tok,
+                                              int ql, int g, int n, int hh, int pslot) {
+  const int lane = threadIdx.x & 63;
+  float m[KG], M = -INFINITY, L = 0.f;
+  #pragma unroll
+  for (int k = 0; k < KG; ++k) {
+    m[k] = group[k * next + 64 * WAVE + lane];
+    M = fmaxf(M, m[k]);
+  }
+  #pragma unroll
+  for (int k = 0; k < KG; ++k) {
+    // a group with no visible key (max -inf) contributes nothing
+    m[k] = m[k] == -INFINITY ? 0.f : fast_exp2(m[k] - M);
+    L += m[k] * group[k * next + 65 * WAVE + lane];
+  }
+  L += __shfl_xor(L, 32);
+  if (tok >= ql) return;
+  const float inv = 1.0f / L;
+  const size_t p = (size_t)(pslot * 8 + g) * a.tmax + (tok >> 3);
+  #pragma unroll
+  for (int i = 0; i < 16 / KG; ++i) {
+    const int quad = kg * (16 / KG) + i;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    #pragma unroll
+    for (int k = 0; k < KG; ++k) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(group + k * next + (quad * WAVE + lane) * 4);
+      #pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] += x[e] * m[k];
+    }
+    const int d = 8 * quad + 4 * hh;
+    if (pslot >= 0) {
+      *reinterpret_cast<f32x4*>(a.part_o + (p * 16 + (n & 15)) * HD + d) = acc;
+    } else {
+      bf16x4 o;
+      #pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = (bf16)(acc[e] * inv);
+      *reinterpret_cast<bf16x4*>(a.out + (size_t)(q0 + tok) * Q_ROW + (size_t)(2 * g + (n & 1)) * HD + d) = o;
+    }
+  }
+  if (pslot >= 0 && kg == 0 && hh == 0) {
+    a.part_ml[(p * 16 + (n & 15)) * 2 + 0] = M;
+    a.part_ml[(p * 16 + (n & 15)) * 2 + 1] = L;
+  }
+}
+
+// A call whose max_q exceeds DECODE_TOKENS is one launch of gridDim.x = 8 x the
+// tiles of max_q: its first `decode_rows` grid rows hold the workgroups that
+// walk the runs for the requests of up to DECODE_TOKENS (they stream from HBM
+// beside the prompts' MFMAs), then one row per segment.  Each request is
+// attended by one of the two forms by its own query count.
+template <bool VERIFY>
+__global__ __launch_bounds__(PF_WAVES * WAVE, 2) void prefill_attn_kernel(VarlenArgs a, int decode_grid, int decode_rows) {
+  // 1 KiB alignment: tile offsets are XORed into LDS addresses.
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[PF_SMEM];
+  static_assert(PF_SMEM >= VARLEN_SMEM && PF_WAVES * WAVE == 256, "one launch shape for both forms");
+  int seg = blockIdx.y + PF_SEGS_Y * blockIdx.z - decode_rows;
+  if (seg < 0) {
+    const int wid = blockIdx.x + gridDim.x * (seg + decode_rows);       // keeps the XCD: gridDim.x is a multiple of 8
+    if (wid < decode_grid) varlen_workgroup<VERIFY, true>(a, smem, wid, decode_grid);
+    return;
+  }
+  const int g = blockIdx.x & 7;
+  const int t = (gridDim.x >> 3) - 1 - (blockIdx.x >> 3);
+  Segment sg;
+  if (a.work) {
+    // from the last record on: a plan puts its prompts after the runs, longest
+    // last, and the empty workgroups of the other records then start behind them
+    seg = a.n_work - 1 - seg;
+    if (seg < 0) return;
+    const int32_t* w = a.work + WORK_INTS * seg;
+    sg = Segment{w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7]};
+  } else if (!chunk_segment(a, VERIFY, seg, sg)) {
+    return;
+  }
+  const int ql = __builtin_amdgcn_readfirstlane(sg.ql);
+  if (ql <= DECODE_TOKENS || PF_TOKENS * t >= ql) return;      // uniform across the workgroup
+  const int q0 = __builtin_amdgcn_readfirstlane(sg.q0);
+  const int kl = __builtin_amdgcn_readfirstlane(sg.kl);
+  const int k0 = __builtin_amdgcn_readfirstlane(sg.k0);
+  const int k1 = __builtin_amdgcn_readfirstlane(sg.k1);
+  const int start = __builtin_amdgcn_readfirstlane(sg.start);
+  const int pslot = __builtin_amdgcn_readfirstlane(sg.pslot);
+  const int n_tok = min(PF_TOKENS, ql - PF_TOKENS * t);
+  const int rg_log2 = n_tok <= PF_GROUP ? 0 : 1;
+  const int kg_count = PF_WAVES >> rg_log2;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int hh = lane >> 5;
+  const int n = lane & 31;
+  const int rg = wave & ((1 << rg_log2) - 1);
+  const int kg = wave >> rg_log2;
+  const int tok0 = PF_TOKENS * t + PF_GROUP * rg;       // the wave's first query token (below ql)
+  const int tok = tok0 + (n >> 1);
+  const bool row_ok = tok < ql;
+  // Keys visible to token x of the request, within this segment.
+  auto limit = [&](int x) { return min(k1, a.causal ? kl - ql + x + 1 : kl); };
+  const int kend = limit(min(PF_TOKENS * t + PF_TOKENS, ql) - 1);      // to any row of the workgroup
+  const int vis = row_ok ? limit(tok) : 0;
+  const int lim0 = limit(min(tok0 + 7, ql - 1));        // to any of the wave's first 8 tokens
+  const int hi = limit(min(tok0 + PF_GROUP, ql) - 1);   // to any row of the wave
+  const int full_lim = min(limit(tok0), hi);            // below: visible to every row
+
+  bf16x8 qf[8];
+  {
+    const bf16* qp = a.q + (size_t)(q0 + (row_ok ? tok : 0)) * Q_ROW + (size_t)(2 * g + (n & 1)) * HD + 8 * hh;
+    #pragma unroll
+    for (int ks = 0; ks < 8; ++ks) qf[ks] = ld8(qp + 16 * ks);
+  }
+
+  // Key j of the request: part A (committed rows) below a_len, else part B.
+  // Wave w loads rows 16w .. 16w+15 of a stage's K and V, 4 rows (1 KiB) per
+  // load: lane L of load i fetches row k = 16w + 4i + L/16 at 16-byte chunk
+  // (L%16) ^ swz(k).
+  const int a_len = VERIFY ? kl - ql : kl;
+  const int64_t b_stride = VERIFY ? KV_ROW : a.a_tok_stride;
+  const size_t abase = VERIFY ? (size_t)start * (size_t)a.slot_stride + (size_t)g * a.a_head_stride
+                              : (size_t)start * KV_ROW + (size_t)g * HD;
+  const size_t bbase = VERIFY ? (size_t)q0 * KV_ROW + (size_t)g * HD : abase;
+  const int row0 = 16 * wave;
+  const uint32_t col[2] = {(uint32_t)(16 * ((lane & 15) ^ swz(row0 + (lane >> 4)))),
+                           (uint32_t)(16 * ((lane & 15) ^ swz(row0 + 8 + (lane >> 4))))};
+  const uint32_t off_a = (uint32_t)((lane >> 4) * a.a_tok_stride * 2);
+  const uint32_t off_b = (uint32_t)((lane >> 4) * b_stride * 2);
+  const uint32_t smem_lds = lds_address(smem);
+  auto issue = [&](int step, bool is_v) {
+    const bf16* pa = (is_v ? a.v_a : a.k_a) + abase;
+    const bf16* pb = (is_v ? a.v_b : a.k_b) + bbase;
+    const uint32_t slot = smem_lds + (is_v ? PF_V : 0) + (uint32_t)((step & 1) * PF_HALF + wave * 4096);
+    const int kt = k0 + step * DSTEP;
+    const bool in_a = kt + DSTEP <= min(a_len, kend);
+    if (in_a || (kt >= a_len && kt + DSTEP <= kend)) {
+      // whole stage in one part: wave-uniform base plus per-lane offset
+      const int64_t stride = in_a ? a.a_tok_stride : b_stride;
+      const bf16* base = (in_a ? pa : pb) + (int64_t)(kt - (in_a ? 0 : a_len) + row0) * stride;
+      const uint32_t off = in_a ? off_a : off_b;
+      #pragma unroll
+      for (int i = 0; i < 4; ++i)
+        lds_dma16_base(base + 4 * i * stride, off + col[i >> 1], __builtin_amdgcn_readfirstlane(slot + 1024u * i));
+    } else {
+      // rows clamped to the last visible key (masked out of the softmax)
+      #pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int kk = min(kt + row0 + 4 * i + (lane >> 4), kend - 1);
+        const bf16* p = kk < a_len ? pa + (int64_t)kk * a.a_tok_stride : pb + (int64_t)(kk - a_len) * b_stride;
+        lds_dma16(reinterpret_cast<const char*>(p) + col[i >> 1], __builtin_amdgcn_readfirstlane(slot + 1024u * i));
+      }
+    }
+  };
+
+  PairState st;
+  st.m = -INFINITY;
+  st.l = 0.f;
+  #pragma unroll
+  for (int D = 0; D < 4; ++D) st.o[D] = f32x16{};
+  const TileOffsets co = ctx_tile_offsets<ROWB>(lane);
+  const int n_steps = kend > k0 ? (kend - k0 + DSTEP - 1) / DSTEP : 0;
+  if (n_steps > 0) {
+    issue(0, false);
+    issue(0, true);
+    if (n_steps > 1) issue(1, false);
+  }
+  // Q completes behind the first stage's loads (the compiler's wait for it
+  // drains them too), so that both round trips overlap.
+  settle(qf[0], qf[1], qf[2], qf[3], qf[4], qf[5], qf[6], qf[7]);
+  #pragma unroll
+  for (int ks = 0; ks < 8; ++ks) qf[ks] = row_ok ? qf[ks] : zero8();
+  settle(qf[0], qf[1], qf[2], qf[3], qf[4], qf[5], qf[6], qf[7]);
+
+  // Half stage 2s + h goes to key group (2s + h) mod kg_count.  Step s takes
+  // V of stage s and forms the scores of stage s + 1, one stage ahead; it
+  // begins once both have landed for every wave (and every wave's LDS reads of
+  // the step before are done), and starts the loads of the next step.
+  const int h = kg & 1;
+  auto turn = [&](int s) { return ((2 * s) & (kg_count - 1)) == (kg & ~1); };
+  auto key0 = [&](int s) { return k0 + s * DSTEP + 32 * h; };
+  auto k_at = [&](int s) { return smem_lds + (uint32_t)((s & 1) * PF_HALF + 32 * h * ROWB) + co.k; };
+  auto v_at = [&](int s) { return smem_lds + (uint32_t)(PF_V + (s & 1) * PF_HALF + 32 * h * ROWB) + co.v; };
+  auto arrive = [&]() {
+    // not before the MFMAs of the step that ends here, which hide the loads
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    asm volatile("s_barrier" ::: "memory");
+  };
+  auto enter = [&](int s) {
+    arrive();
+    if (s + 1 < n_steps) issue(s + 1, true);
+    if (s + 2 < n_steps) issue(s + 2, false);
+  };
+  // Scores of the next stage; past the last stage they are of stale rows and
+  // never used.
+  auto ahead = [&](int s) {
+    bf16x8 kf[8];
+    prefill_k(kf, k_at(s));
+    return prefill_scores(qf, kf);
+  };
+  f32x16 x = {};
+  int s = 0;
+  if (n_steps > 0) {
+    arrive();
+    if (turn(0)) x = ahead(0);
+  }
+  if (kg_count == 2) {
+    // One tile per stage and wave: those below every row's limit first, two
+    // per iteration (no copies of the scores).  The waves of a workgroup may
+    // differ in how many these are; every wave passes one barrier per step.
+    const int span = max(0, full_lim - k0 - 32 * h);
+    const int full = span / DSTEP + (span % DSTEP >= 32 ? 1 : 0);
+    for (; s + 1 < full; s += 2) {
+      enter(s);
+      const f32x16 y = prefill_full_tile(st, qf, x, k_at(s + 1), v_at(s), a.scale_log2);
+      enter(s + 1);
+      x = prefill_full_tile(st, qf, y, k_at(s + 2), v_at(s + 1), a.scale_log2);
+    }
+    if (s < full) {
+      enter(s);
+      x = prefill_full_tile(st, qf, x, k_at(s + 1), v_at(s), a.scale_log2);
+      ++s;
+    }
+  }
+  for (; s < n_steps; ++s) {
+    enter(s);
+    if (turn(s) && key0(s) < hi) {
+      const int kt = key0(s);
+      if (kt + 32 > full_lim) {
+        prefill_edge_tile(st, x, v_at(s), vis - kt - 8 * hh, lim0 - kt, hi - kt, a.scale_log2);
+      } else {
+        const float m_use = prefill_max(st, x, a.scale_log2);
+        bf16x8 pb[2];
+        prefill_probs(st, x, m_use, a.scale_log2, pb);
+        #pragma unroll
+        for (int u = 0; u < 2; ++u)
+          #pragma unroll
+          for (int D = 0; D < 4; ++D)
+            st.o[D] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(prefill_v(v_at(s), u, D), pb[u], st.o[D], 0, 0, 0);
+      }
+    }
+    if (turn(s + 1)) x = ahead(s + 1);
+  }
+  __syncthreads();   // every wave is done with the stages
+
+  // The key groups' states merge with the online-softmax rule: every wave
+  // leaves its state in LDS, then folds and writes its share of the dims.
+  float* mb = reinterpret_cast<float*>(smem + wave * PF_STATE);
+  #pragma unroll
+  for (int D = 0; D < 4; ++D)
+    #pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *reinterpret_cast<f32x4*>(mb + ((4 * D + q) * WAVE + lane) * 4) =
+          f32x4{st.o[D][4 * q], st.o[D][4 * q + 1], st.o[D][4 * q + 2], st.o[D][4 * q + 3]};
+  mb[64 * WAVE + lane] = st.m;
+  mb[65 * WAVE + lane] = st.l;
+  __syncthreads();
+  const float* group = reinterpret_cast<const float*>(smem + rg * PF_STATE);
+  if (kg_count == 2) prefill_merge<2>(a, group, 2 * PF_STATE / 4, kg, q0, tok, ql, g, n, hh, pslot);
+  else prefill_merge<4>(a, group, PF_STATE / 4, kg, q0, tok, ql, g, n, hh, pslot);
+  // Fused stage: the workgroups of the request's last segment copy their own
+  // tokens' new rows of KV head g into the scratch layer.
+  if (VERIFY && a.stage_k && k1 == kl) {
+    const int half = 16 * n_tok;
+    for (int i = threadIdx.x; i < 2 * half; i += PF_WAVES * WAVE) {
+      const bool vh = i >= half;
+      const int rem = vh ? i - half : i;
+      const size_t off = bbase + (size_t)(PF_TOKENS * t + (rem >> 4)) * KV_ROW + (size_t)(rem & 15) * 8;
+      *reinterpret_cast<bf16x8*>((vh ? a.stage_v : a.stage_k) + off) = ld8((vh ? a.v_b : a.k_b) + off);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // split-K merge: one workgroup per (request, KV head, tile) with >1 chunk
 // ---------------------------------------------------------------------------
 struct MergeArgs {
@@ -1551,71 +1988,47 @@ struct MergeArgs {
   int draft;
 };
 
-// Workgroup (8r + g, t) merges request r, KV head g, row tile t (draft: block
-// t) of a request held by more than one chunk: its id is
+// Workgroup (8r + g, y) merges request r, KV head g, row tiles y, y + gridDim.y,
+// .. (draft: blocks) of a request held by more than one chunk: its id is
 // g mod 8, so it runs on the XCD whose L2 holds the partials that the chunk
 // kernel's head-g workgroups (ids = g mod 8 as well) just wrote.
 __global__ __launch_bounds__(256) void merge_kernel(MergeArgs a) {
   const int r = blockIdx.x >> 3;
   const int g = blockIdx.x & 7;
-  const int t = blockIdx.y;
-  int len, out_row0, rows_valid;
+  // First partial slot and segment count of the request, its first output
+  // row and output rows (draft: 7 per block, one block per tile).
+  int first, nch, row0, rows;
   if (a.req) {
     const int32_t* m = a.req + REQ_INTS * r;
-    const int nch = m[1];
-    if (nch == 1) return;
-    int row0, valid;
-    if (a.draft) {
-      if (t >= m[3]) return;
-      row0 = BLOCK_ROWS * (m[2] + t);
-      valid = BLOCK_ROWS;
-    } else {
-      if (8 * t >= m[3]) return;
-      row0 = m[2] + 8 * t;
-      valid = min(8, m[3] - 8 * t);
-    }
-    const int tid = threadIdx.x;
-    const int row = tid >> 4;
-    const int d0 = (tid & 15) * 8;
-    if ((row >> 1) >= valid) return;
+    first = m[0];
+    nch = m[1];
+    row0 = a.draft ? BLOCK_ROWS * m[2] : m[2];
+    rows = a.draft ? BLOCK_ROWS * m[3] : m[3];
+  } else {
+    const int32_t* cu = a.draft ? a.cu_b : a.cu_q;
+    const int unit = a.draft ? BLOCK_ROWS : 1;
+    row0 = unit * cu[r];
+    rows = unit * (cu[r + 1] - cu[r]);
+    nch = chunks_for(a.draft ? a.ctx_len[r] : a.cu_k[r + 1] - a.cu_k[r], a.chunk);
+    first = nch == 1 ? 0 : chunk_base(a.draft ? nullptr : a.cu_k, a.draft ? a.ctx_len : nullptr, r, a.chunk);
+  }
+  if (nch == 1) return;
+  const int step = a.draft ? BLOCK_ROWS : 8;      // output rows per tile
+  const int tid = threadIdx.x;
+  const int row = tid >> 4;
+  const int d0 = (tid & 15) * 8;
+  for (int t = blockIdx.y; step * t < rows; t += gridDim.y) {
+    const int tok = step * t + (row >> 1);
+    if ((row >> 1) >= step || tok >= rows) continue;
     float acc[8];
     float L;
-    merge_partials<8>(a.part_o, a.part_ml, (size_t)(m[0] * 8 + g) * a.tmax + t, (size_t)8 * a.tmax, nch, row, d0,
+    merge_partials<8>(a.part_o, a.part_ml, (size_t)(first * 8 + g) * a.tmax + t, (size_t)8 * a.tmax, nch, row, d0,
                       acc, L);
     bf16x8 ov;
     #pragma unroll
     for (int i = 0; i < 8; ++i) ov[i] = (bf16)(acc[i] / L);
-    *reinterpret_cast<bf16x8*>(a.out + (size_t)(row0 + (row >> 1)) * Q_ROW + (size_t)(2 * g + (row & 1)) * HD + d0) = ov;
-    return;
+    *reinterpret_cast<bf16x8*>(a.out + (size_t)(row0 + tok) * Q_ROW + (size_t)(2 * g + (row & 1)) * HD + d0) = ov;
   }
-  if (a.draft) {
-    const int b0 = a.cu_b[r];
-    if (t >= a.cu_b[r + 1] - b0) return;
-    len = a.ctx_len[r];
-    out_row0 = BLOCK_ROWS * (b0 + t);
-    rows_valid = BLOCK_ROWS;
-  } else {
-    const int q0 = a.cu_q[r];
-    const int ql = a.cu_q[r + 1] - q0;
-    if (8 * t >= ql) return;
-    len = a.cu_k[r + 1] - a.cu_k[r];
-    out_row0 = q0 + 8 * t;
-    rows_valid = min(8, ql - 8 * t);
-  }
-  const int nch = chunks_for(len, a.chunk);
-  if (nch == 1) return;
-  const int first = chunk_base(a.draft ? nullptr : a.cu_k, a.draft ? a.ctx_len : nullptr, r, a.chunk);
-  const int tid = threadIdx.x;
-  const int row = tid >> 4;
-  const int d0 = (tid & 15) * 8;
-  if ((row >> 1) >= rows_valid) return;
-  float acc[8];
-  float L;
-  merge_partials<8>(a.part_o, a.part_ml, (size_t)(first * 8 + g) * a.tmax + t, (size_t)8 * a.tmax, nch, row, d0, acc, L);
-  bf16x8 ov;
-  #pragma unroll
-  for (int i = 0; i < 8; ++i) ov[i] = (bf16)(acc[i] / L);
-  *reinterpret_cast<bf16x8*>(a.out + (size_t)(out_row0 + (row >> 1)) * Q_ROW + (size_t)(2 * g + (row & 1)) * HD + d0) = ov;
 }
 
 }  // namespace dspark
@@ -1630,15 +2043,15 @@ using namespace dspark;
 constexpr float LOG2E = 1.4426950408889634f;
 
 // Workgroups resident at once for the varlen/verify kernel (2 per CU at its
-// register budget), times the number of row tiles sharing the machine.
-unsigned persistent_grid(int n_slots, int tiles) {
+// register budget).
+unsigned persistent_grid(int n_slots) {
   static int cus = 0;
   if (!cus) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
       cus = 256;
   }
-  const int64_t resident = std::max<int64_t>(8, (int64_t)cus * 2 / std::max(tiles, 1) / 8 * 8);
+  const int64_t resident = std::max<int64_t>(8, (int64_t)cus * 2 / 8 * 8);
   return (unsigned)std::min<int64_t>(n_slots, resident);
 }
 
@@ -1652,9 +2065,14 @@ int64_t workspace_bytes(int n_req, int64_t rows_bound, int tiles, int chunk) {
   return items * 16 * (HD + 2) * (int64_t)sizeof(float);
 }
 
+// Workgroups per (request, KV head): prompts have hundreds of row tiles, and a
+// request held by one segment has nothing to merge, so a grid of one workgroup
+// per tile would mostly start empty workgroups.
+constexpr int MERGE_TILES = 32;
+
 int launch_merge(const MergeArgs& m, int n_req, int tiles, hipStream_t s) {
   DSPARK_REQUIRE((int64_t)n_req * HKV <= 0x7fffffffLL, "too many requests for the merge grid (%d)", n_req);
-  hipLaunchKernelGGL(merge_kernel, dim3((unsigned)n_req * HKV, tiles), dim3(256), 0, s, m);
+  hipLaunchKernelGGL(merge_kernel, dim3((unsigned)n_req * HKV, std::min(tiles, MERGE_TILES)), dim3(256), 0, s, m);
   return launch_status("merge_kernel");
 }
 
@@ -1718,9 +2136,18 @@ int varlen_launch(VarlenArgs& a, int64_t key_rows_bound, int max_q, float scale,
   a.scale_log2 = scale * LOG2E;
   a.n_slots = (int)(n_cl * HKV);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const unsigned grid = work ? (unsigned)n_groups * HKV : persistent_grid(a.n_slots, tiles);
-  hipLaunchKernelGGL(varlen_attn_kernel<VERIFY>, dim3(grid, tiles), dim3(256), 0, s, a);
-  rc = launch_status(what);
+  const unsigned grid = work ? (unsigned)n_groups * HKV : persistent_grid(a.n_slots);
+  if (max_q <= DECODE_TOKENS) {
+    hipLaunchKernelGGL(varlen_attn_kernel<VERIFY>, dim3(grid), dim3(256), 0, s, a);
+    rc = launch_status(what);
+  } else {
+    const unsigned gx = HKV * ((max_q + PF_TOKENS - 1) / PF_TOKENS);
+    const unsigned decode_rows = (grid + gx - 1) / gx;
+    const unsigned rows = decode_rows + (unsigned)n_cl;
+    hipLaunchKernelGGL(prefill_attn_kernel<VERIFY>, dim3(gx, std::min(rows, (unsigned)PF_SEGS_Y), (rows + PF_SEGS_Y - 1) / PF_SEGS_Y),
+                       dim3(256), 0, s, a, (int)grid, (int)decode_rows);
+    rc = launch_status("prefill_attn_kernel");
+  }
   if (rc != OK) return rc;
   MergeArgs m{work ? work + WORK_INTS * n_work + n_groups + 1 : nullptr, a.cu_q, a.cu_k, nullptr, nullptr, a.part_o,
               a.part_ml, a.out, a.n_req, chunk, tiles, 0};

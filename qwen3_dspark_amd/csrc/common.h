@@ -127,6 +127,11 @@ __device__ __forceinline__ void lds_dma16_nt(const void* gptr, uint32_t lds) {
   asm volatile("global_load_lds_dwordx4 %0, off nt" ::"v"(gptr), "{m0}"(lds) : "memory");
 }
 
+// The same load from a wave-uniform base plus a per-lane byte offset.
+__device__ __forceinline__ void lds_dma16_base(const void* base, uint32_t offset, uint32_t lds) {
+  asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "{m0}"(lds) : "memory");
+}
+
 // Direct global->LDS load of 4 bytes per lane: lane L's word lands at LDS
 // byte address `lds` + 4*L; ordered like lds_dma16.
 __device__ __forceinline__ void lds_dma4(const void* gptr, uint32_t lds) {

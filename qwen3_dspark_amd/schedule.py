@@ -30,6 +30,10 @@ Draft attention: the same balanced segments over the context rows each
 request streams (up to its largest anchor), one run per (workgroup, KV
 head), cuts on 64-row ring-stage boundaries (draft_work).
 
+Requests of more than DECODE_TOKENS query tokens (prompts) are attended by a
+kernel with one workgroup per (segment, KV head, 32 query tokens); their
+segments follow the runs' records and belong to no run (prompt_segments).
+
 Without a list, both kernels walk fixed chunks of `chunk` rows in request
 order over a grid sized from the row bound.
 """
@@ -46,6 +50,9 @@ SEGMENT_COST = 96             # keys' worth of fixed work per segment in balance
 # later one's waves lose issue arbitration to the older ones, so it streams
 # ~15 % slower (measured; 0.6-0.9 all gain about the same).
 SECOND_SLOT_SHARE = 0.75
+DECODE_TOKENS = 8             # requests with more query tokens take the prefill kernel (attn.hip)
+PROMPT_TOKENS = 32            # query tokens per prefill workgroup (two resident per CU)
+MIN_PROMPT_SEGMENT = 1024     # fewest keys a cut leaves a prompt segment (see prompt_segments)
 DRAFT_TILE = 64               # draft cuts fall on multiples of the ring stage
 DRAFT_SEGMENT_COST = 512      # balanced draft plans: fixed cost of a segment, in context rows (measured)
 DRAFT_BLOCK_WEIGHT = 0.055    # balanced draft plans: extra cost of a row per block beyond the first (measured)
@@ -96,14 +103,15 @@ def run_count(total_keys, n_cu, row_tiles=1):
     return -(-runs // XCDS) * XCDS
 
 
-def _flatten(n, per_run, record, request):
+def _flatten(n, per_run, record, request, loose=()):
     """Flatten per-run [(request, k0, k1)] segment lists into the int32 list
     format, giving split requests consecutive request-major partial slots in
     key order.  record(r, k0, k1, slot) and request(r, first, count) give the
-    8 and 4 ints of a segment and a request.  Returns (list, segment count,
-    run count)."""
+    8 and 4 ints of a segment and a request.  loose: segments of no run, after
+    the runs' records.  Returns (list, segment count, run count)."""
     count = [0] * n
-    for run in per_run:
+    loose = list(loose)
+    for run in [*per_run, loose]:
         for r, _, _ in run:
             count[r] += 1
     first, slot = [], 0
@@ -112,7 +120,7 @@ def _flatten(n, per_run, record, request):
         slot += c if c > 1 else 0
     keyed = {}
     # partial slot of a segment = first slot of its request + its key-order rank
-    for run in per_run:
+    for run in [*per_run, loose]:
         for r, k0, _ in run:
             keyed.setdefault(r, []).append(k0)
     rank = {r: {k0: i for i, k0 in enumerate(sorted(v))} for r, v in keyed.items()}
@@ -121,13 +129,15 @@ def _flatten(n, per_run, record, request):
         for r, k0, k1 in run:
             out += record(r, k0, k1, first[r] + rank[r][k0] if first[r] >= 0 else -1)
         ranges.append(ranges[-1] + len(run))
+    for r, k0, k1 in loose:
+        out += record(r, k0, k1, first[r] + rank[r][k0] if first[r] >= 0 else -1)
     out += ranges
     for r in range(n):
         out += request(r, max(first[r], 0), count[r])
-    return out, ranges[-1], len(per_run)
+    return out, ranges[-1] + len(loose), len(per_run)
 
 
-def _segment_list(query_lengths, key_lengths, starts, per_run):
+def _segment_list(query_lengths, key_lengths, starts, per_run, loose=()):
     """Varlen/verify records: request, k0, k1, slot, first query row, query
     length, key length, start; request records: first slot, count, first
     query row, query length."""
@@ -138,7 +148,7 @@ def _segment_list(query_lengths, key_lengths, starts, per_run):
     return _flatten(len(key_lengths), per_run,
                     lambda r, k0, k1, slot: (r, k0, k1, slot, q0[r], int(query_lengths[r]), int(key_lengths[r]),
                                              int(starts[r])),
-                    lambda r, first, count: (first, count, q0[r], int(query_lengths[r])))
+                    lambda r, first, count: (first, count, q0[r], int(query_lengths[r])), loose)
 
 
 def _balanced_runs(key_lengths, groups, tile, seg_cost=0, weights=None, shares=None):
@@ -244,8 +254,48 @@ def varlen_work(query_lengths, key_lengths, starts, groups, seg_cost=None, xcd_s
     differ in the last bits between batches; request_work keeps them
     apart."""
     cost = SEGMENT_COST if seg_cost is None else seg_cost
-    return _segment_list(query_lengths, key_lengths, starts,
-                         _balanced_runs(key_lengths, groups, TILE, cost, shares=run_shares(groups, xcd_speed, n_cu)))
+    decode = [r for r, q in enumerate(query_lengths) if q <= DECODE_TOKENS]
+    if len(decode) == len(key_lengths):
+        runs = _balanced_runs(key_lengths, groups, TILE, cost, shares=run_shares(groups, xcd_speed, n_cu))
+        return _segment_list(query_lengths, key_lengths, starts, runs)
+    loose = prompt_segments(query_lengths, key_lengths, groups, n_cu)
+    # each cut of a prompt takes a run's cut from the others, so the segments
+    # stay within varlen_list_bound
+    cuts = len(loose) - (len(key_lengths) - len(decode))
+    runs = [[] for _ in range(groups)]
+    if decode:
+        n = groups - cuts
+        runs[:n] = [[(decode[r], k0, k1) for r, k0, k1 in run]
+                    for run in _balanced_runs([key_lengths[r] for r in decode], n, TILE, cost,
+                                              shares=run_shares(n, xcd_speed, n_cu))]
+    return _segment_list(query_lengths, key_lengths, starts, runs, loose)
+
+
+def prompt_segments(query_lengths, key_lengths, groups, n_cu=None):
+    """[(request, k0, k1)] of the requests with more than DECODE_TOKENS query
+    tokens, longest last: one segment each, so that nothing is merged, unless
+    their (32-token tile, KV head) workgroups leave CUs idle over long keys (a
+    later chunk of a prompt): then the request with the longest segments is cut
+    once more, into equal parts of whole ring stages, while every part keeps
+    MIN_PROMPT_SEGMENT keys, the workgroups fit two per CU and fewer than
+    `groups` cuts are made.  A cut costs an FP32 partial write and read per
+    tile (528 bytes a row, what ~260 keys' K and V cost) and a merge."""
+    prompts = [r for r, q in enumerate(query_lengths) if q > DECODE_TOKENS]
+    tiles = {r: -(-int(query_lengths[r]) // PROMPT_TOKENS) for r in prompts}
+    parts = dict.fromkeys(prompts, 1)
+    slots = RESIDENT_PER_CU * int(n_cu or 256) // 8
+    used, cuts = sum(tiles.values()), 0
+    while cuts < groups - 1:
+        r = max(prompts, key=lambda x: key_lengths[x] / parts[x])
+        if used + tiles[r] > slots or key_lengths[r] < MIN_PROMPT_SEGMENT * (parts[r] + 1):
+            break
+        parts[r], used, cuts = parts[r] + 1, used + tiles[r], cuts + 1
+    out = []
+    for r in sorted(prompts, key=lambda x: key_lengths[x]):
+        kl = int(key_lengths[r])
+        at = [i * kl // parts[r] // DRAFT_TILE * DRAFT_TILE for i in range(parts[r])] + [kl]
+        out += [(r, a, b) for a, b in zip(at, at[1:])]
+    return out
 
 
 def request_work(query_lengths, key_lengths, starts, chunk, groups):
@@ -264,11 +314,14 @@ def request_work(query_lengths, key_lengths, starts, chunk, groups):
     groups = -(-max(1, min(int(groups), len(segs))) // XCDS) * XCDS     # whole rounds over the XCDs
     heap = [(0, w) for w in range(groups)]
     per_run = [[] for _ in range(groups)]
+    loose = [(r, k0, k1) for _, r, k0, k1 in reversed(segs) if query_lengths[r] > DECODE_TOKENS]
     for size, r, k0, k1 in segs:
+        if query_lengths[r] > DECODE_TOKENS:
+            continue
         load, w = heapq.heappop(heap)
         per_run[w].append((r, k0, k1))
         heapq.heappush(heap, (load + size + TILE, w))
-    return _segment_list(query_lengths, key_lengths, starts, per_run)
+    return _segment_list(query_lengths, key_lengths, starts, per_run, loose)
 
 
 def varlen_list_bound(n_req, groups, rows_bound=0, chunk=None):

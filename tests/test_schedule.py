@@ -280,3 +280,32 @@ def test_second_slot_runs_get_a_smaller_share():
         assert abs(cost[w] - total * shares[w] / norm) <= 2 * (TILE + SEGMENT_COST)
     assert sum(loads) == sum(kl)
     assert varlen_work([7] * 64, kl, list(range(64)), 32, n_cu=256) == varlen_work([7] * 64, kl, list(range(64)), 32)
+
+
+@pytest.mark.parametrize('ql,kl', [([100], [100]), ([9, 7, 300], [9000, 40, 300]), ([20] * 5, [2000] * 5),
+                                   ([7, 7, 64], [5000, 300, 64]), ([4000], [4000]), ([256], [16000])])
+@pytest.mark.parametrize('split', ['balanced', 'request'])
+def test_prompt_segments_follow_the_runs(ql, kl, split):
+    """Requests with more than 8 query tokens: every key covered once by
+    records of no run, after the runs' records, within the list's bound; the
+    other requests stay in the runs; prompts are cut at whole 64-key stages
+    into parts of at least 1,024 keys (balanced), or at the chunk (request)."""
+    from qwen3_dspark_amd.schedule import MIN_PROMPT_SEGMENT, PROMPT_TOKENS, segment_plan
+    n = len(ql)
+    groups = run_count(sum(kl), 256, (max(ql) + 7) // 8)
+    chunk = 512
+    out, n_seg, runs = segment_plan(split, ql, kl, list(range(n)), groups, chunk, n_cu=256)
+    assert n_seg <= varlen_list_bound(n, groups, sum(kl), None if split == 'balanced' else chunk)
+    rec, ranges, reqs = decode(out, n_seg, runs, n)
+    in_runs = ranges[-1]
+    for r in range(n):
+        segs = sorted((x[1], x[2], x[3], i < in_runs) for i, x in enumerate(rec) if x[0] == r)
+        assert segs[0][0] == 0 and segs[-1][1] == kl[r]
+        assert all(a[1] == b[0] for a, b in zip(segs, segs[1:]))
+        assert all(x[3] == (ql[r] <= 8) for x in segs)
+        first, count = reqs[r][:2]
+        assert count == len(segs) and [x[2] for x in segs] == ([-1] if count == 1 else
+                                                               list(range(first, first + count)))
+        if split == 'balanced' and ql[r] > 8 and count > 1:
+            assert all(x[0] % 64 == 0 and x[1] - x[0] >= MIN_PROMPT_SEGMENT - 64 for x in segs)
+            assert sum(-(-ql[x[0]] // PROMPT_TOKENS) for x in rec[in_runs:]) <= 64
