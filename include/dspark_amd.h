@@ -289,6 +289,20 @@ int dspark_draft_kv_project(const void* x, int tokens, int hidden, const void* w
                             int64_t slot_stride, int64_t head_stride, int32_t* flag, void* stream);
 
 /*
+ * dspark_draft_kv_project for many tokens, in two launches: one computes what
+ * depends on the token alone (context-norm factor, pool row, rotary angles)
+ * into `workspace` (dspark_draft_rows_bytes(tokens) bytes, 16-byte aligned), the
+ * other projects 128-token tiles.  Same arguments and results (FP32
+ * accumulation in another order, every output rounded to bf16 once).
+ */
+int64_t dspark_draft_rows_bytes(int tokens);
+int dspark_draft_kv_project_rows(const void* x, int tokens, int hidden, const void* w, const void* k_norm,
+                                 int layers, const float* inv_freq, const int32_t* req, int n_req,
+                                 float eps_ctx, float eps_k, void* k_pool, void* v_pool, int64_t layer_stride,
+                                 int64_t slot_stride, int64_t head_stride, int32_t* flag, void* workspace,
+                                 int64_t workspace_bytes, void* stream);
+
+/*
  * The same projection after a library GEMM, for large appends: y [tokens,
  * y_stride] holds x Wfold^T (columns [layer][K, V][head][128], the folded
  * weights of dspark_draft_kv_project as one [layers*2*1024, hidden]

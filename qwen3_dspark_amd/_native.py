@@ -47,6 +47,9 @@ SIGNATURES = {
     'dspark_qkv_prologue': (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _F, _P, _P, _P, _L, _P]),
     'dspark_rope_table': (_I, [_P, _P, _I, _P, _P]),
     'dspark_draft_kv_project': (_I, [_P, _I, _I, _P, _P, _I, _P, _P, _I, _F, _F, _P, _P, _L, _L, _L, _P, _P]),
+    'dspark_draft_rows_bytes': (_L, [_I]),
+    'dspark_draft_kv_project_rows': (_I, [_P, _I, _I, _P, _P, _I, _P, _P, _I, _F, _F, _P, _P, _L, _L, _L, _P, _P, _L,
+                                          _P]),
     'dspark_draft_kv_epilogue': (_I, [_P, _I, _L, _P, _I, _I, _I, _P, _I, _P, _P, _I, _F, _F, _P, _P, _L, _L, _L,
                                       _P, _P]),
     'dspark_row_stats_bytes': (_L, [_I, _I]),

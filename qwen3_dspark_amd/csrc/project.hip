@@ -24,7 +24,7 @@
 // (slot, first position, first token, count) covers it; its row goes to
 // (slot, position) of every layer's pool.  A non-finite output sets *flag
 // (the caller publishes the rows only when it is clear).
-#include "head_gemm.h"
+#include "wide_gemm.h"
 
 namespace dspark {
 
@@ -112,11 +112,11 @@ __global__ __launch_bounds__(HG_WAVES * WAVE) void draft_kv_project_kernel(Draft
 
 using namespace dspark;
 
-extern "C" int dspark_draft_kv_project(const void* x, int tokens, int hidden, const void* w, const void* k_norm,
-                                       int layers, const float* inv_freq, const int32_t* req, int n_req,
-                                       float eps_ctx, float eps_k, void* k_pool, void* v_pool, int64_t layer_stride,
-                                       int64_t slot_stride, int64_t head_stride, int32_t* flag, void* stream) {
-  clear_error();
+namespace {
+int project_args(const void* x, int tokens, int hidden, const void* w, const void* k_norm, int layers,
+                 const float* inv_freq, const int32_t* req, int n_req, float eps_ctx, float eps_k, void* k_pool,
+                 void* v_pool, int64_t layer_stride, int64_t slot_stride, int64_t head_stride, int32_t* flag,
+                 DraftProjArgs& a) {
   DSPARK_REQUIRE(x && w && k_norm && inv_freq && req && k_pool && v_pool, "null pointer argument");
   DSPARK_REQUIRE(tokens >= 1 && hidden >= HG_COLS && hidden % HG_COLS == 0, "need tokens >= 1 and hidden a multiple of %d",
                  HG_COLS);
@@ -129,14 +129,156 @@ extern "C" int dspark_draft_kv_project(const void* x, int tokens, int hidden, co
   const uintptr_t any = (uintptr_t)x | (uintptr_t)w | (uintptr_t)k_pool | (uintptr_t)v_pool | (uintptr_t)inv_freq;
   DSPARK_REQUIRE(any % 16 == 0, "tensors must be 16-byte aligned");
   DSPARK_REQUIRE((uintptr_t)k_norm % 8 == 0, "k_norm must be 8-byte aligned");
-  const int64_t tiles = (tokens + HG_TOKENS - 1) / HG_TOKENS;
-  DSPARK_REQUIRE(tiles * layers * 2 * HKV <= 0x7fffffffLL, "too many tokens");
-  DraftProjArgs a{static_cast<const bf16*>(x), static_cast<const bf16*>(w), static_cast<const bf16*>(k_norm), inv_freq,
+  a = DraftProjArgs{static_cast<const bf16*>(x), static_cast<const bf16*>(w), static_cast<const bf16*>(k_norm), inv_freq,
                   req, static_cast<bf16*>(k_pool), static_cast<bf16*>(v_pool), layer_stride, slot_stride, head_stride,
                   flag, tokens, hidden, layers, n_req, eps_ctx, eps_k};
+  return OK;
+}
+}  // namespace
+
+extern "C" int dspark_draft_kv_project(const void* x, int tokens, int hidden, const void* w, const void* k_norm,
+                                       int layers, const float* inv_freq, const int32_t* req, int n_req,
+                                       float eps_ctx, float eps_k, void* k_pool, void* v_pool, int64_t layer_stride,
+                                       int64_t slot_stride, int64_t head_stride, int32_t* flag, void* stream) {
+  clear_error();
+  DraftProjArgs a;
+  const int rc = project_args(x, tokens, hidden, w, k_norm, layers, inv_freq, req, n_req, eps_ctx, eps_k, k_pool, v_pool,
+                              layer_stride, slot_stride, head_stride, flag, a);
+  if (rc != OK) return rc;
+  const int64_t tiles = (tokens + HG_TOKENS - 1) / HG_TOKENS;
+  DSPARK_REQUIRE(tiles * layers * 2 * HKV <= 0x7fffffffLL, "too many tokens");
   hipLaunchKernelGGL(draft_kv_project_kernel, dim3((unsigned)(tiles * layers * 2 * HKV)), dim3(HG_WAVES * WAVE), 0,
                      static_cast<hipStream_t>(stream), a);
   return launch_status("draft_kv_project_kernel");
+}
+
+// ---------------------------------------------------------------------------
+// The same projection for many tokens: 128-token tiles (wide_gemm.h).  What
+// depends on the token alone - its context-norm factor, its pool slot and
+// position, its rotary angles - is computed once per token by
+// draft_rows_kernel and read by the layers' K and V heads.
+// ---------------------------------------------------------------------------
+namespace dspark {
+
+struct DraftRow {
+  int32_t slot, pos;
+  float norm;                // 1 / sqrt(mean(f^2) + eps)
+  int32_t pad;
+};
+static_assert(sizeof(DraftRow) == 16, "a row is one 16-byte load");
+
+// One wave per token; rope[t]: cos of the 64 angles, then their sin.
+__global__ __launch_bounds__(256) void draft_rows_kernel(DraftProjArgs a, DraftRow* __restrict__ rows,
+                                                         float* __restrict__ rope) {
+  const int lane = threadIdx.x & 63;
+  const int tok = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (tok >= a.tokens) return;
+  float ss = 0.f;
+  const bf16* xr = a.x + (size_t)tok * a.hidden;
+  for (int d = 8 * lane; d < a.hidden; d += 8 * WAVE) {
+    const bf16x8 v = ld8(xr + d);
+    #pragma unroll
+    for (int e = 0; e < 8; ++e) ss += (float)v[e] * (float)v[e];
+  }
+  #pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) ss += __shfl_xor(ss, off);
+  int lo = 0, hi = a.n_req - 1;                        // the last record whose first token <= tok
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (a.req[4 * mid + 2] <= tok) lo = mid;
+    else hi = mid - 1;
+  }
+  const int32_t* rq = a.req + 4 * lo;
+  const int pos = rq[1] + (tok - rq[2]);
+  float sn, cs;
+  sincosf((float)pos * a.inv_freq[lane], &sn, &cs);
+  rope[(size_t)tok * 128 + lane] = cs;
+  rope[(size_t)tok * 128 + 64 + lane] = sn;
+  if (lane == 0) rows[tok] = DraftRow{rq[0], pos, rsqrtf(ss / (float)a.hidden + a.eps_ctx), 0};
+}
+
+__global__ __launch_bounds__(WG_WAVES * WAVE, 2) void draft_kv_project_wide_kernel(DraftProjArgs a,
+                                                                                   const DraftRow* __restrict__ rows,
+                                                                                   const float* __restrict__ rope) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem[WG_SMEM];
+  // KV head = id % 8 = XCD; the layers' K and V of a token tile are adjacent,
+  // so that its rows are read from HBM once per XCD.
+  const int head = blockIdx.x & 7;
+  const int slot_id = blockIdx.x >> 3;
+  const int part = slot_id % (2 * a.layers);          // 2 * layer + (V ? 1 : 0)
+  const int t0 = slot_id / (2 * a.layers) * WG_TOKENS;
+  const int layer = part >> 1;
+  const bool is_v = part & 1;                         // workgroup-uniform
+  const bf16* w = a.w + ((size_t)part * KV_ROW + (size_t)head * HD) * a.hidden;
+  f32x16 v[2][2];
+  wide_tile_gemm(w, a.x, a.tokens, a.hidden, t0, smem, v);
+
+  const WideLane L;
+  int tok[2];
+  DraftRow r[2];
+  #pragma unroll
+  for (int tt = 0; tt < 2; ++tt) {
+    tok[tt] = min(t0 + L.token(tt), a.tokens - 1);
+    r[tt] = rows[tok[tt]];
+    #pragma unroll
+    for (int i = 0; i < 2; ++i)
+      #pragma unroll
+      for (int e = 0; e < 16; ++e) v[i][tt][e] *= r[tt].norm;
+  }
+  if (!is_v) {
+    wide_norm_rope(v, a.k_norm + (size_t)layer * HD, a.eps_k, smem, [&](int tt, int dim, f32x4& c, f32x4& s) {
+      const float* row = rope + (size_t)tok[tt] * 128 + dim;
+      c = *reinterpret_cast<const f32x4*>(row);
+      s = *reinterpret_cast<const f32x4*>(row + 64);
+    });
+  }
+  #pragma unroll
+  for (int tt = 0; tt < 2; ++tt) {
+    const bool valid = t0 + L.token(tt) < a.tokens;
+    if (a.flag) {
+      bool bad = false;
+      #pragma unroll
+      for (int i = 0; i < 2; ++i)
+        #pragma unroll
+        for (int e = 0; e < 16; ++e) bad |= !__builtin_isfinite(v[i][tt][e]);
+      if (__builtin_amdgcn_ballot_w64(bad && valid) && (threadIdx.x & 63) == 0) *a.flag = 1;   // idempotent vector store
+    }
+    bf16* out = (is_v ? a.v_pool : a.k_pool) + (size_t)layer * a.layer_stride + (size_t)r[tt].slot * a.slot_stride +
+                (size_t)head * a.head_stride + (size_t)r[tt].pos * HD;
+    wide_store(v, tt, out, valid);
+  }
+}
+
+}  // namespace dspark
+
+extern "C" int64_t dspark_draft_rows_bytes(int tokens) {
+  if (tokens < 1) return -1;
+  return (int64_t)tokens * ((int64_t)sizeof(DraftRow) + 128 * (int64_t)sizeof(float));
+}
+
+extern "C" int dspark_draft_kv_project_rows(const void* x, int tokens, int hidden, const void* w, const void* k_norm,
+                                            int layers, const float* inv_freq, const int32_t* req, int n_req,
+                                            float eps_ctx, float eps_k, void* k_pool, void* v_pool, int64_t layer_stride,
+                                            int64_t slot_stride, int64_t head_stride, int32_t* flag, void* workspace,
+                                            int64_t workspace_bytes, void* stream) {
+  clear_error();
+  DraftProjArgs a;
+  const int rc = project_args(x, tokens, hidden, w, k_norm, layers, inv_freq, req, n_req, eps_ctx, eps_k, k_pool, v_pool,
+                              layer_stride, slot_stride, head_stride, flag, a);
+  if (rc != OK) return rc;
+  DSPARK_REQUIRE(workspace && (uintptr_t)workspace % 16 == 0 && workspace_bytes >= dspark_draft_rows_bytes(tokens),
+                 "workspace must be 16-byte aligned and hold dspark_draft_rows_bytes(tokens) bytes");
+  const int64_t tiles = (tokens + WG_TOKENS - 1) / WG_TOKENS;
+  DSPARK_REQUIRE(tiles * layers * 2 * HKV <= 0x7fffffffLL, "too many tokens");
+  DraftRow* rows = static_cast<DraftRow*>(workspace);
+  float* rope = reinterpret_cast<float*>(rows + tokens);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  hipLaunchKernelGGL(draft_rows_kernel, dim3((unsigned)((tokens + 3) / 4)), dim3(256), 0, s, a, rows, rope);
+  int st = launch_status("draft_rows_kernel");
+  if (st != OK) return st;
+  hipLaunchKernelGGL(draft_kv_project_wide_kernel, dim3((unsigned)(tiles * layers * 2 * HKV)), dim3(WG_WAVES * WAVE), 0, s,
+                     a, rows, rope);
+  return launch_status("draft_kv_project_wide_kernel");
 }
 
 // ---------------------------------------------------------------------------

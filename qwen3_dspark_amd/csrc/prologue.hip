@@ -20,7 +20,7 @@
 // MFMA tile (head_gemm.h); all 8 waves run the epilogue on 16 dims of one
 // token per lane.  Accumulation and the epilogue are FP32; outputs are
 // rounded to bf16 once.
-#include "head_gemm.h"
+#include "wide_gemm.h"
 
 namespace dspark {
 
@@ -85,6 +85,54 @@ __global__ __launch_bounds__(HG_WAVES * WAVE) void qkv_prologue_kernel(PrologueA
   head_store(v, out + (size_t)hh * HD, row < a.tokens);
 }
 
+// The same for many tokens: 128-token tiles (wide_gemm.h), two workgroups per CU.
+template <bool TABLE>
+__global__ __launch_bounds__(WG_WAVES * WAVE, 2) void qkv_prologue_wide_kernel(PrologueArgs a) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem[WG_SMEM];
+  const int tiles = (a.tokens + WG_TOKENS - 1) / WG_TOKENS;
+  const int xcd = blockIdx.x & 7;                // a head's tiles share id % 8 (see above)
+  const int slot = blockIdx.x >> 3;
+  const int head = xcd + 8 * (slot & 3);
+  const int t0 = (slot >> 2) * WG_TOKENS;
+  const int kind = head < HQ ? 0 : (head < HQ + HKV ? 1 : 2);       // workgroup-uniform
+  const int hh = kind == 0 ? head : (kind == 1 ? head - HQ : head - HQ - HKV);
+  const bf16* w = (kind == 0 ? a.wq : (kind == 1 ? a.wk : a.wv)) + (size_t)hh * HD * a.hidden;
+  f32x16 v[2][2];
+  wide_tile_gemm(w, a.x, a.tokens, a.hidden, t0, smem, v);
+  const WideLane L;
+  if (kind < 2) {
+    int tok[2];
+    float pos[2];
+    #pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      tok[tt] = min(t0 + L.token(tt), a.tokens - 1);
+      pos[tt] = TABLE ? 0.f : (float)a.positions[tok[tt]];
+    }
+    wide_norm_rope(v, kind == 0 ? a.q_norm : a.k_norm, a.eps, smem, [&](int tt, int dim, f32x4& c, f32x4& s) {
+      if (TABLE) {
+        const float* row = a.rope + (size_t)tok[tt] * 128 + dim;
+        c = *reinterpret_cast<const f32x4*>(row);
+        s = *reinterpret_cast<const f32x4*>(row + 64);
+      } else {
+        #pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float sn, cs;
+          sincosf(pos[tt] * a.inv_freq[dim + i], &sn, &cs);
+          c[i] = cs;
+          s[i] = sn;
+        }
+      }
+    });
+  }
+  #pragma unroll
+  for (int tt = 0; tt < 2; ++tt) {
+    const int row = t0 + L.token(tt);
+    const int tok = min(row, a.tokens - 1);
+    bf16* out = kind == 0 ? a.q_out + (size_t)tok * Q_ROW : (kind == 1 ? a.k_out : a.v_out) + (size_t)tok * a.kv_row_stride;
+    wide_store(v, tt, out + (size_t)hh * HD, row < a.tokens);
+  }
+}
+
 // cos and sin of pos[t] * inv_freq[d] (FP32 angle, d < 64) for every row:
 // table[t][d] = cos, table[t][64 + d] = sin.
 __global__ __launch_bounds__(256) void rope_table_kernel(const float* __restrict__ inv_freq,
@@ -102,6 +150,12 @@ __global__ __launch_bounds__(256) void rope_table_kernel(const float* __restrict
 }  // namespace dspark
 
 using namespace dspark;
+
+// From here on the 64-token tiles (one workgroup per CU) need a second round of
+// the 256 CUs.  64- against 128-token tiles, us per launch at hidden 1,024: 512
+// tokens 10.3 / 14.8, 640 17.5 / 15.2, 1,024 19.0 / 16.8, 2,048 38.6 / 24.7,
+// 4,096 73 / 45, 8,192 141 / 88.
+constexpr int PROLOGUE_WIDE_TOKENS = 513;
 
 extern "C" int dspark_qkv_prologue(const void* x, const void* wq, const void* wk, const void* wv,
                                    const void* q_norm, const void* k_norm, const float* inv_freq,
@@ -122,6 +176,13 @@ extern "C" int dspark_qkv_prologue(const void* x, const void* wq, const void* wk
                  static_cast<const bf16*>(wv), static_cast<const bf16*>(q_norm), static_cast<const bf16*>(k_norm),
                  inv_freq, positions, rope, static_cast<bf16*>(q_out), static_cast<bf16*>(k_out),
                  static_cast<bf16*>(v_out), kv_row_stride, tokens, hidden, eps};
+  if (tokens >= PROLOGUE_WIDE_TOKENS) {
+    const dim3 grid((HQ + 2 * HKV) * ((tokens + WG_TOKENS - 1) / WG_TOKENS));
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (rope) hipLaunchKernelGGL(qkv_prologue_wide_kernel<true>, grid, dim3(WG_WAVES * WAVE), 0, s, a);
+    else hipLaunchKernelGGL(qkv_prologue_wide_kernel<false>, grid, dim3(WG_WAVES * WAVE), 0, s, a);
+    return launch_status("qkv_prologue_wide_kernel");
+  }
   hipLaunchKernelGGL(qkv_prologue_kernel, dim3((HQ + 2 * HKV) * ((tokens + HG_TOKENS - 1) / HG_TOKENS)), dim3(HG_WAVES * WAVE), 0,
                      static_cast<hipStream_t>(stream), a);
   return launch_status("qkv_prologue_kernel");

@@ -6,7 +6,7 @@ draft pool.
     ctx = context_norm(fc(features))                     [T, hidden]
     k_l = rotate(k_norm_l(k_proj_l(ctx)), cos, sin),  v_l = v_proj_l(ctx)
 
-Two launches for all draft layers and requests:
+For all draft layers and requests:
   * fc, a plain [T, 5*hidden] x [5*hidden, hidden] GEMM, on hipBLASLt
     (torch's bf16 linear, the same rounding point as the draft's autocast);
   * dspark_draft_kv_project: the context norm (its weight folded into the
@@ -14,25 +14,27 @@ Two launches for all draft layers and requests:
     result), every layer's k_proj / k_norm / RoPE and v_proj, and the store
     into each request's pool slot at its absolute positions, with a device
     finiteness flag.
-From GEMM_MIN_TOKENS appended tokens on, the k/v projection itself is a
-plain GEMM that hipBLASLt runs faster than the fused tiles: it then runs as
-one library GEMM per GEMM_CHUNK tokens (all layers' folded weights as one
-matrix, bf16 operands, FP32 output) followed by dspark_draft_kv_epilogue
-(norm factor, k_norm, RoPE, pool store, flag).  Both paths keep the
-projection in FP32 through the norms and RoPE and round every output to
+Once that launch's 64-token tiles would need a second round of the CUs,
+dspark_draft_kv_project_rows projects 128-token tiles instead, after one
+launch that computes what depends on the token alone.  path='gemm' runs the
+k/v projection as a library GEMM per GEMM_CHUNK tokens (all layers' folded
+weights as one matrix, bf16 operands, FP32 output) followed by
+dspark_draft_kv_epilogue; no length takes it by default.  All paths keep
+the projection in FP32 through the norms and RoPE and round every output to
 bf16 once, so the path a given append length takes changes only the
 accumulation order.
 """
 import torch
 
 from . import _native
+from ._device import cu_count
 from .kernels import HEAD_DIM, KV_HEADS
 from .prologue import rope_inv_freq
 
 
-GEMM_MIN_TOKENS = 2048   # appends at least this long take the GEMM + epilogue path
+GEMM_MIN_TOKENS = float('inf')   # appends at least this long take the library GEMM + epilogue path
 GEMM_CHUNK = 16384       # tokens per library GEMM (bounds its FP32 output: 640 MiB at 5 layers)
-PATHS = ('fused', 'gemm')
+PATHS = ('fused', 'wide', 'gemm')
 
 
 class DraftContextProjector:
@@ -94,18 +96,39 @@ class DraftContextProjector:
         """fc over the concatenated features [T, F] -> [T, hidden] bf16."""
         return torch.nn.functional.linear(features, self.fc)
 
+    def _path(self, t):
+        """Path of an append of t tokens.  The 64-token tiles run one
+        workgroup per CU, 16 per layer and tile, in ~12 us per round of the
+        CUs: from the second round on the 128-token tiles are faster.  Fused /
+        wide / library GEMM, us per append at 5 layers: 192 tokens 13.3 / 19.4
+        / 57.5, 256 21.7 / 20.0 / 60.2, 448 28.8 / 25.5 / 61.0, 2,048 104.5 /
+        59.1 / 101.7, 9,840 475.7 / 265.8 / 408.5; at 1 layer: 1,024 13.3 /
+        19.9 / 28.9, 1,536 21.8 / 21.2 / 31.1, 9,840 105.1 / 65.9 / 112.4."""
+        if t >= GEMM_MIN_TOKENS:
+            return 'gemm'
+        return 'wide' if -(-t // 64) * 16 * self.layers > cu_count(self.device) else 'fused'
+
     def project_into(self, fc_out, records, n_req, keys, values, *, flag=None, path=None):
         """The projection of fc_out [T, hidden] into pool tensors keys /
         values [layers, slots, 8, capacity, 128] (bf16); records: int32 device
         tensor of n_req (slot, first position, first token, count) rows.
-        path: 'fused', 'gemm' or None (by length: GEMM_MIN_TOKENS)."""
+        path: 'fused', 'wide', 'gemm' or None (by length: see _path)."""
         if path is not None and path not in PATHS:
             raise ValueError(f'path must be one of {PATHS} or None')
         t = fc_out.shape[0]
         s = keys.stride()
         stream = _native.stream_handle(self.device)
         flag_ptr = None if flag is None else flag.data_ptr()
-        if (path or ('gemm' if t >= GEMM_MIN_TOKENS else 'fused')) == 'fused':
+        path = path or self._path(t)
+        if path == 'wide':
+            need = _native.load().dspark_draft_rows_bytes(t)
+            rows = torch.empty(need, dtype=torch.uint8, device=self.device)
+            _native.call('dspark_draft_kv_project_rows', fc_out.data_ptr(), t, self.hidden, self.w.data_ptr(),
+                         self.k_norm.data_ptr(), self.layers, self.inv_freq.data_ptr(), records.data_ptr(), n_req,
+                         self.eps, self.eps, keys.data_ptr(), values.data_ptr(), s[0], s[1], s[2], flag_ptr,
+                         rows.data_ptr(), need, stream)
+            return
+        if path == 'fused':
             _native.call('dspark_draft_kv_project', fc_out.data_ptr(), t, self.hidden, self.w.data_ptr(),
                          self.k_norm.data_ptr(), self.layers, self.inv_freq.data_ptr(), records.data_ptr(), n_req,
                          self.eps, self.eps, keys.data_ptr(), values.data_ptr(), s[0], s[1], s[2], flag_ptr, stream)
