@@ -489,6 +489,18 @@ int dspark_pool_append(void* k_pool, void* v_pool, int64_t layer_stride, int64_t
                        const int32_t* req, int n_req, int32_t* nonfinite, void* stream);
 
 /*
+ * Rows of n_sources bf16 tensors packed end to end into dst [rows, row_bytes],
+ * with a finiteness flag: the feature concatenation and check of
+ * append_committed (dspark_qwen/packed_draft.py:141-147) in one pass.
+ * sources: int64 device array of the tensors' addresses (contiguous rows,
+ * 16-byte aligned); source s starts at packed row first[s * first_stride]
+ * (int32, ascending from 0).  dst NULL checks without copying.  *nonfinite is
+ * set to 1 if any element is Inf/NaN (never cleared).
+ */
+int dspark_rows_pack(const int64_t* sources, const int32_t* first, int n_sources, int first_stride,
+                     int64_t rows, int64_t row_bytes, void* dst, int32_t* nonfinite, void* stream);
+
+/*
  * Append-order KV cache of PackedTarget (dspark_qwen/packed_target.py:30-113):
  * per layer K/V [1, H, N, piece] with rows in append order and int64
  * key_requests / key_positions [N].

@@ -328,6 +328,54 @@ __global__ __launch_bounds__(256) void pool_append_kernel(AppendArgs a) {
   if (a.nonfinite && bad) atomicOr(a.nonfinite, 1);
 }
 
+// Rows of several bf16 tensors packed end to end, with a finiteness flag: what
+// torch.cat and isfinite().all() do in six passes (cat, abs, two compares, and,
+// reduce) in one.  Source s holds rows first[s * stride] .. of the packed
+// tensor; dst NULL checks the one source without copying.  One workgroup per
+// PACK_ROWS rows; bound: the read and the write (9,840 rows of 10 KiB: 169 us in
+// all before, 34.7 us now, 5.8 TB/s; 290 rows: 38 us before, 6.7 now).
+constexpr int PACK_ROWS = 2;
+
+struct PackArgs {
+  const int64_t* sources;   // [n] device addresses
+  const int32_t* first;     // first row of source s at first[s * stride], ascending from 0
+  int n;
+  int stride;
+  int64_t rows;
+  int row_vecs;             // 16-byte vectors per row
+  u32x4* dst;               // [rows][row_vecs], or NULL
+  int32_t* nonfinite;       // set to 1 on any Inf/NaN (never cleared)
+};
+
+__global__ __launch_bounds__(256) void rows_pack_kernel(PackArgs a) {
+  bool bad = false;
+  for (int k = 0; k < PACK_ROWS; ++k) {
+    const int64_t row = (int64_t)blockIdx.x * PACK_ROWS + k;
+    if (row >= a.rows) break;                       // uniform across the workgroup
+    int lo = 0, hi = a.n - 1;                       // last source whose first row <= row
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (a.first[(int64_t)mid * a.stride] <= row) lo = mid; else hi = mid - 1;
+    }
+    const u32x4* src = reinterpret_cast<const u32x4*>(a.sources[lo]) +
+                       (row - a.first[(int64_t)lo * a.stride]) * a.row_vecs;
+    u32x4* dst = a.dst ? a.dst + row * a.row_vecs : nullptr;
+    for (int v0 = threadIdx.x; v0 < a.row_vecs; v0 += 256 * 4) {
+      u32x4 x[4];
+      #pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (v0 + 256 * u < a.row_vecs) x[u] = src[v0 + 256 * u];
+      #pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (v0 + 256 * u < a.row_vecs) {
+          bad |= vec_nonfinite(x[u], 2);
+          if (dst) dst[v0 + 256 * u] = x[u];
+        }
+    }
+  }
+  if (__builtin_amdgcn_ballot_w64(bad) && (threadIdx.x & 63) == 0) *a.nonfinite = 1;   // idempotent vector store
+}
+
 }  // namespace dspark
 
 // ---------------------------------------------------------------------------
@@ -477,4 +525,19 @@ extern "C" int dspark_pool_append(void* k_pool, void* v_pool, int64_t layer_stri
   hipLaunchKernelGGL(pool_append_kernel, dim3((unsigned)blocks, layers), dim3(256), 0,
                      static_cast<hipStream_t>(stream), a);
   return launch_status("pool_append_kernel");
+}
+
+extern "C" int dspark_rows_pack(const int64_t* sources, const int32_t* first, int n_sources, int first_stride,
+                                int64_t rows, int64_t row_bytes, void* dst, int32_t* nonfinite, void* stream) {
+  clear_error();
+  DSPARK_REQUIRE(sources && first && nonfinite, "null pointer argument");
+  DSPARK_REQUIRE(n_sources >= 1 && first_stride >= 1 && rows >= 1, "sizes must be positive");
+  DSPARK_REQUIRE(row_bytes >= 16 && row_bytes % 16 == 0 && row_bytes < (1LL << 31),
+                 "row bytes must be a positive multiple of 16 below 2^31");
+  DSPARK_REQUIRE(aligned16(dst), "buffers must be 16-byte aligned");
+  const int64_t blocks = (rows + PACK_ROWS - 1) / PACK_ROWS;
+  DSPARK_REQUIRE(blocks <= 0xffffffLL, "too many rows");
+  PackArgs a{sources, first, n_sources, first_stride, rows, (int)(row_bytes / 16), static_cast<u32x4*>(dst), nonfinite};
+  hipLaunchKernelGGL(rows_pack_kernel, dim3((unsigned)blocks), dim3(256), 0, static_cast<hipStream_t>(stream), a);
+  return launch_status("rows_pack_kernel");
 }

@@ -489,7 +489,8 @@ class DraftKVPool:
         self._slots = {}
         self._free = list(range(slots))
         self._attention = HipDraftAttention(self.device, chunk=chunk) if (heads, dim) == (KV_HEADS, HEAD_DIM) else None
-        self._flag = torch.zeros(1, dtype=torch.int32, device=self.device)
+        self._flags = torch.zeros(2, dtype=torch.int32, device=self.device)   # nonfinite output, nonfinite features
+        self._flag = self._flags[:1]
         self.last_append_work = None
         if projector is not None and (projector.layers != layers or projector.device != self.device
                                       or (heads, dim, self.dtype) != (KV_HEADS, HEAD_DIM, torch.bfloat16)):
@@ -674,21 +675,37 @@ class DraftKVPool:
                 raise ValueError('Committed draft context exceeds the pool capacity')
             feats.append(value[0])
         self._reserve(max(self._lengths[r] + f.shape[0] for (r, _), f in zip(order, feats)))
-        x = (torch.cat(feats) if len(feats) > 1 else feats[0]).to(torch.bfloat16).contiguous()
         rec, first = [], 0
         for (request, _), f in zip(order, feats):
             rec += (self._slots[request], self._lengths[request], first, f.shape[0])
             first += f.shape[0]
-        records = upload(self.device, rec)
-        self._flag.zero_()
+        # Rows of whole 16-byte pieces are packed and checked by one launch;
+        # others are concatenated first (one source then).
+        whole = proj.features % 8 == 0
+        if not (whole and all(f.dtype == torch.bfloat16 and f.is_contiguous() and f.data_ptr() % 16 == 0
+                              for f in feats)):
+            feats = [(torch.cat(feats) if len(feats) > 1 else feats[0]).to(torch.bfloat16).contiguous()]
+            whole = whole and feats[0].data_ptr() % 16 == 0
+        sources = np.array([f.data_ptr() for f in feats], dtype=np.int64)
+        head = upload(self.device, np.concatenate((np.array(rec, dtype=np.int32), sources.view(np.int32))))
+        records = head[:len(rec)]
+        self._flags.zero_()
+        x = feats[0] if len(feats) == 1 else torch.empty((first, proj.features), dtype=torch.bfloat16,
+                                                         device=self.device)
+        if whole:
+            _native.call('dspark_rows_pack', head.data_ptr() + 4 * len(rec), head.data_ptr() + 8, len(feats), 4, first,
+                         2 * proj.features, x.data_ptr() if len(feats) > 1 else None, self._flags.data_ptr() + 4,
+                         _native.stream_handle(self.device))
+        else:
+            self._flags[1] = torch.isfinite(x).all().logical_not()
         proj.project_into(proj.fc_forward(x), records, len(order), self.keys, self.values, flag=self._flag)
-        bad_in, bad_out = torch.stack((torch.isfinite(x).all().logical_not().to(torch.int32), self._flag[0])).tolist()
+        bad_out, bad_in = self._flags.tolist()
         if bad_in:
             raise ValueError('Expected finite nonempty [1, tokens, target_features] on draft device')
         if bad_out:
             raise RuntimeError('Nonfinite projected draft context')
-        for request, f in zip(order, feats):
-            self._lengths[request[0]] += f.shape[0]
+        for request, value in order:
+            self._lengths[request] += value.shape[1]
         e, H, D = self._elems[0], self.heads, self.dim
         self.last_append_work = dict(requests=len(order), new_context_tokens=first, context_projection_calls=1,
                                      kv_projection_calls=self.layers, projection_launches=2,
