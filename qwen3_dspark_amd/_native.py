@@ -11,6 +11,8 @@ from .build import LIB_PATH, TIMELINE_LIB_PATH
 
 _lock = threading.Lock()
 _lib = None
+_entries = {}                # entry point name -> bound ctypes function, once loaded
+_raw_stream = None           # torch's (device index) -> hipStream_t of the current stream
 
 _P = ctypes.c_void_p
 _I = ctypes.c_int
@@ -108,10 +110,12 @@ def load():
 
 def call(name, *args):
     """Invoke an entry point and raise NativeError on a non-zero status."""
-    lib = _lib or load()
-    rc = getattr(lib, name)(*args)
+    fn = _entries.get(name)
+    if fn is None:
+        fn = _entries[name] = getattr(load(), name)
+    rc = fn(*args)
     if rc != 0:
-        raise NativeError(f'{name}: {lib.dspark_last_error().decode(errors="replace")}')
+        raise NativeError(f'{name}: {load().dspark_last_error().decode(errors="replace")}')
     return rc
 
 
@@ -127,5 +131,14 @@ def ptr(t):
 
 
 def stream_handle(device):
-    import torch
-    return torch.cuda.current_stream(device).cuda_stream
+    """hipStream_t of torch's current stream on `device`, without building a
+    torch.cuda.Stream object (3 us a call, one call per launch)."""
+    global _raw_stream
+    if _raw_stream is None:
+        import torch
+        _raw_stream = torch._C._cuda_getCurrentRawStream
+    index = device.index
+    if index is None:
+        import torch
+        index = torch.cuda.current_device()
+    return _raw_stream(index)

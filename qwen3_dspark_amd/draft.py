@@ -389,15 +389,16 @@ class HipDraftAttention:
             batch, context_keys)
         out = torch.empty(query.shape, dtype=torch.bfloat16, device=self.device)
         bound = max(batch.context_rows, 1)
-        _native.call('dspark_draft_attn_fwd', _native.ptr(query), int(query.dtype == torch.float32),
-                     _native.ptr(context_keys), _native.ptr(context_values), int(context_keys.dtype == torch.float32),
-                     _native.ptr(batch.context_indices), _native.ptr(offsets), _native.ptr(batch.ctx_len),
-                     tok_stride, head_stride, _native.ptr(block_keys), _native.ptr(block_values),
-                     _native.ptr(batch.cu_blocks), _native.ptr(batch.anchor_rows), batch.request_count, bound,
-                     batch.max_blocks, float(SCALE), chunk, _native.ptr(work), n_work, n_runs,
+        n_req = batch.request_count
+        lens = batch._device_meta().data_ptr()       # int32 [lengths | block offsets | anchors], see DraftBatch
+        _native.call('dspark_draft_attn_fwd', query.data_ptr(), int(query.dtype == torch.float32),
+                     context_keys.data_ptr(), context_values.data_ptr(), int(context_keys.dtype == torch.float32),
+                     _native.ptr(batch.context_indices), offsets.data_ptr(), lens, tok_stride, head_stride,
+                     block_keys.data_ptr(), block_values.data_ptr(), lens + 4 * n_req, lens + 4 * (2 * n_req + 1),
+                     n_req, bound, batch.max_blocks, SCALE, chunk, work.data_ptr(), n_work, n_runs,
                      self._workgroups, self.persistent or 0, _native.ptr(self._queue),
                      _native.ptr(seg_anchors) if self.persistent else None,
-                     _native.ptr(out), _native.ptr(ws), ws.numel(), _native.stream_handle(self.device))
+                     out.data_ptr(), ws.data_ptr(), ws.numel(), _native.stream_handle(self.device))
         return out
 
 

@@ -18,6 +18,8 @@ the kernels read, a fixed-capacity split-K work list and the split-K
 partials.  Every launch argument of a bucket's attention depends only on the
 bucket, so a captured launch replays for every later transaction of it.
 """
+import functools
+
 import torch
 
 from . import _native
@@ -28,6 +30,20 @@ from .schedule import REQ_INTS, WORK_INTS, run_count, segment_plan, varlen_list_
 MAX_BUCKET_REQUESTS = 4096      # requests per transaction (one metadata workgroup scans them in LDS)
 
 
+@functools.lru_cache(maxsize=1024)
+def _list_counts(requests, key_capacity, row_tiles, n_cu, chunk):
+    """(record capacity, runs) of a fixed-capacity work list; chunk None for
+    the balanced split.  A function of five numbers, asked for by every
+    launch (4 us each to work out again)."""
+    runs = run_count(key_capacity, n_cu, row_tiles)
+    return varlen_list_bound(requests, runs, key_capacity, chunk), runs
+
+
+def _list_shape(shape, device, chunk, split):
+    return _list_counts(shape.request_count, shape.key_capacity, (shape.maximum_query_length + 7) // 8,
+                        cu_count(device), None if split == 'balanced' else chunk)
+
+
 def _list_runs(shape, device):
     """Most balanced-list runs any transaction of a bucket uses (its key
     capacity bounds the keys of every transaction)."""
@@ -35,8 +51,7 @@ def _list_runs(shape, device):
 
 
 def _list_segments(shape, device, chunk, split):
-    return varlen_list_bound(shape.request_count, _list_runs(shape, device), shape.key_capacity,
-                             None if split == 'balanced' else chunk)
+    return _list_shape(shape, device, chunk, split)[0]
 
 
 def _list_ints(shape, device, chunk, split):
@@ -122,7 +137,7 @@ class HipKVDevice:
 
     def launch_shape(self, shape):
         """(record capacity, runs) of a bucket's fixed-capacity work list."""
-        return _list_segments(shape, self.device, self.chunk, self.split), _list_runs(shape, self.device)
+        return _list_shape(shape, self.device, self.chunk, self.split)
 
     # -- workspaces -----------------------------------------------------------
     def workspace(self, shape):

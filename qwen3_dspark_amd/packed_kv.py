@@ -150,7 +150,6 @@ class AppendOrderKV:
         self.kv = self._rebuild(self.rows + n_new, added=projected)
         self._record(chunks, n_new)
 
-    @torch.no_grad()
     def append_layer(self, layer, keys, values):
         """Grow one layer's K and V by keys / values [1, H, n, D] (one
         launch) and return the layer's new [1, H, rows + n, D] tensors: what

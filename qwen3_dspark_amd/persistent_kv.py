@@ -639,7 +639,6 @@ class PersistentTargetKV:
         keys, values = self.kv_device.gather(ws, tx.bucket, layer)
         return keys, values, ws.cu_query, ws.cu_key, ws.positions
 
-    @torch.no_grad()
     def attend(self, tx, layer, query, *, scale=SCALE, keys=None, values=None, out=None):
         """Bottom-right causal attention of one layer: request r's queries see
         its committed rows (resident) then its new rows, read in place.

@@ -309,3 +309,22 @@ def test_prompt_segments_follow_the_runs(ql, kl, split):
         if split == 'balanced' and ql[r] > 8 and count > 1:
             assert all(x[0] % 64 == 0 and x[1] - x[0] >= MIN_PROMPT_SEGMENT - 64 for x in segs)
             assert sum(-(-ql[x[0]] // PROMPT_TOKENS) for x in rec[in_runs:]) <= 64
+
+
+@pytest.mark.parametrize('ctx,chunk', [([0], 64), ([64, 65, 63, 0, 1], 64), ([700, 20, 700, 4096, 4097], 256),
+                                       ([9000] * 3, 4096), (list(range(1, 2000, 97)), 320)])
+def test_fixed_chunk_draft_list_is_the_general_one(ctx, chunk):
+    """The fixed-chunk list, written out directly, equals what _flatten makes
+    of the same segments (one per run, longest first)."""
+    from qwen3_dspark_amd.schedule import _flatten, draft_work, n_chunks
+    blocks = [[c // 2, c] if r % 2 else [c] for r, c in enumerate(ctx)]
+    cu = [0]
+    for b in blocks:
+        cu.append(cu[-1] + len(b))
+    segs = [(r, c * chunk, min(n, c * chunk + chunk)) for r, n in enumerate(ctx) for c in range(n_chunks(n, chunk))]
+    segs.sort(key=lambda s: (s[1] - s[2], s[0], s[1]))
+    want = _flatten(len(ctx), [[s] for s in segs],
+                    lambda r, k0, k1, slot: (r, k0, k1, slot, cu[r], cu[r + 1] - cu[r], ctx[r], 10 * r + 1),
+                    lambda r, first, count: (first, count, cu[r], cu[r + 1] - cu[r]))
+    got = draft_work(ctx, cu, [a for b in blocks for a in b], chunk=chunk, offsets=[10 * r for r in range(len(ctx))])
+    assert got == want
