@@ -433,15 +433,21 @@ extern "C" int dspark_pool_gather(const void* k_src, const void* v_src, int64_t 
 //   crop_plan    : keep = (request != marker) | (position < length)
 //                  (packed_target.py:99-108) as a stable compaction: the
 //                  source row of every kept output row, and the compacted
-//                  markers/positions.  Tile counts, a one-workgroup scan of
-//                  the tile totals, then a per-tile scan that scatters.
+//                  markers/positions.  One launch up to CROP_DIRECT_ROWS
+//                  rows; beyond, tile counts, a one-workgroup scan of the
+//                  tile totals, then the scatter.
 //   rows_rebuild : every layer's K and V rebuilt in one launch, output row j
 //                  taken from plan[j] (crop) or, without a plan, from the old
 //                  rows then the appended rows (append: the reference's cat).
 // ---------------------------------------------------------------------------
 namespace dspark {
 
-constexpr int PLAN_TILE = 4096;            // rows per tile (256 threads x 16)
+constexpr int PLAN_TILE = 4096;            // rows per count of the three-launch plan
+constexpr int CROP_ROWS = 1024;            // rows (and threads) per workgroup that writes the plan
+constexpr int CROP_WAVES = CROP_ROWS / WAVE;
+// Most rows planned by crop_direct_kernel alone (at 32,768: 9.9 us
+// against 16 for count, scan and scatter; at 65,536: 17.8 against 16).
+constexpr int64_t CROP_DIRECT_ROWS = 32768;
 constexpr int REBUILD_MAX_LAYERS = 64;
 
 struct CropPlanArgs {
@@ -491,34 +497,69 @@ __global__ __launch_bounds__(LAYOUT_THREADS) void crop_scan_kernel(CropPlanArgs 
   }
 }
 
-// Per tile: rows in order, 16 consecutive rows per thread, block scan of the
-// per-thread counts; kept rows scatter to their output slot.
-__global__ __launch_bounds__(256) void crop_scatter_kernel(CropPlanArgs a) {
-  __shared__ int s_tmp[256];
-  const int64_t base = (int64_t)blockIdx.x * PLAN_TILE + (int64_t)threadIdx.x * 16;
-  int kept = 0;
-  for (int k = 0; k < 16; ++k) {
-    const int64_t i = base + k;
-    if (i < a.n && crop_keeps(a, i)) ++kept;
+// The kept rows among CROP_ROWS rows from `base`, one per thread, written in
+// order from output row `out`: a ballot ranks a wave's rows, the totals of the
+// 16 waves (s_wave, read after one barrier) rank the waves, so the loads and
+// all but the edges of the stores are contiguous.  `mine` rides along: every
+// wave's sum of it is added up and shifts the output (rows kept before `base`).
+// Returns the output row after the tile's last.
+__device__ __forceinline__ int64_t crop_tile(const CropPlanArgs& a, int64_t base, int64_t out, int mine, int* s_wave) {
+  const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x >> 6;
+  const int64_t i = base + threadIdx.x;
+  int64_t kr = 0, kp = 0;
+  bool keep = false;
+  if (i < a.n) {
+    kr = a.kr[i];
+    kp = a.kp[i];
+    keep = kr != a.marker || kp < a.length;
   }
-  s_tmp[threadIdx.x] = kept;
+  #pragma unroll
+  for (int off = WAVE / 2; off; off >>= 1) mine += __shfl_xor(mine, off);
+  const unsigned long long kept = __ballot(keep);
+  if (lane == 0) {
+    s_wave[wave] = __popcll(kept);
+    s_wave[CROP_WAVES + wave] = mine;
+  }
   __syncthreads();
-  for (int off = 1; off < 256; off <<= 1) {   // Hillis-Steele inclusive scan
-    const int v = threadIdx.x >= off ? s_tmp[threadIdx.x - off] : 0;
-    __syncthreads();
-    s_tmp[threadIdx.x] += v;
-    __syncthreads();
+  int64_t end = out;
+  #pragma unroll
+  for (int w = 0; w < CROP_WAVES; ++w) {
+    const int n = s_wave[w];
+    out += s_wave[CROP_WAVES + w] + (w < wave ? n : 0);
+    end += s_wave[CROP_WAVES + w] + n;
   }
-  int64_t out = a.tile_kept[blockIdx.x] + s_tmp[threadIdx.x] - kept;
-  for (int k = 0; k < 16; ++k) {
-    const int64_t i = base + k;
-    if (i < a.n && crop_keeps(a, i)) {
-      a.plan[out] = i;
-      a.out_kr[out] = a.kr[i];
-      a.out_kp[out] = a.kp[i];
-      ++out;
-    }
+  if (keep) {
+    const int64_t o = out + __popcll(kept & ((1ULL << lane) - 1));
+    a.plan[o] = i;
+    a.out_kr[o] = kr;
+    a.out_kp[o] = kp;
   }
+  return end;
+}
+
+// The whole plan in one launch for caches of at most CROP_DIRECT_ROWS rows:
+// the workgroup of a tile first counts the rows kept before it (8 independent
+// coalesced rows a thread in flight), which re-reads at most 16 bytes x that
+// many rows from the L2, and needs neither the counts nor the scan below.
+// Bound by the latency of a few dependent memory trips.  3,600 rows: 4.1 us,
+// where the three launches with 16 consecutive rows per thread took 28.7; 16,384
+// rows 6.2 against 30.9.
+__global__ __launch_bounds__(CROP_ROWS) void crop_direct_kernel(CropPlanArgs a) {
+  __shared__ int s_wave[2 * CROP_WAVES];
+  const int64_t base = (int64_t)blockIdx.x * CROP_ROWS;
+  int before = 0;
+  #pragma unroll 8
+  for (int64_t i = threadIdx.x; i < base; i += CROP_ROWS) before += a.kr[i] != a.marker || a.kp[i] < a.length;
+  crop_tile(a, base, 0, before, s_wave);
+}
+
+// Larger caches, after the counts and their scan.
+__global__ __launch_bounds__(CROP_ROWS) void crop_scatter_kernel(CropPlanArgs a) {
+  __shared__ int s_wave[PLAN_TILE / CROP_ROWS][2 * CROP_WAVES];
+  int64_t out = a.tile_kept[blockIdx.x];
+  #pragma unroll
+  for (int k = 0; k < PLAN_TILE / CROP_ROWS; ++k)
+    out = crop_tile(a, (int64_t)blockIdx.x * PLAN_TILE + k * CROP_ROWS, out, 0, s_wave[k]);
 }
 
 struct RebuildArgs {
@@ -575,9 +616,13 @@ extern "C" int dspark_crop_plan(const int64_t* key_requests, const int64_t* key_
                  plan, out_requests, out_positions, (n + PLAN_TILE - 1) / PLAN_TILE};
   DSPARK_REQUIRE(a.tiles <= 0x7fffffffLL, "dspark_crop_plan: too many rows");
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (n <= CROP_DIRECT_ROWS) {
+    hipLaunchKernelGGL(crop_direct_kernel, dim3((unsigned)((n + CROP_ROWS - 1) / CROP_ROWS)), dim3(CROP_ROWS), 0, s, a);
+    return launch_status("dspark_crop_plan");
+  }
   hipLaunchKernelGGL(crop_count_kernel, dim3((unsigned)a.tiles), dim3(256), 0, s, a);
   hipLaunchKernelGGL(crop_scan_kernel, dim3(1), dim3(LAYOUT_THREADS), 0, s, a);
-  hipLaunchKernelGGL(crop_scatter_kernel, dim3((unsigned)a.tiles), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(crop_scatter_kernel, dim3((unsigned)a.tiles), dim3(CROP_ROWS), 0, s, a);
   return launch_status("dspark_crop_plan");
 }
 
