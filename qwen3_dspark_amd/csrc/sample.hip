@@ -19,6 +19,7 @@
 // tape of draws fixes every integer outcome.  All probability arithmetic is
 // float64 (the model's logits are bf16 or fp32).
 #include <cfloat>
+#include <type_traits>
 
 #include "common.h"
 
@@ -90,24 +91,52 @@ constexpr double EXP_L1 = 0x1.62e42fefa0000p-6;      // ln2/32, high 37 bits
 constexpr double EXP_L2 = 0x1.cf79abc9e3b3ap-45;      // ln2/32 - L1
 
 struct LawScale {
-  double T, rT;
+  double T, rT, rL;       // the temperature, 1/T and what rounding 1/T left off
   bool fast;
   __device__ __forceinline__ double operator()(double x) const {
     if (!fast) return x / T;
     const double q = __dmul_rn(x, rT);
     return __fma_rn(__fma_rn(-q, T, x), rT, q);
   }
+  // The same quotient for a fast T: x (rT + rL) rounded once, to 2^-53 of an ulp.
+  __device__ __forceinline__ double near(double x) const { return __fma_rn(x, rT, __dmul_rn(x, rL)); }
 };
 
 inline LawScale law_scale(double T) {
-  return LawScale{T, 1.0 / T, T >= 0x1p-100 && T <= 0x1p100};
+  const double rT = 1.0 / T;
+  return LawScale{T, rT, std::fma(-rT, T, 1.0) / T, T >= 0x1p-100 && T <= 0x1p100};
 }
 
-// tab: LAW_EXP_TAB, or a copy of it in LDS (stage_exp_table).
+// Copies the table into LDS; the caller's next barrier publishes it.  (One
+// copy: 16 copies, in which no two lanes of a read share a bank, measured the
+// same; the vector units are the bound.)
+__device__ __forceinline__ void stage_exp_table(double* lds) {
+  for (int i = threadIdx.x; i < 64; i += blockDim.x) lds[i] = LAW_EXP_TAB[i];
+}
+
+// The table of law_exp_normal: 2^(j/32) with j << 15 taken off its high word,
+// and l_j / t_j.
+__device__ __forceinline__ void stage_exp_normal_table(double* lds) {
+  for (int j = threadIdx.x; j < 32; j += blockDim.x) {
+    const double t = LAW_EXP_TAB[2 * j];
+    lds[2 * j] = __hiloint2double(__double2hiint(t) - (j << 15), __double2loint(t));
+    lds[2 * j + 1] = LAW_EXP_TAB[2 * j + 1] / t;
+  }
+}
+
+// k = rint(x) for |x| < 2^31 by adding and taking away 1.5 * 2^52 (where a
+// double's ulp is 1, so the sum is rounded as rint rounds); n is its low word.
+__device__ __forceinline__ double round_to_int(double x, int& n) {
+  const double shifted = __dadd_rn(x, 0x1.8p52);
+  n = (int)__double_as_longlong(shifted);
+  return __dsub_rn(shifted, 0x1.8p52);
+}
+
+// tab: the table in LDS.
 __device__ __forceinline__ double law_exp(double z, const double* tab) {
   z = fmax(z, -746.0);
-  const double k = rint(__dmul_rn(z, EXP_INV_L));
-  const int n = (int)k;
+  int n;
+  const double k = round_to_int(__dmul_rn(z, EXP_INV_L), n);
   const double r = __fma_rn(-k, EXP_L2, __fma_rn(-k, EXP_L1, z));
   double c = __fma_rn(r, 1.0 / 720, 1.0 / 120);
   c = __fma_rn(r, c, 1.0 / 24);
@@ -118,14 +147,39 @@ __device__ __forceinline__ double law_exp(double z, const double* tab) {
   return ldexp(__dadd_rn(t.x, __fma_rn(t.x, p, t.y)), n >> 5);
 }
 
-// Copies the table into LDS; the caller's next barrier publishes it.
-__device__ __forceinline__ void stage_exp_table(double* lds) {
-  if (threadIdx.x < 64) lds[threadIdx.x] = LAW_EXP_TAB[threadIdx.x];
+// exp(z) for z in [-708, 0] (a normal result; NaN gives NaN) in 14 vector
+// instructions instead of law_exp's 20: no clamp, k rounded by one fused
+// operation, and 2^(k >> 5) 2^(j/32) formed by adding k << 15 to the table's high
+// word, u, from which exp(z) = u + u (p + l_j / t_j) is rounded once.  Measured
+// error <= 0.52 ulp (tests/test_law_ratio.py).
+__device__ __forceinline__ double law_exp_normal(double z, const double* tab) {
+  const double shifted = __fma_rn(z, EXP_INV_L, 0x1.8p52);
+  const int n = (int)__double_as_longlong(shifted);
+  const double k = __dsub_rn(shifted, 0x1.8p52);
+  const double r = __fma_rn(-k, EXP_L2, __fma_rn(-k, EXP_L1, z));
+  double c = __fma_rn(r, 1.0 / 720, 1.0 / 120);
+  c = __fma_rn(r, c, 1.0 / 24);
+  c = __fma_rn(r, c, 1.0 / 6);
+  c = __fma_rn(r, c, 0.5);
+  const double p = __fma_rn(__dmul_rn(r, r), c, r);
+  const double2 t = *reinterpret_cast<const double2*>(tab + 2 * (n & 31));
+  const double u = __hiloint2double(__double2hiint(t.x) + (n << 15), __double2loint(t.x));
+  return __fma_rn(u, __dadd_rn(p, t.y), u);
+}
+
+// e / S for e = exp(z) in [0, 1] and S in [1, 2^31]: the product with rS = 1/S
+// and one fused correction step, as in LawScale, in 3 instructions where a
+// division takes 11.  The correctly rounded quotient for e >= 2^-960; below,
+// where the correction's remainder is subnormal, within one ulp.
+__device__ __forceinline__ double law_ratio(double e, double S, double rS) {
+  const double q = __dmul_rn(e, rS);
+  return __fma_rn(__fma_rn(-q, S, e), rS, q);
 }
 
 // p(v) = exp(x_v / T - M) / S.
-__device__ __forceinline__ double law_p(double x, const LawScale& sc, double M, double S, const double* tab) {
-  return law_exp(sc(x) - M, tab) / S;
+__device__ __forceinline__ double law_p(double x, const LawScale& sc, double M, double S, double rS,
+                                        const double* tab) {
+  return law_ratio(law_exp(sc(x) - M, tab), S, rS);
 }
 
 // Block-wide sum for 256 threads (4 waves); `buf` holds 4 doubles.
@@ -148,7 +202,10 @@ __device__ __forceinline__ double block_sum(double x, double* buf) {
 // values in registers (bf16 and fp32 logits are exact in float) between the
 // max and the sum.  A full chunk of a 16-byte aligned row is read with
 // 16-byte loads (a wave reads 1 KiB contiguous per load); other chunks with
-// element loads.
+// element loads.  Bound by the vector units: a value costs law_exp_normal, two
+// conversions, the quotient and the max and min, about 23 instructions of 4
+// cycles (31 with law_exp, its clamp and a finiteness check per value).  512
+// rows of 151,936 bf16 logits: 74 us, with law_exp 81; the 156 MB would take 31.
 // ---------------------------------------------------------------------------
 constexpr int ST_THREADS = 256;
 constexpr int ST_PER = ST_CHUNK / ST_THREADS;   // logits per thread
@@ -158,8 +215,9 @@ __global__ __launch_bounds__(ST_THREADS) void row_stats_kernel(const void* logit
                                                                LawScale sc, int chunks, double* stats,
                                                                int32_t* bad) {
   constexpr int VEC = DT == 0 ? 8 : 4;                 // logits per 16-byte load
-  __shared__ double buf[4];
+  __shared__ double buf[8];
   __shared__ __attribute__((aligned(16))) double tab[64];
+  __shared__ __attribute__((aligned(16))) double normal_tab[64];
   const int row = blockIdx.x / chunks;
   const int c = blockIdx.x - row * chunks;
   const int v0 = c * ST_CHUNK;
@@ -169,6 +227,7 @@ __global__ __launch_bounds__(ST_THREADS) void row_stats_kernel(const void* logit
   const bool vec = v1 - v0 == ST_CHUNK && ((base * (DT == 0 ? 2 : 4)) & 15) == 0 &&
                    ((uintptr_t)logits & 15) == 0;        // uniform over the workgroup
   stage_exp_table(tab);
+  stage_exp_normal_table(normal_tab);
   // Values this thread does not hold are -inf: they leave the max alone and
   // add exp(-inf) = 0 to the sum.
   float xs[ST_PER];
@@ -188,8 +247,6 @@ __global__ __launch_bounds__(ST_THREADS) void row_stats_kernel(const void* logit
         for (int u = 0; u < VEC; ++u) xs[VEC * j + u] = v[u];
       }
     }
-    #pragma unroll
-    for (int i = 0; i < ST_PER; ++i) nonfinite |= !isfinite(xs[i]);
   } else {
     // value i of this thread: element tid + ST_THREADS * i (when below v1)
     #pragma unroll
@@ -200,25 +257,43 @@ __global__ __launch_bounds__(ST_THREADS) void row_stats_kernel(const void* logit
       nonfinite |= held && !isfinite(xs[i]);
     }
   }
-  float xmax = -INFINITY;
+  float xmax = -INFINITY, xmin = INFINITY;                 // of the values that are not NaN
   #pragma unroll
-  for (int i = 0; i < ST_PER; ++i) xmax = fmaxf(xmax, xs[i]);
+  for (int i = 0; i < ST_PER; ++i) {
+    xmax = fmaxf(xmax, xs[i]);
+    xmin = fminf(xmin, xs[i]);
+  }
   #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) xmax = fmaxf(xmax, __shfl_xor(xmax, off));
+  for (int off = 32; off >= 1; off >>= 1) {
+    xmax = fmaxf(xmax, __shfl_xor(xmax, off));
+    xmin = fminf(xmin, __shfl_xor(xmin, off));
+  }
   const int wave = tid >> 6;
-  if ((tid & 63) == 0) buf[wave] = xmax;
-  __syncthreads();   // also publishes the exp table
+  if ((tid & 63) == 0) {
+    buf[wave] = xmax;
+    buf[4 + wave] = xmin;
+  }
+  __syncthreads();   // also publishes the exp tables
   const double m = sc((double)fmaxf(fmaxf(buf[0], buf[1]), fmaxf(buf[2], buf[3])));
+  const double zmin = sc((double)fminf(fminf(buf[4], buf[5]), fminf(buf[6], buf[7]))) - m;
   double sum = 0.0;
-  if (sc.fast) {
+  if (sc.fast && vec && zmin >= -708.0) {
+    // Every term is normal (an infinity leaves zmin below, or NaN), and a NaN
+    // makes its thread's sum NaN.
+    #pragma unroll
+    for (int i = 0; i < ST_PER; ++i) sum += law_exp_normal(sc.near((double)xs[i]) - m, normal_tab);
+    nonfinite = sum != sum;
+  } else if (sc.fast) {
     // finite x / T stays finite: only the logits need the check
+    #pragma unroll
+    for (int i = 0; i < ST_PER; ++i) nonfinite |= vec && !isfinite(xs[i]);
     #pragma unroll
     for (int i = 0; i < ST_PER; ++i) sum += law_exp(sc((double)xs[i]) - m, tab);
   } else {
     #pragma unroll
     for (int i = 0; i < ST_PER; ++i) {
       const double y = (double)xs[i] / sc.T;
-      nonfinite |= (vec || v0 + tid + ST_THREADS * i < v1) && !isfinite(y);
+      nonfinite |= (vec || v0 + tid + ST_THREADS * i < v1) && !isfinite(y);   // also a logit's own
       sum += law_exp(y - m, tab);
     }
   }
@@ -230,13 +305,31 @@ __global__ __launch_bounds__(ST_THREADS) void row_stats_kernel(const void* logit
   if (__builtin_amdgcn_ballot_w64(nonfinite) && (tid & 63) == 0 && bad) bad[row] = 1;   // vector store
 }
 
-// Combined (max, sum) of one row from its chunk statistics.
-__device__ __forceinline__ void row_law(const double* stats, int row, int chunks, double& M, double& S) {
-  const double* st = stats + 2 * (int64_t)row * chunks;
+// Combined (max, sum) of one row from its chunk statistics, by one wave: each
+// lane forms the term of one chunk, then every lane adds them up in chunk
+// order.  `terms` holds 2 x 64 doubles of this wave's LDS.
+__device__ __forceinline__ void row_law(const double* stats, int64_t row, int chunks, const double* tab, double* terms,
+                                        double& M, double& S) {
+  const int lane = threadIdx.x & (WAVE - 1);
+  const double2* st = reinterpret_cast<const double2*>(stats) + row * chunks;
   M = -INFINITY;
-  for (int c = 0; c < chunks; ++c) M = fmax(M, st[2 * c]);
+  for (int c = lane; c < chunks; c += WAVE) M = fmax(M, st[c].x);
+  #pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) M = fmax(M, __shfl_xor(M, off));
   S = 0.0;
-  for (int c = 0; c < chunks; ++c) S += st[2 * c + 1] * law_exp(st[2 * c] - M, LAW_EXP_TAB);
+  for (int c0 = 0; c0 < chunks; c0 += WAVE) {
+    const int n = min(WAVE, chunks - c0);
+    if (lane < n) {
+      const double2 x = st[c0 + lane];
+      terms[2 * lane] = x.y;
+      terms[2 * lane + 1] = law_exp(x.x - M, tab);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    for (int i = 0; i < n; ++i) S += terms[2 * i] * terms[2 * i + 1];
+    __builtin_amdgcn_wave_barrier();
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -255,7 +348,7 @@ __device__ __forceinline__ void row_law(const double* stats, int row, int chunks
 // within about an ulp of a boundary can land on the neighbouring index.
 // ---------------------------------------------------------------------------
 constexpr int NSEG = 256;                 // segments per job
-constexpr int SEG_SLICES = 32;            // segment-sum workgroups per job
+constexpr int SEG_SLICES = 64;            // segment-sum workgroups per job: a segment per wave
 constexpr int SEG_PER_SLICE = NSEG / SEG_SLICES;
 static_assert(SEG_PER_SLICE % 4 == 0, "each wave sums the same number of segments");
 
@@ -281,52 +374,75 @@ struct DrawSrc {
   int vocab;
 };
 
-__device__ __forceinline__ double draw_value(const DrawSrc& s, const DrawJob& j, int v, const double* tab) {
-  if (j.kind == DK_PROBS) return s.probs[j.src + v];
-  const double p = law_p(load_logit(s.logits, s.dtype, j.src + v), s.sc, j.M, j.S, tab);
-  return j.kind == DK_RESIDUAL ? fmax(p - s.q[j.qrow + v], 0.0) : p;
-}
-
 __device__ __forceinline__ void segment_bounds(int seg, int vocab, int& s0, int& s1) {
   const int per = (vocab + NSEG - 1) / NSEG;
   s0 = min(seg * per, vocab);
   s1 = min(s0 + per, vocab);
 }
 
-// This lane's share of one segment's sum and last index of positive mass:
-// values v = s0 + lane + 64 i in increasing order (the order of a plain
-// strided loop), their loads issued SEG_BATCH strips at a time (indices
-// clamped into the segment, values past it dropped) so that a wave waits
-// for one round trip per batch instead of one per strip.
-constexpr int SEG_BATCH = 8;
+// A segment is read in strips of 64 values, a value per lane, a batch of strips
+// at a time: their loads are all issued first (indices clamped into the
+// segment; values past it are not used), so that a wave waits for one round
+// trip per batch instead of one per strip.  Strips past a segment's end are
+// formed in vain and a long batch holds more registers than waves can share:
+// 64 residual draws over 151,936 tokens, segment sums with batches of 2, 4, 5
+// and 8: 21.4, 21.6, 21.1 and 26.4 us; 64 draws from materialised laws with 4,
+// 5 and 8: 15.3, 14.2 and 15.2 us.
+constexpr int SEG_BATCH = 5;
 
+// This lane's values v0 + 64 u of a job, unnormalised for RESIDUAL.
 template <int KIND, int DT>
-__device__ __forceinline__ void segment_part(const DrawSrc& src, const DrawJob& j, int s0, int s1, int lane,
+__device__ __forceinline__ void segment_values(const DrawSrc& src, const DrawJob& j, double rS, int v0, int s1,
+                                               const double* tab, double (&r)[SEG_BATCH]) {
+  double x[SEG_BATCH], qv[SEG_BATCH];
+  #pragma unroll
+  for (int u = 0; u < SEG_BATCH; ++u) {
+    const int v = min(v0 + WAVE * u, s1 - 1);
+    if (KIND == DK_PROBS) x[u] = src.probs[j.src + v];
+    else x[u] = DT == 0 ? (double)(float)static_cast<const bf16*>(src.logits)[j.src + v]
+                        : (double)static_cast<const float*>(src.logits)[j.src + v];
+    if (KIND == DK_RESIDUAL) qv[u] = src.q[j.qrow + v];
+  }
+  #pragma unroll
+  for (int u = 0; u < SEG_BATCH; ++u) {
+    r[u] = KIND == DK_PROBS ? x[u] : law_p(x[u], src.sc, j.M, j.S, rS, tab);
+    if (KIND == DK_RESIDUAL) r[u] = fmax(r[u] - qv[u], 0.0);
+  }
+}
+
+// f(integral constants KIND, DT) of a job (uniform across its workgroup); PROBS:
+// the launch's jobs all draw from materialised laws, else none does.
+template <bool PROBS, class F>
+__device__ __forceinline__ void with_job_kind(const DrawSrc& src, const DrawJob& j, F f) {
+  using std::integral_constant;
+  if (PROBS) f(integral_constant<int, DK_PROBS>{}, integral_constant<int, 0>{});
+  else if (src.dtype == 0 && j.kind == DK_LAW) f(integral_constant<int, DK_LAW>{}, integral_constant<int, 0>{});
+  else if (src.dtype == 0) f(integral_constant<int, DK_RESIDUAL>{}, integral_constant<int, 0>{});
+  else if (j.kind == DK_LAW) f(integral_constant<int, DK_LAW>{}, integral_constant<int, 1>{});
+  else f(integral_constant<int, DK_RESIDUAL>{}, integral_constant<int, 1>{});
+}
+
+// This lane's share of one segment's sum and last index of positive mass, in
+// increasing order.
+template <int KIND, int DT>
+__device__ __forceinline__ void segment_part(const DrawSrc& src, const DrawJob& j, double rS, int s0, int s1, int lane,
                                              const double* tab, double& part, int& last) {
   for (int v0 = s0 + lane; v0 < s1; v0 += WAVE * SEG_BATCH) {
-    double x[SEG_BATCH], qv[SEG_BATCH];
-    #pragma unroll
-    for (int u = 0; u < SEG_BATCH; ++u) {
-      const int v = min(v0 + WAVE * u, s1 - 1);
-      if (KIND == DK_PROBS) x[u] = src.probs[j.src + v];
-      else x[u] = DT == 0 ? (double)(float)static_cast<const bf16*>(src.logits)[j.src + v]
-                          : (double)static_cast<const float*>(src.logits)[j.src + v];
-      if (KIND == DK_RESIDUAL) qv[u] = src.q[j.qrow + v];
-    }
+    double r[SEG_BATCH];
+    segment_values<KIND, DT>(src, j, rS, v0, s1, tab, r);
     #pragma unroll
     for (int u = 0; u < SEG_BATCH; ++u) {
       const int v = v0 + WAVE * u;
-      double r = KIND == DK_PROBS ? x[u] : law_p(x[u], src.sc, j.M, j.S, tab);
-      if (KIND == DK_RESIDUAL) r = fmax(r - qv[u], 0.0);
       if (v < s1) {
-        part += r;
-        if (r > 0.0) last = v;
+        part += r[u];
+        if (r[u] > 0.0) last = v;
       }
     }
   }
 }
 
 // grid: jobs x SEG_SLICES; each wave sums SEG_PER_SLICE / 4 segments.
+template <bool PROBS>
 __global__ __launch_bounds__(256) void segment_sums_kernel(DrawSrc src, const DrawJob* jobs, double* segsum,
                                                            int32_t* seglast) {
   __shared__ __attribute__((aligned(16))) double tab[64];
@@ -334,8 +450,11 @@ __global__ __launch_bounds__(256) void segment_sums_kernel(DrawSrc src, const Dr
   const int slice = blockIdx.x - job * SEG_SLICES;
   const DrawJob j = jobs[job];
   if (j.kind == DK_NONE) return;                    // uniform across the workgroup
-  stage_exp_table(tab);
-  __syncthreads();
+  if (!PROBS) {
+    stage_exp_table(tab);
+    __syncthreads();
+  }
+  const double rS = 1.0 / j.S;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   for (int i = 0; i < SEG_PER_SLICE / 4; ++i) {
@@ -344,14 +463,9 @@ __global__ __launch_bounds__(256) void segment_sums_kernel(DrawSrc src, const Dr
     segment_bounds(seg, src.vocab, s0, s1);
     double part = 0.0;
     int last = -1;
-    if (j.kind == DK_PROBS)
-      segment_part<DK_PROBS, 0>(src, j, s0, s1, lane, tab, part, last);
-    else if (src.dtype == 0)
-      j.kind == DK_LAW ? segment_part<DK_LAW, 0>(src, j, s0, s1, lane, tab, part, last)
-                       : segment_part<DK_RESIDUAL, 0>(src, j, s0, s1, lane, tab, part, last);
-    else
-      j.kind == DK_LAW ? segment_part<DK_LAW, 1>(src, j, s0, s1, lane, tab, part, last)
-                       : segment_part<DK_RESIDUAL, 1>(src, j, s0, s1, lane, tab, part, last);
+    with_job_kind<PROBS>(src, j, [&](auto kind, auto dt) {
+      segment_part<decltype(kind)::value, decltype(dt)::value>(src, j, rS, s0, s1, lane, tab, part, last);
+    });
     #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
       part += __shfl_xor(part, off);
@@ -392,13 +506,16 @@ __device__ __forceinline__ bool is_stop(const int32_t* stops, int n_stops, int64
 }
 
 // grid: jobs; 256 threads (thread t owns segment t).
+template <bool PROBS>
 __global__ __launch_bounds__(256) void draw_kernel(DrawSrc src, const DrawJob* jobs, const double* segsum,
                                                    const int32_t* seglast, DrawOut o) {
   __shared__ double scan[NSEG];
   __shared__ double buf[4];
   __shared__ int found[2];
+  __shared__ __attribute__((aligned(16))) double tab[64];
   const DrawJob j = jobs[blockIdx.x];
   if (j.kind == DK_NONE) return;                    // uniform across the workgroup
+  stage_exp_table(tab);                         // read after the barriers below
   const int t = threadIdx.x;
   const int lane = t & 63;
   const int wave = t >> 6;
@@ -439,15 +556,29 @@ __global__ __launch_bounds__(256) void draw_kernel(DrawSrc src, const DrawJob* j
       segment_bounds(seg, src.vocab, s0, s1);
       double run = seg ? scan[seg - 1] : 0.0;
       int hit = INT32_MAX, pos = -1;
-      for (int v0 = s0; v0 < s1 && hit == INT32_MAX; v0 += WAVE) {
-        const int v = v0 + lane;
-        const double r = v < s1 ? draw_value(src, j, v, LAW_EXP_TAB) / norm : 0.0;
-        if (r > 0.0) pos = v;
-        const double incl = run + wave_inclusive_scan(r, lane);
-        const unsigned long long over = __builtin_amdgcn_ballot_w64(v < s1 && incl > j.u);
-        if (over) hit = v0 + __builtin_ctzll(over);
-        run = __shfl(incl, WAVE - 1);
-      }
+      with_job_kind<PROBS>(src, j, [&](auto kind, auto dt) {
+        for (int b0 = s0; b0 < s1 && hit == INT32_MAX; b0 += WAVE * SEG_BATCH) {
+          double r[SEG_BATCH], incl[SEG_BATCH];
+          segment_values<decltype(kind)::value, decltype(dt)::value>(src, j, 1.0 / j.S, b0 + lane, s1,
+                                                                     tab, r);
+          #pragma unroll
+          for (int u = 0; u < SEG_BATCH; ++u) {
+            r[u] = b0 + WAVE * u + lane < s1 ? r[u] / norm : 0.0;
+            incl[u] = wave_inclusive_scan(r[u], lane);
+          }
+          #pragma unroll
+          for (int u = 0; u < SEG_BATCH; ++u) {
+            const int v = b0 + WAVE * u + lane;
+            if (hit == INT32_MAX && b0 + WAVE * u < s1) {        // uniform across the wave
+              if (r[u] > 0.0) pos = v;
+              const double sum = run + incl[u];
+              const unsigned long long over = __builtin_amdgcn_ballot_w64(v < s1 && sum > j.u);
+              if (over) hit = b0 + WAVE * u + __builtin_ctzll(over);
+              run = __shfl(sum, WAVE - 1);
+            }
+          }
+        }
+      });
       // no crossing reproduced: the segment's last index of positive mass
       #pragma unroll
       for (int off = 32; off >= 1; off >>= 1) pos = max(pos, __shfl_xor(pos, off));
@@ -500,20 +631,31 @@ struct VerifyArgs {
 
 constexpr int MAX_PROPOSAL = 255;          // draft tokens per request in one verification
 
-// One wave per request: the lanes form every row's (max, sum) and every
-// proposed token's acceptance ratio min(1, p/q) in parallel, then lane 0
-// walks the proposal in order.
-__global__ __launch_bounds__(64) void verify_plan_kernel(VerifyArgs a) {
+// One workgroup per request: its waves form the rows' (max, sum) a row at a
+// time and its threads every proposed token's acceptance ratio min(1, p/q), and
+// all that the walk over the proposal reads is put into LDS; then thread 0 walks
+// the proposal in order.  The kernel is a chain of memory trips: with one lane
+// per row's chunks and the walk reading global memory it took 13.5 us for 64
+// proposals of 7 tokens, now 7.2.
+constexpr int PLAN_WAVES = 8;
+
+__global__ __launch_bounds__(PLAN_WAVES * WAVE) void verify_plan_kernel(VerifyArgs a) {
   __shared__ double alpha[MAX_PROPOSAL];
   __shared__ double law[2 * (MAX_PROPOSAL + 1)];
+  __shared__ double uniform[MAX_PROPOSAL + 1];
+  __shared__ int64_t token[MAX_PROPOSAL];
+  __shared__ bool stops_at[MAX_PROPOSAL];
+  __shared__ int s_err;
+  __shared__ double terms[PLAN_WAVES][2 * WAVE];
+  __shared__ __attribute__((aligned(16))) double tab[64];
   const int r = blockIdx.x;
-  const int lane = threadIdx.x;
+  const int tid = threadIdx.x;
   const int row0 = a.cu_rows[r];
   const int n = a.cu_rows[r + 1] - row0 - 1;
   const int d0 = row0 - r;
   const int V = a.vocab;
-  if (n < 0 || n > MAX_PROPOSAL) {                       // wave-uniform; nothing else is read
-    if (lane == 0) {
+  if (n < 0 || n > MAX_PROPOSAL) {                       // uniform; nothing else is read
+    if (tid == 0) {
       DrawJob job{};
       job.kind = DK_NONE;
       job.req = r;
@@ -524,48 +666,58 @@ __global__ __launch_bounds__(64) void verify_plan_kernel(VerifyArgs a) {
     }
     return;
   }
-  int err = VE_OK;
-  for (int j = lane; j <= n; j += WAVE) {
-    if (a.bad[row0 + j]) err = max(err, 3 * 16);            // ordered: logits, then token range, then zero q
+  if (tid == 0) s_err = 0;
+  stage_exp_table(tab);
+  __syncthreads();
+  // MAX_PROPOSAL + 1 rows at most, fewer than threads: thread j has row j and token j.
+  static_assert(MAX_PROPOSAL < PLAN_WAVES * WAVE, "a thread per row");
+  const int j = tid;
+  double qj = 0.0;
+  if (j <= n) {
+    int err = 0;                                            // ordered: logits, then token range, then zero q
+    uniform[j] = a.uniforms[row0 + j];
+    if (a.bad[row0 + j]) err = 3;
     if (j < n) {
       const int64_t tok = a.tokens[d0 + j];
-      if (tok < 0 || tok >= V) err = max(err, 2 * 16);
-    }
-  }
-  #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) err = max(err, __shfl_xor(err, off));
-  if (err == 0) {
-    for (int j = lane; j < n; j += WAVE)
-      if (!(a.q[(int64_t)(d0 + j) * V + a.tokens[d0 + j]] > 0.0)) err = 1 * 16;
-    #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) err = max(err, __shfl_xor(err, off));
-  }
-  err = err == 3 * 16 ? VE_LOGITS : (err == 2 * 16 ? VE_TOKEN : (err == 1 * 16 ? VE_ZERO_Q : VE_OK));
-  if (err == VE_OK) {
-    for (int j = lane; j <= n; j += WAVE) {
-      double M, S;
-      row_law(a.stats, row0 + j, a.chunks, M, S);
-      law[2 * j] = M;
-      law[2 * j + 1] = S;
-      if (j < n) {
-        const int64_t tok = a.tokens[d0 + j];
-        const double p = law_p(load_logit(a.logits, a.dtype, (int64_t)(row0 + j) * a.row_stride + tok), a.sc, M, S,
-                               LAW_EXP_TAB);
-        alpha[j] = fmin(p / a.q[(int64_t)(d0 + j) * V + tok], 1.0);
+      token[j] = tok;
+      stops_at[j] = is_stop(a.stops, a.n_stops, tok);
+      if (tok < 0 || tok >= V) {
+        err = max(err, 2);
+      } else {
+        qj = a.q[(int64_t)(d0 + j) * V + tok];
+        if (!(qj > 0.0)) err = max(err, 1);
       }
     }
+    if (err) atomicMax(&s_err, err);
   }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __syncthreads();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-  if (lane != 0) return;
+  int err = s_err == 3 ? VE_LOGITS : (s_err == 2 ? VE_TOKEN : (s_err == 1 ? VE_ZERO_Q : VE_OK));
+  if (err == VE_OK) {                                       // uniform across the workgroup
+    for (int i = tid / WAVE; i <= n; i += PLAN_WAVES) {
+      double M, S;
+      row_law(a.stats, row0 + i, a.chunks, tab, terms[tid / WAVE], M, S);
+      if ((tid & (WAVE - 1)) == 0) {
+        law[2 * i] = M;
+        law[2 * i + 1] = S;
+      }
+    }
+    __syncthreads();
+    if (j < n) {
+      const double M = law[2 * j], S = law[2 * j + 1];
+      const double p = law_p(load_logit(a.logits, a.dtype, (int64_t)(row0 + j) * a.row_stride + token[j]), a.sc, M, S,
+                             1.0 / S, tab);
+      alpha[j] = fmin(p / qj, 1.0);
+    }
+    __syncthreads();
+  }
+  if (tid != 0) return;
   int emitted = 0, accepted = 0, rejected = -1, extra = EX_NONE, stop = ST_ROUND, draws = 0, final_row = -1;
   if (err == VE_OK && a.budget[r] == 0) {
     stop = ST_BUDGET;
   } else if (err == VE_OK) {
     bool done = false;
     for (int j = 0; j < n && !done; ++j) {
-      const double u = a.uniforms[row0 + draws++];
+      const double u = uniform[draws++];
       if (!(u >= 0.0 && u < 1.0)) {
         err = VE_UNIFORM;
         break;
@@ -578,10 +730,10 @@ __global__ __launch_bounds__(64) void verify_plan_kernel(VerifyArgs a) {
         done = true;
         break;
       }
-      const int64_t tok = a.tokens[d0 + j];
+      const int64_t tok = token[j];
       a.out_tokens[row0 + emitted++] = tok;
       accepted = j + 1;
-      if (is_stop(a.stops, a.n_stops, tok)) {
+      if (stops_at[j]) {
         stop = ST_EOS;
         done = true;
       } else if (emitted == a.budget[r]) {
@@ -600,7 +752,7 @@ __global__ __launch_bounds__(64) void verify_plan_kernel(VerifyArgs a) {
   job.req = r;
   job.out = row0;
   if (err == VE_OK && final_row >= 0) {
-    const double u = a.uniforms[row0 + draws++];
+    const double u = uniform[draws++];
     if (!(u >= 0.0 && u < 1.0)) {
       err = VE_UNIFORM;
     } else {
@@ -627,17 +779,35 @@ __global__ __launch_bounds__(64) void verify_plan_kernel(VerifyArgs a) {
 // ---------------------------------------------------------------------------
 // Materialised laws and plain categorical draws (the draft's proposal side).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void probs_kernel(const void* logits, int dtype, int64_t row_stride, int vocab,
-                                                    LawScale sc, const double* stats, int chunks, double* probs) {
+// grid: (ceil(vocab / PROBS_TILE), rows).  A thread forms PROBS_PER values of its
+// workgroup's tile, 256 apart, all loads issued first.  Bound by writing the law
+// (8 bytes a value): 64 rows of 151,936 fp32 logits, 117 MB, in 26
+// us; with every thread forming the row's law itself and dividing, 37.
+constexpr int PROBS_PER = 16;
+constexpr int PROBS_TILE = 256 * PROBS_PER;
+
+template <int DT>   // 0: bf16 logits, 1: fp32
+__global__ __launch_bounds__(256) void probs_kernel(const void* logits, int64_t row_stride, int vocab, LawScale sc,
+                                                    const double* stats, int chunks, double* probs) {
+  __shared__ double terms[4][2 * WAVE];
   __shared__ __attribute__((aligned(16))) double tab[64];
+  const int row = blockIdx.y;
+  const int64_t v0 = (int64_t)blockIdx.x * PROBS_TILE + threadIdx.x;
+  const int64_t base = (int64_t)row * row_stride;
+  float x[PROBS_PER];                                       // both logit types are exact in float
+  #pragma unroll
+  for (int i = 0; i < PROBS_PER; ++i)
+    x[i] = (float)load_logit(logits, DT, base + min<int64_t>(v0 + 256 * i, vocab - 1));
   stage_exp_table(tab);
   __syncthreads();
-  const int row = blockIdx.y;
   double M, S;
-  row_law(stats, row, chunks, M, S);
-  const int64_t base = (int64_t)row * row_stride;
-  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < vocab; v += gridDim.x * blockDim.x)
-    probs[(int64_t)row * vocab + v] = law_p(load_logit(logits, dtype, base + v), sc, M, S, tab);
+  row_law(stats, row, chunks, tab, terms[threadIdx.x / WAVE], M, S);
+  const double rS = 1.0 / S;
+  #pragma unroll
+  for (int i = 0; i < PROBS_PER; ++i) {
+    const int64_t v = v0 + 256 * i;
+    if (v < vocab) probs[(int64_t)row * vocab + v] = law_p((double)x[i], sc, M, S, rS, tab);
+  }
 }
 
 __global__ __launch_bounds__(256) void row_jobs_kernel(int rows, int vocab, const double* uniforms, DrawJob* jobs) {
@@ -687,14 +857,15 @@ namespace {
 // [jobs: DrawJob][segment sums: double x 256][segment last indices: int32 x 256] per job
 int64_t draw_workspace(int jobs) { return (int64_t)jobs * ((int64_t)sizeof(DrawJob) + NSEG * 12); }
 
+template <bool PROBS>
 int launch_draws(const DrawSrc& src, DrawJob* jobs, int n_jobs, const DrawOut& o, hipStream_t s) {
   double* segsum = reinterpret_cast<double*>(jobs + n_jobs);
   int32_t* seglast = reinterpret_cast<int32_t*>(segsum + (int64_t)n_jobs * NSEG);
-  hipLaunchKernelGGL(segment_sums_kernel, dim3((unsigned)((int64_t)n_jobs * SEG_SLICES)), dim3(256), 0, s, src, jobs,
+  hipLaunchKernelGGL(segment_sums_kernel<PROBS>, dim3((unsigned)((int64_t)n_jobs * SEG_SLICES)), dim3(256), 0, s, src, jobs,
                      segsum, seglast);
   int rc = launch_status("segment_sums_kernel");
   if (rc != OK) return rc;
-  hipLaunchKernelGGL(draw_kernel, dim3(n_jobs), dim3(256), 0, s, src, jobs, segsum, seglast, o);
+  hipLaunchKernelGGL(draw_kernel<PROBS>, dim3(n_jobs), dim3(256), 0, s, src, jobs, segsum, seglast, o);
   return launch_status("draw_kernel");
 }
 }  // namespace
@@ -724,12 +895,12 @@ extern "C" int dspark_spec_verify(const void* logits, int dtype, int64_t row_str
   VerifyArgs a{logits, dtype, row_stride, vocab, law_scale(temperature), stats, stat_chunks(vocab), bad, cu_rows, tokens, q,
                uniforms, budget, stops, n_stops, n_req, out_tokens, out_meta, jobs};
   hipStream_t s = static_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(verify_plan_kernel, dim3(n_req), dim3(64), 0, s, a);
+  hipLaunchKernelGGL(verify_plan_kernel, dim3(n_req), dim3(PLAN_WAVES * WAVE), 0, s, a);
   int rc = launch_status("verify_plan_kernel");
   if (rc != OK) return rc;
   const DrawSrc src{logits, dtype, law_scale(temperature), q, nullptr, vocab};
   const DrawOut o{out_tokens, out_meta, budget, stops, n_stops};
-  return launch_draws(src, jobs, n_req, o, s);
+  return launch_draws<false>(src, jobs, n_req, o, s);
 }
 
 extern "C" int dspark_logits_to_probs(const void* logits, int dtype, int rows, int vocab, int64_t row_stride,
@@ -740,9 +911,13 @@ extern "C" int dspark_logits_to_probs(const void* logits, int dtype, int rows, i
   DSPARK_REQUIRE(rows >= 1 && rows <= 65535 && vocab >= 1 && row_stride >= vocab,
                  "need rows in [1, 65535], vocab >= 1 and row_stride >= vocab");
   DSPARK_REQUIRE(temperature > 0.0 && temperature < DBL_MAX, "temperature must be finite and positive");
-  const unsigned gx = (unsigned)std::min<int64_t>((vocab + 255) / 256, 64);
-  hipLaunchKernelGGL(probs_kernel, dim3(gx, rows), dim3(256), 0, static_cast<hipStream_t>(stream), logits, dtype,
-                     row_stride, vocab, law_scale(temperature), stats, stat_chunks(vocab), probs);
+  const dim3 grid((unsigned)(((int64_t)vocab + PROBS_TILE - 1) / PROBS_TILE), rows);
+  if (dtype == 0)
+    hipLaunchKernelGGL(probs_kernel<0>, grid, dim3(256), 0, static_cast<hipStream_t>(stream), logits, row_stride, vocab,
+                       law_scale(temperature), stats, stat_chunks(vocab), probs);
+  else
+    hipLaunchKernelGGL(probs_kernel<1>, grid, dim3(256), 0, static_cast<hipStream_t>(stream), logits, row_stride, vocab,
+                       law_scale(temperature), stats, stat_chunks(vocab), probs);
   return launch_status("probs_kernel");
 }
 
@@ -760,5 +935,5 @@ extern "C" int dspark_sample_rows(const double* probs, int rows, int vocab, cons
   if (rc != OK) return rc;
   const DrawSrc src{nullptr, 0, law_scale(1.0), nullptr, probs, vocab};
   const DrawOut o{out, nullptr, nullptr, nullptr, 0};
-  return launch_draws(src, jobs, rows, o, s);
+  return launch_draws<true>(src, jobs, rows, o, s);
 }
