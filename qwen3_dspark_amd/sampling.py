@@ -10,7 +10,7 @@ per-request loop of packed_sampling.py:250-259).
         last row; EOS and the budget stop early
 
 Four launches for the whole batch: per-(row, chunk) max / sum-of-exp
-statistics of the logits; one lane per request for the accept / reject
+statistics of the logits; one workgroup per request for the accept / reject
 decisions; then the final categorical draws (a float64 CDF over the
 vocabulary as 256 segment sums per draw from a wide grid, and one workgroup
 per draw that scans them and walks the segment holding u).

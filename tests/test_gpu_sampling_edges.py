@@ -57,3 +57,21 @@ def test_verification(counts, vocab):
         assert as_tuple(got[r]) == (ref.tokens, ref.accepted_draft_tokens, ref.rejected_index, ref.extra_token_kind,
                                     ref.stop_reason), r
         assert got[r].draws == ref.draws
+
+
+@pytest.mark.parametrize('value', [float('nan'), float('inf'), -float('inf'), 3.0e38, -3.0e38, -600.0])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float32])
+def test_a_value_of_a_full_chunk(dtype, value):
+    """A full aligned chunk whose terms are all normal takes the short exp; one
+    NaN or infinity in it is refused, and one finite value whose term underflows
+    takes the general exp."""
+    from qwen3_dspark_amd.sampling import logits_to_probabilities
+    gen = torch.Generator(device=DEV).manual_seed(SEED)
+    logits = torch.randn(4, 3 * 8192, generator=gen, device=DEV).to(dtype)
+    logits[2, 8192 + 4321] = value
+    if not np.isfinite(value):
+        with pytest.raises(ValueError, match='finite'):
+            logits_to_probabilities(logits, 0.8)
+        return
+    ref = oracle.logits_to_probabilities(logits.float().cpu().numpy(), 0.8)
+    np.testing.assert_allclose(logits_to_probabilities(logits, 0.8).cpu().numpy(), ref, rtol=1e-12, atol=1e-300)
