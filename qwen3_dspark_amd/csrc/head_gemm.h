@@ -29,6 +29,10 @@
 // the weights are read once per workgroup and shared by the 8 waves, with 2
 // stages in flight.  The last two stages issue nothing (the waits count
 // down to zero instead), so no load outlives the tile.
+//
+// With TG = 1 the workgroup is 4 waves for 32 tokens (tg = 0, dh = w & 1, kq =
+// w >> 1): the same sums in the same order, in stages of 40 KiB, of which the
+// ring holds 4.  For so few tokens that the 64-token tiles leave CUs idle.
 #pragma once
 #include "common.h"
 
@@ -43,11 +47,20 @@ constexpr int HG_SUB = 2;                        // sub-stages per ring stage (o
 constexpr int HG_STAGES = 3;                     // ring depth (2 stages in flight)
 constexpr int HG_W_BYTES = HD * HG_KB * 2;       // 128 weight rows x 128 B = 16 KiB
 constexpr int HG_X_BYTES = 16 * HG_KB * 2;       // 16 token rows x 128 B
-constexpr int HG_SUB_BYTES = HG_W_BYTES + 4 * HG_X_BYTES;     // 24 KiB
-constexpr int HG_STAGE_BYTES = HG_SUB * HG_SUB_BYTES;         // 48 KiB
-constexpr int HG_SMEM = HG_STAGES * HG_STAGE_BYTES;            // 144 KiB
+
+// The ring of a tile of 32 TG tokens.
+template <int TG>
+struct HeadRing {
+  static constexpr int WAVES = 4 * TG;
+  static constexpr int STAGES = TG == 2 ? HG_STAGES : 4;
+  static constexpr int SUB_BYTES = HG_W_BYTES + 2 * TG * HG_X_BYTES;     // 24 or 20 KiB
+  static constexpr int STAGE_BYTES = HG_SUB * SUB_BYTES;                 // 48 or 40 KiB
+  static constexpr int SMEM = STAGES * STAGE_BYTES;                      // 144 or 160 KiB
+  static constexpr int PIECES = 16 / WAVES;                              // weight pieces per wave and sub-stage
+  static constexpr int LOADS = HG_SUB * (PIECES + 1);                    // loads per thread and stage
+};
+constexpr int HG_SMEM = HeadRing<2>::SMEM;
 constexpr int HG_COLS = HG_KB * HG_SUB;          // hidden columns per ring stage (hidden must be a multiple)
-static_assert(HG_STAGES == 3, "the ring's wait counts assume one stage in flight behind the current one");
 
 // LDS reused once the ring is drained: the K-half exchange (32 KiB), the
 // row sums of squares of the token rows (2 KiB) and the per-token partial
@@ -62,22 +75,24 @@ static_assert(HG_ROW_OFF + 2 * 4 * 32 * 4 <= HG_SMEM, "epilogue scratch exceeds 
 __device__ __forceinline__ int hg_swz(int row) { return (row >> 1) & 7; }
 
 // Where this lane's values live (see the layout above).
-struct HeadLane {
+template <int TG>
+struct HeadLaneOf {
   int n, hl, tg, dh, kq;
-  __device__ __forceinline__ HeadLane() {
+  __device__ __forceinline__ HeadLaneOf() {
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     n = lane & 31;
     hl = lane >> 5;
-    tg = wave & 1;
-    dh = (wave >> 1) & 1;
-    kq = wave >> 2;
+    tg = TG == 2 ? wave & 1 : 0;
+    dh = (wave >> (TG - 1)) & 1;
+    kq = wave >> TG;
   }
   // first of the 4 consecutive dims of v[a][4 jj .. 4 jj + 3]
   __device__ __forceinline__ int dim(int a, int jj) const { return 32 * (dh + 2 * a) + 8 * (2 * kq + jj) + 4 * hl; }
   // the lane's token within the workgroup's tile
   __device__ __forceinline__ int token() const { return 32 * tg + n; }
 };
+using HeadLane = HeadLaneOf<2>;
 
 // w: first of the head's 128 weight rows (row stride `hidden`); x: token
 // rows (row stride `hidden`), `tokens` of them; t0: the workgroup's first
@@ -88,28 +103,29 @@ struct HeadLane {
 // value in all lanes of that token).  The exchange is read after the
 // function's last barrier: afterwards the caller may use only the
 // HG_ROW_OFF region (head_row_sumsq) of the ring's LDS.
-template <bool SUMSQ, typename PreCombine>
+template <bool SUMSQ, int TG = 2, typename PreCombine>
 __device__ __forceinline__ void head_tile_gemm(const bf16* __restrict__ w, const bf16* __restrict__ x, int tokens,
                                                int hidden, int t0, unsigned char* smem, float (&v)[2][8], float& ss,
                                                PreCombine&& pre_combine) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  const HeadLane L;
+  using Ring = HeadRing<TG>;
+  const HeadLaneOf<TG> L;
   const int steps = hidden / HG_COLS;
 
   // Direct loads: lane L of a 1 KiB piece (8 rows x 128 B) fetches row
   // 8*piece + L/8, global chunk (L%8) ^ swz(row), landing at LDS chunk L%8.
-  // Wave w loads weight pieces 2w, 2w+1 and token rows 8w .. 8w+7.
+  // Wave w loads PIECES weight pieces from PIECES w on and token rows 8w .. 8w+7.
   const uint32_t smem_lds = lds_address(smem);
   const int prow = lane >> 3;
   auto issue = [&](int step) {
     #pragma unroll
     for (int sub = 0; sub < HG_SUB; ++sub) {
-      const uint32_t base = smem_lds + (uint32_t)((step % HG_STAGES) * HG_STAGE_BYTES + sub * HG_SUB_BYTES);
+      const uint32_t base = smem_lds + (uint32_t)((step % Ring::STAGES) * Ring::STAGE_BYTES + sub * Ring::SUB_BYTES);
       const int k0 = (step * HG_SUB + sub) * HG_KB;
       #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int piece = 2 * wave + i;
+      for (int i = 0; i < Ring::PIECES; ++i) {
+        const int piece = Ring::PIECES * wave + i;
         const int row = 8 * piece + prow;
         const bf16* src = w + (size_t)row * hidden + k0 + 8 * ((lane & 7) ^ hg_swz(row));
         lds_dma16(src, __builtin_amdgcn_readfirstlane(base + (uint32_t)(piece * 1024)));
@@ -127,17 +143,19 @@ __device__ __forceinline__ void head_tile_gemm(const bf16* __restrict__ w, const
     #pragma unroll
     for (int r = 0; r < 16; ++r) acc[a][r] = 0.f;
   ss = 0.f;
-  issue(0);
-  if (steps > 1) issue(1);
+  #pragma unroll
+  for (int i = 0; i < Ring::STAGES - 1; ++i)
+    if (i < steps) issue(i);
   const int R = L.token();
   for (int s = 0; s < steps; ++s) {
-    // this thread's stage-s loads landed (stage s + 1, when there is one,
-    // may still be in flight: its 3 loads per sub-stage) ...
-    if (s + 1 < steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * HG_SUB) : "memory");
+    // this thread's stage-s loads landed (the STAGES - 2 stages behind it, as
+    // far as there are any, may still be in flight) ...
+    if (Ring::STAGES == 4 && s + 2 < steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * Ring::LOADS) : "memory");
+    else if (s + 1 < steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(Ring::LOADS) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     asm volatile("s_barrier" ::: "memory");            // ... and everyone else's
-    if (s + 2 < steps) issue(s + 2);
-    const unsigned char* wst = smem + (s % HG_STAGES) * HG_STAGE_BYTES + L.kq * HG_SUB_BYTES;
+    if (s + Ring::STAGES - 1 < steps) issue(s + Ring::STAGES - 1);
+    const unsigned char* wst = smem + (s % Ring::STAGES) * Ring::STAGE_BYTES + L.kq * Ring::SUB_BYTES;
     const unsigned char* xst = wst + HG_W_BYTES;
     #pragma unroll
     for (int ks = 0; ks < HG_KB / 16; ++ks) {
@@ -154,6 +172,7 @@ __device__ __forceinline__ void head_tile_gemm(const bf16* __restrict__ w, const
         acc[a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wa, xb, acc[a], 0, 0, 0);
       }
     }
+    if (TG == 1) __builtin_amdgcn_sched_barrier(0);    // no barrier of the next stage above these MFMAs' reads
   }
   pre_combine();
   __syncthreads();   // every wave is done with the ring: reuse it for the exchange
@@ -161,7 +180,7 @@ __device__ __forceinline__ void head_tile_gemm(const bf16* __restrict__ w, const
   // Reduce-scatter of the K halves: wave kq hands over registers
   // 8 (1 - kq) .. + 7 and keeps 8 kq .. + 7.  Slots are [pair][kq][quad][lane]
   // f32x4, so each 16-byte LDS access of a wave is contiguous.
-  const int pair = wave & 3;
+  const int pair = wave & (2 * TG - 1);
   f32x4* xch = reinterpret_cast<f32x4*>(smem + HG_XCH_OFF);
   #pragma unroll
   for (int a = 0; a < 2; ++a)
@@ -186,14 +205,15 @@ __device__ __forceinline__ void head_tile_gemm(const bf16* __restrict__ w, const
       #pragma unroll
       for (int i = 0; i < 4; ++i) v[a][4 * q + i] = (L.kq == 0 ? acc[a][4 * q + i] : acc[a][8 + 4 * q + i]) + o[i];
     }
-  if (SUMSQ) ss += ssx[(wave ^ 4) * 64 + lane];  // the other column half of the row
+  if (SUMSQ) ss += ssx[(wave ^ (2 * TG)) * 64 + lane];  // the other column half of the row
 }
 
 // sum over the 128 dims of v^2 for the lane's token.  Every wave of the
 // workgroup must call it (it holds a barrier); all lanes of a token get the
 // same value.
+template <int TG = 2>
 __device__ __forceinline__ float head_row_sumsq(const float (&v)[2][8], unsigned char* smem) {
-  const HeadLane L;
+  const HeadLaneOf<TG> L;
   float s = 0.f;
   #pragma unroll
   for (int a = 0; a < 2; ++a)
@@ -207,19 +227,22 @@ __device__ __forceinline__ float head_row_sumsq(const float (&v)[2][8], unsigned
 }
 
 // The lane's 16 norm weights of a [128] RMSNorm weight vector.
-struct HeadNormW {
+template <int TG>
+struct HeadNormWOf {
   bf16x4 w[2][2];
   __device__ __forceinline__ void load(const bf16* __restrict__ nw) {
-    const HeadLane L;
+    const HeadLaneOf<TG> L;
     #pragma unroll
     for (int a = 0; a < 2; ++a)
       #pragma unroll
       for (int jj = 0; jj < 2; ++jj) w[a][jj] = *reinterpret_cast<const bf16x4*>(nw + L.dim(a, jj));
   }
 };
+using HeadNormW = HeadNormWOf<2>;
 
 // RMSNorm y = w x / sqrt(mean(x^2) + eps) with the row's sum of squares.
-__device__ __forceinline__ void head_rms_norm(float (&v)[2][8], const HeadNormW& nw, float eps, float sumsq) {
+template <int TG>
+__device__ __forceinline__ void head_rms_norm(float (&v)[2][8], const HeadNormWOf<TG>& nw, float eps, float sumsq) {
   const float r = rsqrtf(sumsq * (1.0f / HD) + eps);
   #pragma unroll
   for (int a = 0; a < 2; ++a)
@@ -230,11 +253,12 @@ __device__ __forceinline__ void head_rms_norm(float (&v)[2][8], const HeadNormW&
 }
 
 // cos / sin of the lane's 8 rotary angles (dims L.dim(0, jj) + i < 64).
-struct HeadRope {
+template <int TG>
+struct HeadRopeOf {
   f32x4 c[2], s[2];
   // from a precomputed row: cos of the 64 angles, then their sin (float32)
   __device__ __forceinline__ void load(const float* __restrict__ row) {
-    const HeadLane L;
+    const HeadLaneOf<TG> L;
     #pragma unroll
     for (int jj = 0; jj < 2; ++jj) {
       c[jj] = *reinterpret_cast<const f32x4*>(row + L.dim(0, jj));
@@ -243,7 +267,7 @@ struct HeadRope {
   }
   // angle pos * inv_freq[d] formed in FP32, the model's float32 table
   __device__ __forceinline__ void compute(const float* __restrict__ inv_freq, float pos) {
-    const HeadLane L;
+    const HeadLaneOf<TG> L;
     #pragma unroll
     for (int jj = 0; jj < 2; ++jj) {
       const f32x4 f = *reinterpret_cast<const f32x4*>(inv_freq + L.dim(0, jj));
@@ -258,8 +282,11 @@ struct HeadRope {
   }
 };
 
+using HeadRope = HeadRopeOf<2>;
+
 // Rotate-half RoPE: (x_d, x_{d+64}) -> (x_d cos - x_{d+64} sin, x_{d+64} cos + x_d sin).
-__device__ __forceinline__ void head_rope(float (&v)[2][8], const HeadRope& r) {
+template <int TG>
+__device__ __forceinline__ void head_rope(float (&v)[2][8], const HeadRopeOf<TG>& r) {
   #pragma unroll
   for (int jj = 0; jj < 2; ++jj)
     #pragma unroll
@@ -275,8 +302,9 @@ __device__ __forceinline__ void head_rope(float (&v)[2][8], const HeadRope& r) {
 // 32 (dh + 2a) + 16 kq + 8 hl .. + 7 for a = 0, 1, after swapping one
 // 8-byte half with its partner.  Both lanes of the pair must execute it;
 // `valid` gates the store only.
+template <int TG = 2>
 __device__ __forceinline__ void head_store(const float (&v)[2][8], bf16* row, bool valid) {
-  const HeadLane L;
+  const HeadLaneOf<TG> L;
   #pragma unroll
   for (int a = 0; a < 2; ++a) {
     uint32_t pk[2][2];

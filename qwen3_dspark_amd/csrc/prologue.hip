@@ -16,8 +16,8 @@
 // model computes its position embeddings once per forward) or are formed
 // in the epilogue from the positions; both give the same bits.
 //
-// Work: one workgroup per (head, 64-token tile) on the shared 32x32x16
-// MFMA tile (head_gemm.h); all 8 waves run the epilogue on 16 dims of one
+// Work: one workgroup per (head, 64- or 32-token tile) on the shared 32x32x16
+// MFMA tile (head_gemm.h); all its waves run the epilogue on 16 dims of one
 // token per lane.  Accumulation and the epilogue are FP32; outputs are
 // rounded to bf16 once.
 #include "wide_gemm.h"
@@ -43,33 +43,34 @@ struct PrologueArgs {
   float eps;
 };
 
-// grid: 32 heads (0-15 q, 16-23 k, 24-31 v) x ceil(T / 64) token tiles, one
-// dimension (see the XCD mapping below); 8 waves.
-__global__ __launch_bounds__(HG_WAVES * WAVE) void qkv_prologue_kernel(PrologueArgs a) {
-  __shared__ __attribute__((aligned(16))) unsigned char smem[HG_SMEM];
+// grid: 32 heads (0-15 q, 16-23 k, 24-31 v) x ceil(T / (32 TG)) token tiles, one
+// dimension (see the XCD mapping below); 4 TG waves.
+template <int TG>
+__global__ __launch_bounds__(4 * TG * WAVE) void qkv_prologue_kernel(PrologueArgs a) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem[HeadRing<TG>::SMEM];
   // XCD-aware placement: workgroups are dealt round-robin over the 8 XCDs
   // (each with its own L2), so the token tiles of one head are given ids
   // that share id % 8 - the head's weight slice is then fetched from HBM by
   // one L2 and served to all of its tiles from there.
-  const int tiles = (a.tokens + HG_TOKENS - 1) / HG_TOKENS;
+  const int tiles = (a.tokens + 32 * TG - 1) / (32 * TG);
   const int xcd = blockIdx.x & 7;
   const int slot = blockIdx.x >> 3;
   const int head = xcd + 8 * (slot / tiles);
-  const int t0 = (slot % tiles) * HG_TOKENS;
+  const int t0 = (slot % tiles) * (32 * TG);
   const int kind = head < HQ ? 0 : (head < HQ + HKV ? 1 : 2);       // workgroup-uniform
   const int hh = kind == 0 ? head : (kind == 1 ? head - HQ : head - HQ - HKV);
   const bf16* w = (kind == 0 ? a.wq : (kind == 1 ? a.wk : a.wv)) + (size_t)hh * HD * a.hidden;
 
-  const HeadLane L;
+  const HeadLaneOf<TG> L;
   const int row = t0 + L.token();
   const int tok = min(row, a.tokens - 1);
-  HeadNormW nw;
-  HeadRope rope;
+  HeadNormWOf<TG> nw;
+  HeadRopeOf<TG> rope;
   float pos = 0.f;
   float v[2][8];
   float ss;
   // the epilogue's operands are fetched while the K halves are exchanged
-  head_tile_gemm<false>(w, a.x, a.tokens, a.hidden, t0, smem, v, ss, [&]() {
+  head_tile_gemm<false, TG>(w, a.x, a.tokens, a.hidden, t0, smem, v, ss, [&]() {
     if (kind < 2) {
       nw.load(kind == 0 ? a.q_norm : a.k_norm);
       if (a.rope) rope.load(a.rope + (size_t)tok * 128);
@@ -77,12 +78,12 @@ __global__ __launch_bounds__(HG_WAVES * WAVE) void qkv_prologue_kernel(PrologueA
     }
   });
   if (kind < 2) {
-    head_rms_norm(v, nw, a.eps, head_row_sumsq(v, smem));
+    head_rms_norm(v, nw, a.eps, head_row_sumsq<TG>(v, smem));
     if (!a.rope) rope.compute(a.inv_freq, pos);
     head_rope(v, rope);
   }
   bf16* out = kind == 0 ? a.q_out + (size_t)tok * Q_ROW : (kind == 1 ? a.k_out : a.v_out) + (size_t)tok * a.kv_row_stride;
-  head_store(v, out + (size_t)hh * HD, row < a.tokens);
+  head_store<TG>(v, out + (size_t)hh * HD, row < a.tokens);
 }
 
 // The same for many tokens: 128-token tiles (wide_gemm.h), two workgroups per CU.
@@ -157,6 +158,13 @@ using namespace dspark;
 // 4,096 73 / 45, 8,192 141 / 88.
 constexpr int PROLOGUE_WIDE_TOKENS = 513;
 
+// Up to here 32-token tiles are one round of the 256 CUs (one workgroup each)
+// and stream a sixth fewer bytes per workgroup with more of them in flight than
+// 64-token tiles on half of the CUs.  32- against 64-token tiles, us per
+// launch at hidden 1,024 over the weights of 28 layers: 7 tokens 9.6 / 10.2, 64
+// 10.4 / 12.1, 224 10.3 / 11.6, 256 10.3 / 11.8.
+constexpr int PROLOGUE_NARROW_TOKENS = 256;
+
 extern "C" int dspark_qkv_prologue(const void* x, const void* wq, const void* wk, const void* wv,
                                    const void* q_norm, const void* k_norm, const float* inv_freq,
                                    const int64_t* positions, const float* rope, int tokens, int hidden, float eps,
@@ -183,8 +191,13 @@ extern "C" int dspark_qkv_prologue(const void* x, const void* wq, const void* wk
     else hipLaunchKernelGGL(qkv_prologue_wide_kernel<false>, grid, dim3(WG_WAVES * WAVE), 0, s, a);
     return launch_status("qkv_prologue_wide_kernel");
   }
-  hipLaunchKernelGGL(qkv_prologue_kernel, dim3((HQ + 2 * HKV) * ((tokens + HG_TOKENS - 1) / HG_TOKENS)), dim3(HG_WAVES * WAVE), 0,
-                     static_cast<hipStream_t>(stream), a);
+  if (tokens <= PROLOGUE_NARROW_TOKENS) {
+    hipLaunchKernelGGL(qkv_prologue_kernel<1>, dim3((HQ + 2 * HKV) * ((tokens + 31) / 32)), dim3(4 * WAVE), 0,
+                       static_cast<hipStream_t>(stream), a);
+    return launch_status("qkv_prologue_kernel");
+  }
+  hipLaunchKernelGGL(qkv_prologue_kernel<2>, dim3((HQ + 2 * HKV) * ((tokens + HG_TOKENS - 1) / HG_TOKENS)),
+                     dim3(HG_WAVES * WAVE), 0, static_cast<hipStream_t>(stream), a);
   return launch_status("qkv_prologue_kernel");
 }
 
