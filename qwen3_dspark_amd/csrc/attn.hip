@@ -1586,11 +1586,11 @@ __device__ __forceinline__ bf16x8 prefill_v(uint32_t va, int t, int D) {
   return v;
 }
 
-// Raw scores S^T = K Q^T of a 32-key tile.
-__device__ __forceinline__ f32x16 prefill_scores(const bf16x8 (&qf)[8], const bf16x8 (&kf)[8]) {
-  f32x16 x = {};
+// Raw scores S^T = K Q^T of a 32-key tile, over 16-dim steps FROM .. TO - 1 on top of x.
+template <int FROM = 0, int TO = 8>
+__device__ __forceinline__ f32x16 prefill_scores(const bf16x8 (&qf)[8], const bf16x8 (&kf)[8], f32x16 x = f32x16{}) {
   #pragma unroll
-  for (int ks = 0; ks < 8; ++ks) x = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks], qf[ks], x, 0, 0, 0);
+  for (int ks = FROM; ks < TO; ++ks) x = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks], qf[ks], x, 0, 0, 0);
   return x;
 }
 
@@ -1615,21 +1615,52 @@ __device__ __forceinline__ float prefill_max(PairState& st, const f32x16& x, flo
   return (st.m == -INFINITY) ? 0.f : st.m;
 }
 
+// Probabilities as two bf16 operands of PV, so that they reach V to 15 bits: with
+// e = p / PROB_UP, ph is e rounded and pl = p - ph rounded.  PROB_UP - 1 is above
+// twice the rounding of ph, so pl is positive where p is, and an infinite value
+// row gives an infinite sum (a pl of zero or below would make it NaN).
+//
+// One operand alone (p rounded to bf16) has an error that depends on how finely
+// a row's keys are divided: a key that is the maximum of its running state has p =
+// 1 exactly, and this kernel keeps 2 states per row where one workgroup per 8
+// tokens kept 4 per segment.  Error against float64 (2-norm, logits of deviation
+// 1.5; bf16 outputs alone: 1.64e-3), one operand here / the 8-token workgroups /
+// two operands: prompts of 300 1.95 / 1.82 / 1.63e-3, of 1,024 2.07 / 1.83 / 1.63, of
+// 4,096 2.14 / 2.04 / 1.64, 200 tokens after 1,000 2.34 / 1.91 / 1.66.  Rescaling
+// whenever the maximum doubles, with one operand: 1.86, 1.91, 1.97 and
+// 2.05.  Cost of the second operand per call: 300 tokens 12.5 -> 13.3 us, 1,024
+// 22.1 -> 23.7, 2,048 39 -> 48, 4,096 92 -> 120.
+constexpr float PROB_UP = 1.0078125f;                    // 1 + 2^-7: one bf16 step
+constexpr float PROB_UP_LOG2 = 0.011227255423254f;
+
 __device__ __forceinline__ void prefill_probs(PairState& st, const f32x16& x, float m_use, float scale_log2,
-                                              bf16x8 (&pb)[2]) {
+                                              bf16x8 (&ph)[2], bf16x8 (&pl)[2]) {
+  const float shift = -m_use - PROB_UP_LOG2;
   float ps[2] = {0.f, 0.f};
   #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const float p = fast_exp2(__builtin_fmaf(x[r], scale_log2, -m_use));
-    ps[r & 1] += p;
-    pb[r >> 3][r & 7] = (bf16)p;
+  for (int r = 0; r < 16; r += 2) {
+    float e[2];
+    #pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      e[i] = fast_exp2(__builtin_fmaf(x[r + i], scale_log2, shift));
+      ps[i] += e[i];
+    }
+    const bf16x2 hi = {(bf16)e[0], (bf16)e[1]};
+    const uint32_t w = __builtin_bit_cast(uint32_t, hi);
+    const float back[2] = {__builtin_bit_cast(float, w << 16), __builtin_bit_cast(float, w & 0xffff0000u)};
+    #pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      ph[r >> 3][(r & 7) + i] = hi[i];
+      pl[r >> 3][(r & 7) + i] = (bf16)__builtin_fmaf(e[i], PROB_UP, -back[i]);
+    }
   }
-  st.l += ps[0] + ps[1];
+  st.l = __builtin_fmaf(ps[0] + ps[1], PROB_UP, st.l);
 }
 
 // A tile below every row's limit whose scores x are known: its probabilities
 // and output, and the scores of the next tile (K at LDS address ka), whose
-// MFMAs are spread among the exponentials.
+// MFMAs are spread over the search for the maximum and the exponentials, as
+// the first half of PV is over the second half of the exponentials.
 __device__ __forceinline__ f32x16 prefill_full_tile(PairState& st, const bf16x8 (&qf)[8], const f32x16& x, uint32_t ka,
                                                     uint32_t va, float scale_log2) {
   bf16x8 kf[8], vt[2][4];
@@ -1639,19 +1670,26 @@ __device__ __forceinline__ f32x16 prefill_full_tile(PairState& st, const bf16x8 
     #pragma unroll
     for (int D = 0; D < 4; ++D) vt[t][D] = prefill_v(va, t, D);
   __builtin_amdgcn_sched_barrier(0);
+  constexpr int EARLY = 3;                               // score MFMAs beside the maximum
+  f32x16 nx = prefill_scores<0, EARLY>(qf, kf);
   const float m_use = prefill_max(st, x, scale_log2);
-  bf16x8 pb[2];
-  const f32x16 nx = prefill_scores(qf, kf);
-  prefill_probs(st, x, m_use, scale_log2, pb);
+  bf16x8 ph[2], pl[2];
+  nx = prefill_scores<EARLY, 8>(qf, kf, nx);
+  prefill_probs(st, x, m_use, scale_log2, ph, pl);
   #pragma unroll
   for (int t = 0; t < 2; ++t)
     #pragma unroll
-    for (int D = 0; D < 4; ++D)
-      st.o[D] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vt[t][D], pb[t], st.o[D], 0, 0, 0);
+    for (int D = 0; D < 8; ++D)
+      st.o[D & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vt[t][D & 3], D < 4 ? ph[t] : pl[t], st.o[D & 3], 0, 0, 0);
+  #pragma unroll
+  for (int i = EARLY; i < 8; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // a score MFMA,
+    __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);   // then VALU of the first half's keys
+  }
   #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // a score MFMA,
-    __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);   // then two keys' worth of VALU
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // an MFMA of the first half's PV,
+    __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);   // then VALU of the second half's keys
   }
   __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
   return nx;
@@ -1668,8 +1706,8 @@ __device__ __forceinline__ void prefill_edge_tile(PairState& st, f32x16 x, uint3
   for (int r = 0; r < 16; ++r)
     if (acc_row(r, 0) >= lim) x[r] = -INFINITY;
   const float m_use = prefill_max(st, x, scale_log2);
-  bf16x8 pb[2];
-  prefill_probs(st, x, m_use, scale_log2, pb);
+  bf16x8 ph[2], pl[2];
+  prefill_probs(st, x, m_use, scale_log2, ph, pl);
   typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
   const int lane = threadIdx.x & 63;
   #pragma unroll 1
@@ -1688,7 +1726,8 @@ __device__ __forceinline__ void prefill_edge_tile(PairState& st, f32x16 x, uint3
           keep[i] = row + 1 < lim_h ? 0xffffffffu : (row < lim_h ? 0xffffu : 0u);
         }
         const bf16x8 v = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4_t, prefill_v(va, t, D)) & keep);
-        o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v, pb[t], o, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v, ph[t], o, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v, pl[t], o, 0, 0, 0);
       }
       #pragma unroll
       for (int e = 0; e < 16; ++e) st.o[D][e] = mine ? o[e] : st.o[D][e];
@@ -1929,13 +1968,16 @@ __global__ __launch_bounds__(PF_WAVES * WAVE, 2) void prefill_attn_kernel(Varlen
         prefill_edge_tile(st, x, v_at(s), vis - kt - 8 * hh, lim0 - kt, hi - kt, a.scale_log2);
       } else {
         const float m_use = prefill_max(st, x, a.scale_log2);
-        bf16x8 pb[2];
-        prefill_probs(st, x, m_use, a.scale_log2, pb);
+        bf16x8 ph[2], pl[2];
+        prefill_probs(st, x, m_use, a.scale_log2, ph, pl);
         #pragma unroll
         for (int u = 0; u < 2; ++u)
           #pragma unroll
-          for (int D = 0; D < 4; ++D)
-            st.o[D] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(prefill_v(v_at(s), u, D), pb[u], st.o[D], 0, 0, 0);
+          for (int D = 0; D < 4; ++D) {
+            const bf16x8 v = prefill_v(v_at(s), u, D);
+            st.o[D] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v, ph[u], st.o[D], 0, 0, 0);
+            st.o[D] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v, pl[u], st.o[D], 0, 0, 0);
+          }
       }
     }
     if (turn(s + 1)) x = ahead(s + 1);

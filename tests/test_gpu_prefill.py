@@ -101,3 +101,38 @@ def test_values_past_a_rows_limit_never_reach_it():
         out = kernel(q.to(DEV), k.to(DEV), bad.to(DEV), layout, scale=SCALE)
         assert torch.equal(out[:j // 8 * 8], clean[:j // 8 * 8])
         assert not torch.isfinite(out[j:]).any()
+
+
+@pytest.mark.parametrize('q_lens,k_lens', [([300], [300]), ([1024], [1024]), ([200], [1200]), ([9, 16, 40], [700, 2000, 1064])])
+def test_error_is_that_of_the_output_rounding(q_lens, k_lens):
+    """The probabilities reach V to 15 bits and everything else is FP32, so the
+    2-norm error is the one rounding of the outputs to bf16, however few key
+    groups a request has (one bf16 probability operand is 10 to 40 % above it)."""
+    from qwen3_dspark_amd.kernels import HipVarlenKernel
+    layout, q, k, v = layout_of(q_lens, k_lens)
+    q = (q.float() * 1.5).bfloat16()
+    out = HipVarlenKernel(DEV)(q.to(DEV), k.to(DEV), v.to(DEV), layout, scale=SCALE).double().cpu()
+    wrong = rounding = 0.0
+    for a, b, n, m in zip(layout.cu_query.tolist(), layout.cu_key.tolist(), q_lens, k_lens):
+        seen = torch.arange(m)[None] <= torch.arange(m - n, m)[:, None]
+        for h in range(16):
+            x = (q[a:a + n, h].double() @ k[b:b + m, h // 2].double().t() * SCALE).masked_fill(~seen, -torch.inf)
+            ref = torch.softmax(x, -1) @ v[b:b + m, h // 2].double()
+            wrong += (out[a:a + n, h] - ref).square().sum()
+            rounding += (ref.bfloat16().double() - ref).square().sum()
+    # what is left off: probabilities at 1.5 x 2^-15 and FP32 sums, each under 1 % of
+    # the rounding's 2^-8 / sqrt(12) to the outputs' own scale
+    assert wrong.sqrt() <= 1.02 * rounding.sqrt()
+
+
+@pytest.mark.parametrize('value', [float('inf'), -float('inf')])
+def test_an_infinite_value_row_gives_its_infinity(value):
+    """Not NaN: every part of a visible key's weight has its sign.  One infinite
+    row per request; equal keys, so that its weight is far from underflow."""
+    from qwen3_dspark_amd.kernels import HipVarlenKernel
+    for n, j in ((20, 3), (64, 40), (200, 100), (300, 299)):
+        layout, q, k, v = layout_of([n], [n])
+        v[j] = value
+        k[:] = k[:1]
+        out = HipVarlenKernel(DEV)(q.to(DEV), k.to(DEV), v.to(DEV), layout, scale=SCALE)
+        assert bool((out[j:] == value).all()) and bool(torch.isfinite(out[:j // 8 * 8]).all())
