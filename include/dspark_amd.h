@@ -184,6 +184,29 @@ int dspark_verify_attn_staged_fwd(const void* q, const void* k_res, const void* 
                                   void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * The three attention calls above for a batch of prompts (more than 8 query
+ * tokens) and shorter requests, planned so that neither holds the other back:
+ *   k_new NULL:            dspark_varlen_attn_fwd (k/v [k_rows, 8, 128]; strides ignored)
+ *   k_new, k_scr NULL:     dspark_verify_attn_fwd (k_new/v_new: the staged scratch rows)
+ *   k_new and k_scr given: dspark_verify_attn_staged_fwd
+ * with the same arguments and results.  The work list has the same form, with
+ *   - after the request records, n_columns pairs (1 + record, tile): a workgroup per
+ *     KV head attends query tokens 32 tile .. 32 tile + 31 of that record's
+ *     request (more than 8 tokens) over the record's keys, started in the
+ *     order of the list ((0, 0): none).  The runs hold the records of the rest;
+ *   - partial slots counted in tiles of 8 query tokens: a segment takes
+ *     ceil(query count / 8) from its slot on, the segments of a split request one
+ *     after the other.  part_tiles of them are reserved; 0: every request record
+ *     has one segment, and nothing is merged.
+ * workspace: dspark_attn_workspace_bytes(part_tiles, 0, 1, 32) bytes (none for 0).
+ */
+int dspark_mixed_attn_fwd(const void* q, const void* k, const void* v, const void* k_new, const void* v_new,
+                          void* k_scr, void* v_scr, int n_req, int64_t slot_stride, int64_t tok_stride,
+                          int64_t head_stride, int max_q, int causal, float scale, const int32_t* work, int n_work,
+                          int n_groups, int n_columns, int part_tiles, void* out, void* workspace,
+                          int64_t workspace_bytes, void* stream);
+
+/*
  * Multi-block DSpark draft attention.  Request r owns blocks
  * cu_blocks[r]..cu_blocks[r+1] (1..8 blocks), each 7 query rows; block b
  * sees context positions j < anchors[b] of its request plus its own 7 rows

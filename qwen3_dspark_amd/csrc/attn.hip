@@ -269,11 +269,12 @@ struct VarlenArgs {
   int64_t a_tok_stride;   // segment A elements between token rows
   int64_t a_head_stride;  // segment A elements between KV heads
   const int32_t* work;    // optional segment list (see the C ABI)
+  const int32_t* columns; // mixed batches: (1 + record, 32-token tile) of every prompt workgroup
   bf16* stage_k;          // verify with staging: scratch written from segment B (k_b/v_b = new rows)
   bf16* stage_v;
   bf16* out;              // [nq, 16, 128]
-  float* part_o;          // [n_cl*8*tmax][16][128]
-  float* part_ml;         // [n_cl*8*tmax][16][2]
+  float* part_o;          // [partial tiles][16][128], see part_tile
+  float* part_ml;         // [partial tiles][16][2]
   int n_req;
   int n_work;             // segment records in the work list
   int n_slots;            // no list: (chunk, KV head) slots, 8 * chunks
@@ -320,6 +321,12 @@ __device__ __forceinline__ bool chunk_segment(const VarlenArgs& a, bool verify, 
 // 16-row tiles on, one workgroup per tile would stream the keys once per 8
 // tokens.
 constexpr int DECODE_TOKENS = 8;
+
+// Partial tile of row tile t (8 query tokens) of a segment's partial slot for KV
+// head g.  tmax 0: slots are counted in tiles, and a segment takes those of its own rows.
+__device__ __forceinline__ size_t part_tile(int slot, int g, int t, int tmax) {
+  return tmax ? ((size_t)slot * 8 + g) * tmax + t : (size_t)(slot + t) * 8 + g;
+}
 
 // The addressing of one segment for one KV head; every field is
 // wave-uniform.  Key j of the request lives in part A (committed rows) for
@@ -578,7 +585,7 @@ __device__ __forceinline__ void varlen_run(const VarlenArgs& a, unsigned char* s
       const int tok_r = row >> 1;
       const int head_r = 2 * g + (row & 1);
       if (cur.pslot >= 0) {
-        const size_t p = (size_t)(cur.pslot * 8 + g) * a.tmax;
+        const size_t p = part_tile(cur.pslot, g, 0, a.tmax);
         float* po = a.part_o + (p * 16 + row) * HD + d0;
         *reinterpret_cast<f32x4*>(po) = f32x4{acc[0], acc[1], acc[2], acc[3]};
         *reinterpret_cast<f32x4*>(po + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]};
@@ -1758,7 +1765,7 @@ __device__ __forceinline__ void prefill_merge(const VarlenArgs& a, const float* 
   L += __shfl_xor(L, 32);
   if (tok >= ql) return;
   const float inv = 1.0f / L;
-  const size_t p = (size_t)(pslot * 8 + g) * a.tmax + (tok >> 3);
+  const size_t p = part_tile(pslot, g, tok >> 3, a.tmax);
   #pragma unroll
   for (int i = 0; i < 16 / KG; ++i) {
     const int quad = kg * (16 / KG) + i;
@@ -1785,32 +1792,38 @@ __device__ __forceinline__ void prefill_merge(const VarlenArgs& a, const float* 
   }
 }
 
-// A call whose max_q exceeds DECODE_TOKENS is one launch of gridDim.x = 8 x the
-// tiles of max_q: its first `decode_rows` grid rows hold the workgroups that
-// walk the runs for the requests of up to DECODE_TOKENS (they stream from HBM
-// beside the prompts' MFMAs), then one row per segment.  Each request is
-// attended by one of the two forms by its own query count.
+// A call whose max_q exceeds DECODE_TOKENS is one launch: first the workgroups that
+// walk the runs for the requests of up to DECODE_TOKENS, then the prompts'.  With
+// `columns` (a mixed plan) those are the listed (record, tile) pairs, in the
+// order of the list, which starts with the longest; else the grid is
+// gridDim.x = 8 x the tiles of max_q wide, its first `decode_rows` rows walk
+// the runs, and one row follows per record: each request is then attended by one
+// of the two forms by its own query count.
 template <bool VERIFY>
 __global__ __launch_bounds__(PF_WAVES * WAVE, 2) void prefill_attn_kernel(VarlenArgs a, int decode_grid, int decode_rows) {
   // 1 KiB alignment: tile offsets are XORed into LDS addresses.
   __shared__ __attribute__((aligned(1024))) unsigned char smem[PF_SMEM];
   static_assert(PF_SMEM >= VARLEN_SMEM && PF_WAVES * WAVE == 256, "one launch shape for both forms");
-  int seg = blockIdx.y + PF_SEGS_Y * blockIdx.z - decode_rows;
-  if (seg < 0) {
-    const int wid = blockIdx.x + gridDim.x * (seg + decode_rows);       // keeps the XCD: gridDim.x is a multiple of 8
+  const int row = blockIdx.y + PF_SEGS_Y * blockIdx.z;
+  const int wid = (int)(blockIdx.x + gridDim.x * (unsigned)row);        // keeps the XCD: gridDim.x is a multiple of 8
+  if (a.columns ? wid < decode_grid : row < decode_rows) {
     if (wid < decode_grid) varlen_workgroup<VERIFY, true>(a, smem, wid, decode_grid);
     return;
   }
   const int g = blockIdx.x & 7;
-  const int t = (gridDim.x >> 3) - 1 - (blockIdx.x >> 3);
+  int t = (gridDim.x >> 3) - 1 - (blockIdx.x >> 3);
+  int seg = row - decode_rows;
+  if (a.columns) {
+    const int32_t* column = a.columns + 2 * ((wid - decode_grid) >> 3);
+    seg = min(__builtin_amdgcn_readfirstlane(column[0]), a.n_work) - 1;
+    t = max(__builtin_amdgcn_readfirstlane(column[1]), 0);
+  } else if (a.work) {
+    seg = a.n_work - 1 - seg;        // a plan puts its prompts after the runs, longest last
+  }
   Segment sg;
   if (a.work) {
-    // from the last record on: a plan puts its prompts after the runs, longest
-    // last, and the empty workgroups of the other records then start behind them
-    seg = a.n_work - 1 - seg;
-    if (seg < 0) return;
-    const int32_t* w = a.work + WORK_INTS * seg;
-    sg = Segment{w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7]};
+    const int32_t* w = a.work + WORK_INTS * max(seg, 0);        // no record: no query tokens
+    sg = Segment{w[0], w[1], w[2], w[3], w[4], seg < 0 ? 0 : w[5], w[6], w[7]};
   } else if (!chunk_segment(a, VERIFY, seg, sg)) {
     return;
   }
@@ -2064,8 +2077,8 @@ __global__ __launch_bounds__(256) void merge_kernel(MergeArgs a) {
     if ((row >> 1) >= step || tok >= rows) continue;
     float acc[8];
     float L;
-    merge_partials<8>(a.part_o, a.part_ml, (size_t)(first * 8 + g) * a.tmax + t, (size_t)8 * a.tmax, nch, row, d0,
-                      acc, L);
+    merge_partials<8>(a.part_o, a.part_ml, part_tile(first, g, t, a.tmax),
+                      (size_t)8 * (a.tmax ? a.tmax : (rows + 7) / 8), nch, row, d0, acc, L);
     bf16x8 ov;
     #pragma unroll
     for (int i = 0; i < 8; ++i) ov[i] = (bf16)(acc[i] / L);
@@ -2150,6 +2163,17 @@ extern "C" int64_t dspark_attn_workspace_bytes(int n_req, int64_t key_rows_bound
 
 namespace {
 
+// `grid` workgroups over the runs (or fixed chunks), then `prompts` rows of the prompt form.
+template <bool VERIFY>
+int launch_prefill(const VarlenArgs& a, unsigned grid, unsigned prompts, int max_q, hipStream_t s) {
+  const unsigned gx = HKV * ((max_q + PF_TOKENS - 1) / PF_TOKENS);
+  const unsigned decode_rows = (grid + gx - 1) / gx;
+  const unsigned rows = decode_rows + prompts;
+  hipLaunchKernelGGL(prefill_attn_kernel<VERIFY>, dim3(gx, std::min(rows, (unsigned)PF_SEGS_Y), (rows + PF_SEGS_Y - 1) / PF_SEGS_Y),
+                     dim3(256), 0, s, a, (int)grid, (int)decode_rows);
+  return launch_status("prefill_attn_kernel");
+}
+
 // Shared by the varlen and verification entry points: argument checks that
 // depend on the dispatch form, the split-K workspace layout and both launches.
 // With a work list the partial slots are bounded by its record count, else by
@@ -2183,12 +2207,7 @@ int varlen_launch(VarlenArgs& a, int64_t key_rows_bound, int max_q, float scale,
     hipLaunchKernelGGL(varlen_attn_kernel<VERIFY>, dim3(grid), dim3(256), 0, s, a);
     rc = launch_status(what);
   } else {
-    const unsigned gx = HKV * ((max_q + PF_TOKENS - 1) / PF_TOKENS);
-    const unsigned decode_rows = (grid + gx - 1) / gx;
-    const unsigned rows = decode_rows + (unsigned)n_cl;
-    hipLaunchKernelGGL(prefill_attn_kernel<VERIFY>, dim3(gx, std::min(rows, (unsigned)PF_SEGS_Y), (rows + PF_SEGS_Y - 1) / PF_SEGS_Y),
-                       dim3(256), 0, s, a, (int)grid, (int)decode_rows);
-    rc = launch_status("prefill_attn_kernel");
+    rc = launch_prefill<VERIFY>(a, grid, (unsigned)n_cl, max_q, s);
   }
   if (rc != OK) return rc;
   MergeArgs m{work ? work + WORK_INTS * n_work + n_groups + 1 : nullptr, a.cu_q, a.cu_k, nullptr, nullptr, a.part_o,
@@ -2277,6 +2296,70 @@ extern "C" int dspark_verify_attn_fwd(const void* q, const void* k_res, const vo
   return verify_launch(q, k_res, v_res, k_scr, v_scr, nullptr, nullptr, cu_q, cu_k, slots, n_req, slot_stride,
                        tok_stride, head_stride, key_rows_bound, max_q, scale, chunk, work, n_work, n_groups, out,
                        workspace, workspace_bytes_, stream);
+}
+
+extern "C" int dspark_mixed_attn_fwd(const void* q, const void* k, const void* v, const void* k_new, const void* v_new,
+                                     void* k_scr, void* v_scr, int n_req, int64_t slot_stride, int64_t tok_stride,
+                                     int64_t head_stride, int max_q, int causal, float scale, const int32_t* work,
+                                     int n_work, int n_groups, int n_columns, int part_tiles, void* out,
+                                     void* workspace, int64_t workspace_bytes_, void* stream) {
+  clear_error();
+  const bool verify = k_new != nullptr;
+  DSPARK_REQUIRE(q && k && v && work && out, "null pointer argument");
+  DSPARK_REQUIRE((k_new != nullptr) == (v_new != nullptr) && (k_scr != nullptr) == (v_scr != nullptr) && (verify || !k_scr),
+                 "k_new and v_new, k_scr and v_scr go together, and staging needs new rows");
+  DSPARK_REQUIRE(aligned16(q) && aligned16(k) && aligned16(v) && aligned16(k_new) && aligned16(v_new) && aligned16(k_scr) &&
+                 aligned16(v_scr) && aligned16(out), "Q/K/V/out must be 16-byte aligned");
+  DSPARK_REQUIRE(!verify || (slot_stride >= 0 && tok_stride >= HD && tok_stride % 8 == 0 && head_stride >= HD && head_stride % 8 == 0),
+                 "resident strides must be multiples of 8 elements (token/head strides >= 128)");
+  DSPARK_REQUIRE(!verify || causal, "verification attention is causal");
+  DSPARK_REQUIRE(max_q >= 1, "max_q must be >= 1");
+  DSPARK_REQUIRE(n_work >= 1 && n_groups >= 8 && n_groups <= (1 << 24) && n_groups % 8 == 0 && n_columns >= 0 &&
+                 n_columns <= (1 << 24), "need n_work >= 1, n_groups a multiple of 8 in [8, 2^24] and n_columns in [0, 2^24]");
+  const int tiles = (max_q + 7) / 8;
+  int rc = check_shape(n_req, 0, tiles, 32, scale);
+  if (rc != OK) return rc;
+  DSPARK_REQUIRE(part_tiles >= 0, "part_tiles must be >= 0");
+  const int64_t need = part_tiles ? dspark_attn_workspace_bytes(part_tiles, 0, 1, 32) : 0;
+  DSPARK_REQUIRE(workspace_bytes_ >= need, "workspace too small: %lld < %lld bytes", (long long)workspace_bytes_,
+                 (long long)need);
+  DSPARK_REQUIRE(need == 0 || (workspace != nullptr && aligned16(workspace)),
+                 "workspace must be a 16-byte aligned device pointer");
+  VarlenArgs a{};
+  a.q = static_cast<const bf16*>(q);
+  a.k_a = static_cast<const bf16*>(k);
+  a.v_a = static_cast<const bf16*>(v);
+  a.k_b = verify ? static_cast<const bf16*>(k_new) : a.k_a;
+  a.v_b = verify ? static_cast<const bf16*>(v_new) : a.v_a;
+  a.stage_k = static_cast<bf16*>(k_scr);
+  a.stage_v = static_cast<bf16*>(v_scr);
+  a.slot_stride = slot_stride;
+  a.a_tok_stride = verify ? tok_stride : KV_ROW;
+  a.a_head_stride = verify ? head_stride : HD;
+  a.work = work;
+  a.out = static_cast<bf16*>(out);
+  a.part_o = static_cast<float*>(workspace);
+  a.part_ml = a.part_o + (int64_t)part_tiles * HKV * 16 * HD;
+  a.n_req = n_req;
+  a.n_work = n_work;
+  a.causal = causal ? 1 : 0;
+  a.tmax = 0;
+  a.scale_log2 = scale * LOG2E;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int32_t* requests = work + WORK_INTS * n_work + n_groups + 1;
+  const unsigned grid = (unsigned)n_groups * HKV;
+  if (n_columns == 0) {
+    hipLaunchKernelGGL(verify ? varlen_attn_kernel<true> : varlen_attn_kernel<false>, dim3(grid), dim3(256), 0, s, a);
+    rc = launch_status("varlen_attn_kernel");
+  } else {
+    a.columns = requests + REQ_INTS * n_req;
+    hipLaunchKernelGGL(verify ? prefill_attn_kernel<true> : prefill_attn_kernel<false>,
+                       dim3(grid + (unsigned)n_columns * HKV), dim3(256), 0, s, a, (int)grid, 0);
+    rc = launch_status("prefill_attn_kernel");
+  }
+  if (rc != OK || part_tiles == 0) return rc;
+  MergeArgs m{requests, nullptr, nullptr, nullptr, nullptr, a.part_o, a.part_ml, a.out, n_req, 0, 0, 0};
+  return launch_merge(m, n_req, tiles, s);
 }
 
 // ---------------------------------------------------------------------------

@@ -16,7 +16,8 @@ import torch
 
 from . import _native, backends
 from ._device import Workspace, cu_count, require_gfx950
-from .schedule import DEFAULT_CHUNK, SPLITS, run_count, segment_plan, upload_work
+from .schedule import (DECODE_TOKENS, DEFAULT_CHUNK, PART_TILE_BYTES, SPLITS, mixed_plan, run_count, segment_plan,
+                       upload_work)
 
 Q_HEADS, KV_HEADS, HEAD_DIM = 16, 8, 128
 SCALE = 128 ** -0.5
@@ -102,10 +103,14 @@ class HipVarlenKernel:
                 starts.append(acc)
                 acc += k
             n_cu = cu_count(self.device)
-            runs = run_count(acc, n_cu, tiles)
-            records, n_segments, runs = segment_plan(self.split, layout.query_lengths, layout.key_lengths, starts,
-                                                     runs, self.chunk, n_cu=n_cu)
-            self._work = (upload_work(records, self.device), n_segments, runs)
+            if self.split == 'balanced' and max(layout.query_lengths) > DECODE_TOKENS:
+                plan = mixed_plan(layout.query_lengths, layout.key_lengths, starts, n_cu, causal=self.causal)
+                self._work = (upload_work(plan.records, self.device), *plan[1:])
+            else:
+                runs = run_count(acc, n_cu, tiles)
+                records, n_segments, runs = segment_plan(self.split, layout.query_lengths, layout.key_lengths, starts,
+                                                         runs, self.chunk, n_cu=n_cu)
+                self._work = (upload_work(records, self.device), n_segments, runs)
             self._work_for = key
         return self._work
 
@@ -113,7 +118,16 @@ class HipVarlenKernel:
         out = torch.empty_like(query)
         n_req = len(layout.query_lengths)
         tiles = (max_q + 7) // 8
-        work, n_work, runs = self._work_list(layout, tiles) or (None, 0, 0)
+        listed = self._work_list(layout, tiles) or (None, 0, 0)
+        if len(listed) > 3:
+            work, n_work, runs, records, columns, tiles = listed
+            ws = self._workspace.get(PART_TILE_BYTES * tiles)
+            _native.call('dspark_mixed_attn_fwd', _native.ptr(query), _native.ptr(key), _native.ptr(value), None, None,
+                         None, None, records, 0, 0, 0, max_q, int(self.causal), float(SCALE), _native.ptr(work), n_work,
+                         runs, columns, tiles, _native.ptr(out), _native.ptr(ws), ws.numel(),
+                         _native.stream_handle(self.device))
+            return out
+        work, n_work, runs = listed
         lib = _native.load()
         need = (lib.dspark_attn_workspace_bytes(n_work, 0, tiles, self.chunk) if work is not None
                 else lib.dspark_attn_workspace_bytes(n_req, key_rows, tiles, self.chunk))

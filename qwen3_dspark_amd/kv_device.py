@@ -25,7 +25,8 @@ import torch
 from . import _native
 from ._device import KV_PAIR_SKEW, cu_count, kv_pair, require_gfx950, upload
 from .kernels import HEAD_DIM, KV_HEADS, SCALE
-from .schedule import REQ_INTS, WORK_INTS, run_count, segment_plan, varlen_list_bound
+from .schedule import (DECODE_TOKENS, PART_TILE_BYTES, REQ_INTS, WORK_INTS, mixed_capacity, mixed_ints, mixed_plan, run_count,
+                       segment_plan, varlen_list_bound)
 
 MAX_BUCKET_REQUESTS = 4096      # requests per transaction (one metadata workgroup scans them in LDS)
 
@@ -39,32 +40,41 @@ def _list_counts(requests, key_capacity, row_tiles, n_cu, chunk):
     return varlen_list_bound(requests, runs, key_capacity, chunk), runs
 
 
+def _mixed_shape(shape, device, split, limit=None):
+    """The fixed capacity of a bucket's mixed plans (mixed_capacity), or None for
+    a bucket without prompts or a request-local split."""
+    if split != 'balanced' or shape.maximum_query_length <= DECODE_TOKENS:
+        return None
+    lengths = getattr(shape, 'query_lengths', None)              # a bucket's are exact, a family's bounded
+    return mixed_capacity(shape.request_count, shape.query_tokens, shape.key_capacity, shape.maximum_query_length,
+                          cu_count(device), limit, lengths is None or min(lengths) <= DECODE_TOKENS)
+
+
 def _list_shape(shape, device, chunk, split):
+    c = _mixed_shape(shape, device, split)
+    if c is not None:
+        return c.run_records + c.prompt_records, c.runs
     return _list_counts(shape.request_count, shape.key_capacity, (shape.maximum_query_length + 7) // 8,
                         cu_count(device), None if split == 'balanced' else chunk)
 
 
-def _list_runs(shape, device):
-    """Most balanced-list runs any transaction of a bucket uses (its key
-    capacity bounds the keys of every transaction)."""
-    return run_count(shape.key_capacity, cu_count(device), (shape.maximum_query_length + 7) // 8)
-
-
-def _list_segments(shape, device, chunk, split):
-    return _list_shape(shape, device, chunk, split)[0]
-
-
 def _list_ints(shape, device, chunk, split):
     """int32 length of the largest work list of a bucket."""
-    return (WORK_INTS * _list_segments(shape, device, chunk, split) + _list_runs(shape, device) + 1
-            + REQ_INTS * shape.request_count)
+    c = _mixed_shape(shape, device, split)
+    if c is not None:
+        return mixed_ints(c)
+    records, runs = _list_shape(shape, device, chunk, split)
+    return WORK_INTS * records + runs + 1 + REQ_INTS * shape.request_count
 
 
 def _partials_bytes(shape, device, chunk, split):
     """Split-K partials for the largest work list of a bucket (one slot per
     segment at most)."""
     tiles = (shape.maximum_query_length + 7) // 8
-    return max(16, int(_native.load().dspark_attn_workspace_bytes(_list_segments(shape, device, chunk, split), 0,
+    c = _mixed_shape(shape, device, split)
+    if c is not None:
+        return max(16, PART_TILE_BYTES * c.tiles)
+    return max(16, int(_native.load().dspark_attn_workspace_bytes(_list_shape(shape, device, chunk, split)[0], 0,
                                                                   tiles, chunk)))
 
 
@@ -75,6 +85,7 @@ class Workspace:
         for name, t in tensors.items():
             setattr(self, name, t)
         self._names = tuple(tensors)
+        self.mixed = None        # counts of the bucket's mixed plans (MixedPlan without its list), from the first on
 
     def tensors(self):
         return {name: getattr(self, name) for name in self._names}
@@ -191,10 +202,16 @@ class HipKVDevice:
         published if the list does not fit or a launch fails."""
         key_lengths = [c + q for c, q in zip(contexts, query_lengths)]
         n_cu = cu_count(self.device)
-        runs = run_count(sum(key_lengths), n_cu, (shape.maximum_query_length + 7) // 8)
-        records, _, _ = segment_plan(self.split, query_lengths, key_lengths, slots, runs, self.chunk,
-                                     self.launch_shape(shape), xcd_speed=self.xcd_speed,
-                                     n_cu=n_cu if self.slot_balance else None)
+        capacity = _mixed_shape(shape, self.device, self.split, ws.attn.numel() // PART_TILE_BYTES)
+        if capacity is not None:
+            plan = mixed_plan(query_lengths, key_lengths, slots, n_cu, capacity=capacity, xcd_speed=self.xcd_speed,
+                              slot_balance=self.slot_balance)
+            records, ws.mixed = plan.records, plan[1:]
+        else:
+            runs = run_count(sum(key_lengths), n_cu, (shape.maximum_query_length + 7) // 8)
+            records, _, _ = segment_plan(self.split, query_lengths, key_lengths, slots, runs, self.chunk,
+                                         self.launch_shape(shape), xcd_speed=self.xcd_speed,
+                                         n_cu=n_cu if self.slot_balance else None)
         if len(records) > ws.work.numel():
             raise ValueError('Work list exceeds the bucket workspace')
         r = len(slots)
@@ -230,6 +247,14 @@ class HipKVDevice:
         time."""
         C = self.capacity
         k, v, sk, sv = self.layer_pointers[layer]
+        if ws.mixed is not None:
+            n_work, runs, requests, columns, tiles = ws.mixed
+            new = (sk, sv, None, None) if keys is None else (keys, values, sk, sv)
+            _native.call('dspark_mixed_attn_fwd', query, k, v, *new, requests, KV_HEADS * C * HEAD_DIM, HEAD_DIM,
+                         C * HEAD_DIM, shape.maximum_query_length, 1, SCALE, ws.work.data_ptr(), n_work, runs,
+                         columns, tiles, out, ws.attn.data_ptr(), ws.attn.numel(),
+                         _native.stream_handle(self.device))
+            return
         tail = (ws.cu_query.data_ptr(), ws.cu_key.data_ptr(), ws.req.data_ptr(),
                 shape.request_count, KV_HEADS * C * HEAD_DIM, HEAD_DIM, C * HEAD_DIM,
                 shape.key_capacity, shape.maximum_query_length, SCALE, self.chunk,

@@ -33,10 +33,18 @@ head), cuts on 64-row ring-stage boundaries (draft_work).
 Requests of more than DECODE_TOKENS query tokens (prompts) are attended by a
 kernel with one workgroup per (segment, KV head, 32 query tokens); their
 segments follow the runs' records and belong to no run (prompt_segments).
+Balanced plans of batches that hold prompts have a list of their own
+(mixed_plan): the runs are cut for the other requests alone, partial slots are
+counted in tiles of 8 query tokens, and the prompts' workgroups are listed.
 
 Without a list, both kernels walk fixed chunks of `chunk` rows in request
 order over a grid sized from the row bound.
 """
+import functools
+from collections import namedtuple
+
+import numpy as np
+
 from ._device import upload
 
 DEFAULT_CHUNK = 1024          # verification / varlen: fixed chunks when no list is given
@@ -63,6 +71,10 @@ DRAFT_CHUNK = 4096
 MIN_DRAFT_CHUNK = 256         # the batch-sized draft chunk never falls below this many rows
 WORK_INTS = 8
 REQ_INTS = 4
+PART_TILE_BYTES = 8 * 16 * (128 + 2) * 4      # split-K partials of one 8-token tile, every KV head
+
+MixedCapacity = namedtuple('MixedCapacity', 'run_records prompt_records runs requests columns tiles')
+MixedPlan = namedtuple('MixedPlan', 'records n_work runs requests columns tiles')
 
 
 def n_chunks(n, chunk):
@@ -103,37 +115,38 @@ def run_count(total_keys, n_cu, row_tiles=1):
     return -(-runs // XCDS) * XCDS
 
 
-def _flatten(n, per_run, record, request, loose=()):
+def _flatten(n, per_run, record, request, loose=(), width=None):
     """Flatten per-run [(request, k0, k1)] segment lists into the int32 list
     format, giving split requests consecutive request-major partial slots in
     key order.  record(r, k0, k1, slot) and request(r, first, count) give the
     8 and 4 ints of a segment and a request.  loose: segments of no run, after
-    the runs' records.  Returns (list, segment count, run count)."""
-    count = [0] * n
+    the runs' records.  width(r): slots that a segment of request r takes (one
+    without).  Returns (list, segment count, run count)."""
     loose = list(loose)
-    for run in [*per_run, loose]:
-        for r, _, _ in run:
-            count[r] += 1
-    first, slot = [], 0
-    for c in count:
-        first.append(slot if c > 1 else -1)
-        slot += c if c > 1 else 0
-    keyed = {}
-    # partial slot of a segment = first slot of its request + its key-order rank
+    keyed = [[] for _ in range(n)]               # first keys of each request's segments
     for run in [*per_run, loose]:
         for r, k0, _ in run:
-            keyed.setdefault(r, []).append(k0)
-    rank = {r: {k0: i for i, k0 in enumerate(sorted(v))} for r, v in keyed.items()}
+            keyed[r].append(k0)
+    first, slot, rank = [], 0, {}
+    for r, keys in enumerate(keyed):
+        if len(keys) <= 1:
+            first.append(-1)
+            continue
+        # partial slot of a segment = first slot of its request + its key-order rank (in units of width)
+        w = 1 if width is None else width(r)
+        first.append(slot)
+        rank[r] = {k0: slot + w * i for i, k0 in enumerate(sorted(keys))}
+        slot += len(keys) * w
     out, ranges = [], [0]
     for run in per_run:
         for r, k0, k1 in run:
-            out += record(r, k0, k1, first[r] + rank[r][k0] if first[r] >= 0 else -1)
+            out += record(r, k0, k1, rank[r][k0] if first[r] >= 0 else -1)
         ranges.append(ranges[-1] + len(run))
     for r, k0, k1 in loose:
-        out += record(r, k0, k1, first[r] + rank[r][k0] if first[r] >= 0 else -1)
+        out += record(r, k0, k1, rank[r][k0] if first[r] >= 0 else -1)
     out += ranges
     for r in range(n):
-        out += request(r, max(first[r], 0), count[r])
+        out += request(r, max(first[r], 0), len(keyed[r]))
     return out, ranges[-1] + len(loose), len(per_run)
 
 
@@ -256,40 +269,46 @@ def varlen_work(query_lengths, key_lengths, starts, groups, seg_cost=None, xcd_s
     cost = SEGMENT_COST if seg_cost is None else seg_cost
     decode = [r for r, q in enumerate(query_lengths) if q <= DECODE_TOKENS]
     if len(decode) == len(key_lengths):
-        runs = _balanced_runs(key_lengths, groups, TILE, cost, shares=run_shares(groups, xcd_speed, n_cu))
-        return _segment_list(query_lengths, key_lengths, starts, runs)
-    loose = prompt_segments(query_lengths, key_lengths, groups, n_cu)
-    # each cut of a prompt takes a run's cut from the others, so the segments
-    # stay within varlen_list_bound
-    cuts = len(loose) - (len(key_lengths) - len(decode))
-    runs = [[] for _ in range(groups)]
-    if decode:
-        n = groups - cuts
-        runs[:n] = [[(decode[r], k0, k1) for r, k0, k1 in run]
-                    for run in _balanced_runs([key_lengths[r] for r in decode], n, TILE, cost,
-                                              shares=run_shares(n, xcd_speed, n_cu))]
+        runs, loose = _balanced_runs(key_lengths, groups, TILE, cost, shares=run_shares(groups, xcd_speed, n_cu)), ()
+    else:
+        # each cut of a prompt takes a run's cut from the others, so the segments
+        # stay within varlen_list_bound; the others keep at least half of the runs
+        loose = prompt_segments(query_lengths, key_lengths, (groups - 1) // 2 if decode else groups - 1, n_cu)
+        n = groups - (len(loose) - (len(key_lengths) - len(decode)))
+        runs = _decode_runs(decode, key_lengths, n, cost, xcd_speed, n_cu) + [[] for _ in range(groups - n)]
     return _segment_list(query_lengths, key_lengths, starts, runs, loose)
 
 
-def prompt_segments(query_lengths, key_lengths, groups, n_cu=None):
+def _decode_runs(decode, key_lengths, groups, cost, xcd_speed, n_cu):
+    """Balanced runs of the requests `decode` of a batch."""
+    if not decode:
+        return [[] for _ in range(groups)]
+    return [[(decode[r], k0, k1) for r, k0, k1 in run]
+            for run in _balanced_runs([key_lengths[r] for r in decode], groups, TILE, cost,
+                                      shares=run_shares(groups, xcd_speed, n_cu))]
+
+
+def prompt_segments(query_lengths, key_lengths, cuts, n_cu=None, pool=None):
     """[(request, k0, k1)] of the requests with more than DECODE_TOKENS query
     tokens, longest last: one segment each, so that nothing is merged, unless
     their (32-token tile, KV head) workgroups leave CUs idle over long keys (a
-    later chunk of a prompt): then the request with the longest segments is cut
+    later chunk of a prompt).  Then the request with the longest segments is cut
     once more, into equal parts of whole ring stages, while every part keeps
-    MIN_PROMPT_SEGMENT keys, the workgroups fit two per CU and fewer than
-    `groups` cuts are made.  A cut costs an FP32 partial write and read per
-    tile (528 bytes a row, what ~260 keys' K and V cost) and a merge."""
+    MIN_PROMPT_SEGMENT keys, the workgroups fit two per CU, at most `cuts` cuts
+    are made and the cut requests' segments fit `pool` partial tiles of 8 tokens."""
     prompts = [r for r, q in enumerate(query_lengths) if q > DECODE_TOKENS]
     tiles = {r: -(-int(query_lengths[r]) // PROMPT_TOKENS) for r in prompts}
     parts = dict.fromkeys(prompts, 1)
-    slots = RESIDENT_PER_CU * int(n_cu or 256) // 8
-    used, cuts = sum(tiles.values()), 0
-    while cuts < groups - 1:
+    per_head = int(n_cu or 256) // 8             # CUs per KV head
+    used = sum(tiles.values())
+    while prompts and cuts > 0:
         r = max(prompts, key=lambda x: key_lengths[x] / parts[x])
-        if used + tiles[r] > slots or key_lengths[r] < MIN_PROMPT_SEGMENT * (parts[r] + 1):
+        need = -(-int(query_lengths[r]) // DECODE_TOKENS) * (2 if parts[r] == 1 else 1)
+        used += tiles[r]
+        if (used > RESIDENT_PER_CU * per_head or pool is not None and need > pool
+                or key_lengths[r] < MIN_PROMPT_SEGMENT * (parts[r] + 1)):
             break
-        parts[r], used, cuts = parts[r] + 1, used + tiles[r], cuts + 1
+        parts[r], pool, cuts = parts[r] + 1, None if pool is None else pool - need, cuts - 1
     out = []
     for r in sorted(prompts, key=lambda x: key_lengths[x]):
         kl = int(key_lengths[r])
@@ -362,6 +381,114 @@ def segment_plan(split, query_lengths, key_lengths, starts, groups, chunk, capac
     ranges = out[base:base + runs + 1]
     padded = out[:base] + [0] * (WORK_INTS * (seg_cap - n_seg)) + ranges + [ranges[-1]] * (run_cap - runs)
     return padded + out[base + runs + 1:], seg_cap, run_cap
+
+
+def mixed_ints(c):
+    """int32 length of a mixed list of capacity c."""
+    return WORK_INTS * (c.run_records + c.prompt_records) + c.runs + 1 + REQ_INTS * c.requests + 2 * c.columns
+
+
+@functools.lru_cache(maxsize=1024)
+def mixed_capacity(n_req, query_tokens, key_capacity, max_q, n_cu, limit=None, short=True):
+    """The regions of a fixed-capacity mixed list (MixedCapacity) for n_req
+    requests of query_tokens query tokens in all, at most max_q > DECODE_TOKENS
+    each (short: some may have up to DECODE_TOKENS), and key_capacity keys in
+    all; limit: the workspace's partial tiles.  List and partials take no more
+    bytes than one balanced list of the whole batch would (a record per
+    request and run, each of the longest request's tiles): a bucket's workspace
+    then fits the memory budget it always did."""
+    slots = max(XCDS, RESIDENT_PER_CU * n_cu // 8 // XCDS * XCDS)
+    units = n_req if short else 0
+    runs = run_count(key_capacity, n_cu) if short else XCDS
+    longest = -(-max_q // DECODE_TOKENS)
+    one_list = run_count(key_capacity, n_cu, longest)
+    records = n_req + one_list - 1
+    # what plans use at most: a tile per segment of the runs, and four per 32-token
+    # workgroup of the prompts, which are cut only while all fit the CUs at once
+    tiles = units + runs - 1 + PROMPT_TOKENS // DECODE_TOKENS * slots
+    c = MixedCapacity(units + runs - 1, n_req + slots - 1, runs, n_req,
+                      max(slots, query_tokens // PROMPT_TOKENS + n_req), 0)
+    grown = 4 * (mixed_ints(c) - (WORK_INTS * records + one_list + 1 + REQ_INTS * n_req))
+    tiles = min(tiles, records * longest - -(-grown // PART_TILE_BYTES))
+    return c._replace(tiles=tiles if limit is None else min(tiles, limit))
+
+
+def mixed_plan(query_lengths, key_lengths, starts, n_cu, *, causal=True, capacity=None, xcd_speed=None,
+               slot_balance=True):
+    """Balanced plan of a batch that holds prompts (requests of more than
+    DECODE_TOKENS query tokens), as dspark_mixed_attn_fwd takes it: MixedPlan(list,
+    records, runs, request records, prompt columns, partial tiles).  The
+    requests of up to DECODE_TOKENS are cut into runs by their own keys, as without
+    prompts, and the prompts by prompt_segments.  capacity (mixed_capacity's) lays the list out in regions
+    of fixed size, with counts that every transaction shares."""
+    units, prompts, q0 = [], [], 0                # (request, first query row, query length, key length, start)
+    for r, (q, k) in enumerate(zip(query_lengths, key_lengths)):
+        (prompts if q > DECODE_TOKENS else units).append((r, q0, q, k, starts[r]))
+        q0 += q
+    per_head = max(XCDS, n_cu // 8 // XCDS * XCDS)                # CUs per KV head
+    cuts, pool = RESIDENT_PER_CU * n_cu, None
+    if capacity is not None:
+        cuts, pool = capacity.prompt_records - len(prompts), capacity.tiles
+        if prompts and units:                     # half each, and enough for 8 runs
+            pool = max(pool // 2, min(len(units) + XCDS - 1, 2 * (XCDS - 1)))
+    keys = [u[3] for u in units]
+    if not units:
+        per_run = [[] for _ in range(XCDS)]
+    else:
+        # At most one workgroup per CU: the other slot is the prompts'.  63 requests of
+        # 7 tokens (157,000 keys) beside 64 tokens over 8,000 keys, 16 / 24 / 32 / 48
+        # / 64 runs: 168, 138, 131, 139, 136 us; beside 4 prompts of 1,500
+        # 184, 157, 169, 172, 181; alone 159, 123, 116, 127, 118.
+        groups = min(run_count(sum(keys), n_cu), per_head)
+        while pool is not None and groups > XCDS and min(len(units) + groups - 1, 2 * (groups - 1)) > pool:
+            groups -= XCDS
+        per_run = _balanced_runs(keys, groups, TILE, SEGMENT_COST,
+                                 shares=run_shares(groups, xcd_speed, n_cu if slot_balance else None))
+    spare = None
+    if capacity is not None:
+        held = {}
+        for run in per_run:
+            for u, _, _ in run:
+                held[u] = held.get(u, 0) + 1
+        spare = capacity.tiles - sum(c for c in held.values() if c > 1)
+        if spare < 0:
+            raise ValueError('Segment plan exceeds its fixed capacity')
+    loose = prompt_segments([u[2] for u in prompts], [u[3] for u in prompts], cuts, n_cu, spare)
+    n, every = len(units), units + prompts
+    out, n_seg, groups = _flatten(len(every), per_run,
+                                  lambda u, k0, k1, slot: (every[u][0], k0, k1, slot, *every[u][1:]),
+                                  lambda u, first, count: (first, count, *every[u][1:3]),
+                                  [(n + p, k0, k1) for p, k0, k1 in loose], lambda u: -(-every[u][2] // DECODE_TOKENS))
+    first = n_seg - len(loose)
+    columns = _prompt_columns(prompts, loose, first if capacity is None else capacity.run_records, causal)
+    if capacity is None:
+        counts = out[-REQ_INTS * len(every) + 1::REQ_INTS]
+        tiles = sum(c * -(-u[2] // DECODE_TOKENS) for c, u in zip(counts, every) if c > 1)
+        return MixedPlan(out + columns, n_seg, groups, len(every), len(columns) // 2, tiles)
+    c = capacity
+    if (first > c.run_records or len(loose) > c.prompt_records or groups > c.runs or len(every) > c.requests
+            or len(columns) > 2 * c.columns):
+        raise ValueError('Segment plan exceeds its fixed capacity')
+    cut, ranges, n_work = WORK_INTS * first, WORK_INTS * n_seg, c.run_records + c.prompt_records
+    padded = np.zeros(mixed_ints(c), dtype=np.int32)
+    requests = WORK_INTS * n_work + c.runs + 1
+    for at, part in ((0, out[:cut]), (WORK_INTS * c.run_records, out[cut:ranges]),
+                     (WORK_INTS * n_work, out[ranges:ranges + groups + 1] + [first] * (c.runs - groups)),
+                     (requests, out[ranges + groups + 1:]), (requests + REQ_INTS * c.requests, columns)):
+        padded[at:at + len(part)] = part
+    return MixedPlan(padded, n_work, c.runs, c.requests, c.columns, c.tiles)
+
+
+def _prompt_columns(prompts, loose, first, causal):
+    """(1 + record, tile) of every 32-token tile of the prompts' segments, the
+    records counted from `first`, most keys first."""
+    out = []
+    for i, (p, k0, k1) in enumerate(loose, 1 + first):
+        _, _, q, k, _ = prompts[p]
+        seen = k - q + PROMPT_TOKENS if causal else k            # keys up to the first tile's last token
+        out += [(k0 - min(k1, seen + PROMPT_TOKENS * t), i, t) for t in range(-(-q // PROMPT_TOKENS))]
+    out.sort()
+    return [x for column in out for x in column[1:]]
 
 
 def draft_work(context_lengths, cu_blocks, anchors, groups=None, *, chunk=None, offsets=None):

@@ -1,0 +1,96 @@
+"""dspark_mixed_attn_fwd: batches of prompts, chunks of prompts and decoding
+requests at the sizes where a plan changes form (prompts alone and beside decoding requests,
+cut and uncut; nothing to merge), packed and from the store, staged by the launch or
+before it, against the CPU oracle at the attention tolerance."""
+import pytest
+import torch
+
+from helpers import SCALE, SEED, attention_gate, bits, f64, randn_bf16, segments
+from oracle import cref
+from test_gpu_prefill import layout_of
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device('cuda:0')
+
+BATCHES = [([9], [0]), ([9], [700]), ([16, 64], [0, 300]), ([96], [300]), ([97], [300]), ([12, 33, 9], [1500, 0, 40]),
+           ([7, 7, 9], [600, 30, 1900]), ([8, 1, 64, 200], [500, 0, 1200, 0]), ([17], [3000]), ([40, 7], [2500, 900]),
+           ([64, 7, 7, 300], [1800, 700, 9, 1900]), ([20] * 20, [30] * 20)]
+
+
+@pytest.mark.parametrize('ql,ctx', BATCHES)
+def test_packed(ql, ctx):
+    from qwen3_dspark_amd.kernels import HipDraftVarlenKernel, HipVarlenKernel
+    print(f'[mixed] packed q={ql} ctx={ctx}', flush=True)
+    layout, q, k, v = layout_of(ql, [c + n for c, n in zip(ctx, ql)])
+    cu_q = layout.cu_query.tolist()
+    for cls in (HipVarlenKernel, HipDraftVarlenKernel):
+        out = cls(DEV)(q.to(DEV), k.to(DEV), v.to(DEV), layout, scale=SCALE)
+        ref = cref.varlen_attention(bits(q), bits(k), bits(v), cu_q, layout.cu_key.tolist(), causal=cls.causal,
+                                    scale=SCALE)
+        attention_gate(f64(out), ref, segments(cu_q))
+
+
+@pytest.mark.parametrize('ql,ctx', BATCHES)
+def test_store(ql, ctx):
+    """Through a bucket and through a family that also takes other lengths;
+    rows past a context and other slots hold NaN."""
+    from qwen3_dspark_amd.persistent_kv import Bucket, PersistentTargetKV, QueryFamily
+    print(f'[mixed] store q={ql} ctx={ctx}', flush=True)
+    gen = torch.Generator().manual_seed(SEED + sum(ql) + sum(ctx))
+    n, rows = len(ql), sum(ql)
+    store = PersistentTargetKV(layers=1, slots=n + 1, context_capacity=3400, max_query_tokens=rows, heads=8, dim=128,
+                               device=DEV)
+    store.keys.fill_(float('nan'))
+    store.values.fill_(float('nan'))
+    handles = [store.add_request(f'r{i}') for i in range(n)][::-1]
+    for h, c in zip(handles, ctx):
+        if c:
+            kv = randn_bf16(gen, 2, 1, c, 8, 128).to(DEV)
+            store.load_prefix(h, kv[0], kv[1])
+    bucket = Bucket(tuple(ql), tuple(c + 100 for c in ctx), 'mixed')
+    family = QueryFamily(n, rows, max(ql) + 20, rows + sum(ctx) + 500, 3400, 'mixed family')
+    store.register_bucket(bucket)
+    store.register_families((family,))
+    q, nk, nv = (randn_bf16(gen, rows, h, 128).to(DEV) for h in (16, 8, 8))
+    cu_q = [sum(ql[:i]) for i in range(n + 1)]
+    ref = cref.verify_attention(bits(q), bits(store.keys[0]), bits(store.values[0]), bits(nk), bits(nv),
+                                [h.index for h in handles], ctx, cu_q, scale=SCALE)
+    for shape in (bucket, family):
+        tx = store.begin(handles, shape, query_lengths=tuple(ql))
+        store.scratch_keys.zero_()
+        out = store.attend(tx, 0, q, keys=nk, values=nv)
+        assert torch.equal(store.scratch_keys[0], nk) and torch.equal(store.scratch_values[0], nv)
+        attention_gate(f64(out), ref, segments(cu_q))
+        store.abort(tx)
+        tx = store.begin(handles, shape, query_lengths=tuple(ql))
+        store.stage_layer(tx, 0, nk, nv)
+        assert torch.equal(store.attend(tx, 0, q), out)
+        store.abort(tx)
+
+
+def test_families_of_one_arena():
+    """A decoding family and one with prompts share a workspace: the lists and
+    partials of both fit, whatever the transaction holds."""
+    from qwen3_dspark_amd.persistent_kv import PersistentTargetKV, QueryFamily
+    gen = torch.Generator().manual_seed(SEED)
+    store = PersistentTargetKV(layers=1, slots=4, context_capacity=3000, max_query_tokens=400, heads=8, dim=128,
+                               device=DEV)
+    handles = [store.add_request(f'r{i}') for i in range(4)]
+    ctx = [2500, 40, 1800, 700]
+    for h, c in zip(handles, ctx):
+        kv = randn_bf16(gen, 2, 1, c, 8, 128).to(DEV)
+        store.load_prefix(h, kv[0], kv[1])
+    small = QueryFamily(4, 20, 8, 6000, 3000, 'decoding')
+    large = QueryFamily(4, 220, 200, 6000, 3000, 'with prompts')
+    store.register_families((small, large))
+    for family, ql in ((small, (7, 1, 8, 4)), (large, (7, 200, 9, 4)), (large, (55, 55, 55, 55)), (small, (5,) * 4),
+                       (large, (1, 1, 18, 200))):
+        rows = sum(ql)
+        q, nk, nv = (randn_bf16(gen, rows, h, 128).to(DEV) for h in (16, 8, 8))
+        tx = store.begin(handles, family, query_lengths=ql)
+        out = store.attend(tx, 0, q, keys=nk, values=nv)
+        cu_q = [sum(ql[:i]) for i in range(5)]
+        ref = cref.verify_attention(bits(q), bits(store.keys[0]), bits(store.values[0]), bits(nk), bits(nv),
+                                    [h.index for h in handles], ctx, cu_q, scale=SCALE)
+        attention_gate(f64(out), ref, segments(cu_q))
+        store.abort(tx)
