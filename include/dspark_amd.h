@@ -194,6 +194,11 @@ int dspark_verify_attn_staged_fwd(const void* q, const void* k_res, const void* 
  *     KV head attends query tokens 32 tile .. 32 tile + 31 of that record's
  *     request (more than 8 tokens) over the record's keys, started in the
  *     order of the list ((0, 0): none).  The runs hold the records of the rest;
+ *   - a request of more than 8 query tokens either there or, as its tiles of 8
+ *     tokens, in the runs: tile t has records and a request record of its own, with
+ *     t in bits 24-30 of the records' first word, the tile's first query row and
+ *     query count, and (causal) the key length that ends with its last token;
+ *   - n_req request records, the tiles counted;
  *   - partial slots counted in tiles of 8 query tokens: a segment takes
  *     ceil(query count / 8) from its slot on, the segments of a split request one
  *     after the other.  part_tiles of them are reserved; 0: every request record

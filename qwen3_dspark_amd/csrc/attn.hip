@@ -277,6 +277,7 @@ struct VarlenArgs {
   float* part_ml;         // [partial tiles][16][2]
   int n_req;
   int n_work;             // segment records in the work list
+  int tile_shift;         // a record's first word from this bit on: its tile of 8 query tokens
   int n_slots;            // no list: (chunk, KV head) slots, 8 * chunks
   int causal;
   int chunk;
@@ -336,7 +337,7 @@ struct SegView {
   const bf16* vA;
   const bf16* kB;
   const bf16* vB;
-  size_t bbase;   // part B offset of the request's first new row, KV head g
+  size_t bbase;   // part B offset of the row of the first query here, KV head g
   int a_len;
   int k0;
   int kend;       // keys [k0, kend) are visible to some row of the tile
@@ -363,13 +364,15 @@ __device__ __forceinline__ SegView seg_view(const VarlenArgs& a, const Segment& 
   v.live = v.ql > 0 && (!MIXED || v.ql <= DECODE_TOKENS);
   v.ends = k1 == v.kl && (!MIXED || v.live);
   if (VERIFY) {
-    v.a_len = v.kl - v.ql;
+    // query rows of the request before this tile (kl ends with the tile)
+    const int before = DECODE_TOKENS * (__builtin_amdgcn_readfirstlane(sg.r) >> a.tile_shift);
+    v.a_len = v.kl - v.ql - before;
     const size_t abase = (size_t)start * (size_t)a.slot_stride + (size_t)g * a.a_head_stride;
     v.kA = a.k_a + abase;
     v.vA = a.v_a + abase;
     v.bbase = (size_t)v.q0 * KV_ROW + (size_t)g * HD;
-    v.kB = a.k_b + v.bbase;
-    v.vB = a.v_b + v.bbase;
+    v.kB = a.k_b + v.bbase - (size_t)before * KV_ROW;
+    v.vB = a.v_b + v.bbase - (size_t)before * KV_ROW;
   } else {
     v.a_len = v.kl;
     const size_t abase = (size_t)start * KV_ROW + (size_t)g * HD;
@@ -2199,6 +2202,7 @@ int varlen_launch(VarlenArgs& a, int64_t key_rows_bound, int max_q, float scale,
   a.part_ml = a.part_o + n_cl * HKV * tiles * 16 * HD;
   a.chunk = chunk;
   a.tmax = tiles;
+  a.tile_shift = 31;
   a.scale_log2 = scale * LOG2E;
   a.n_slots = (int)(n_cl * HKV);
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -2344,6 +2348,7 @@ extern "C" int dspark_mixed_attn_fwd(const void* q, const void* k, const void* v
   a.n_work = n_work;
   a.causal = causal ? 1 : 0;
   a.tmax = 0;
+  a.tile_shift = 24;
   a.scale_log2 = scale * LOG2E;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int32_t* requests = work + WORK_INTS * n_work + n_groups + 1;

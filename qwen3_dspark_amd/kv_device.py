@@ -25,7 +25,7 @@ import torch
 from . import _native
 from ._device import KV_PAIR_SKEW, cu_count, kv_pair, require_gfx950, upload
 from .kernels import HEAD_DIM, KV_HEADS, SCALE
-from .schedule import (DECODE_TOKENS, PART_TILE_BYTES, REQ_INTS, WORK_INTS, mixed_capacity, mixed_ints, mixed_plan, run_count,
+from .schedule import (DECODE_TOKENS, PART_TILE_BYTES, REQ_INTS, TILED_TOKENS, WORK_INTS, mixed_capacity, mixed_ints, mixed_plan, run_count,
                        segment_plan, varlen_list_bound)
 
 MAX_BUCKET_REQUESTS = 4096      # requests per transaction (one metadata workgroup scans them in LDS)
@@ -47,7 +47,7 @@ def _mixed_shape(shape, device, split, limit=None):
         return None
     lengths = getattr(shape, 'query_lengths', None)              # a bucket's are exact, a family's bounded
     return mixed_capacity(shape.request_count, shape.query_tokens, shape.key_capacity, shape.maximum_query_length,
-                          cu_count(device), limit, lengths is None or min(lengths) <= DECODE_TOKENS)
+                          cu_count(device), limit, lengths is None or min(lengths) <= TILED_TOKENS)
 
 
 def _list_shape(shape, device, chunk, split):

@@ -60,7 +60,24 @@ SEGMENT_COST = 96             # keys' worth of fixed work per segment in balance
 SECOND_SLOT_SHARE = 0.75
 DECODE_TOKENS = 8             # requests with more query tokens take the prefill kernel (attn.hip)
 PROMPT_TOKENS = 32            # query tokens per prefill workgroup (two resident per CU)
-MIN_PROMPT_SEGMENT = 1024     # fewest keys a cut leaves a prompt segment (see prompt_segments)
+# A prompt is cut while its segments keep this many keys on CUs of their own (in
+# 1 / 2 / 4 / 8 / 16 segments, us a call: 200 tokens over 1,000 keys 26.7, 20.9, 17.5,
+# 18.7, -; 128 over 4,096 61, 38, 26, 22, 23; 64 over 8,000 111, 63, 38, 27, 23) and this many
+# where two workgroups share a CU (8 prompts of 100 tokens over 1,000 keys uncut 28,
+# in halves 32; 256 over 8,000 in 4 / 8 43, 38).
+MIN_PROMPT_SEGMENT = 256
+SHARED_PROMPT_SEGMENT = 1024
+MAX_PROMPT_SEGMENTS = 16      # more gain nothing: 16 / 24 / 32 of 64 tokens over 8,000 keys 22.8, 25.5, 25.9 us
+# Prompts of up to TILED_TOKENS are attended as tiles of DECODE_TOKENS while their tiles'
+# keys number at most TILED_KEYS per workgroup slot (two per CU): the prompt form
+# waits for one 64-key stage after the other (~1 us each), which few tokens on an
+# idle machine do not hide, while tiles read the keys once per 8 tokens.  Prompt
+# form / tiles, us: 9 tokens over 700 keys 14.2 / 9.0, over 8,000 22.6 / 21.2; 64 over 300 14.0
+# / 10.4, over 2,000 17.4 / 13.7, over 4,096 18.4 / 19; 96 over 700 16.4 / 11.9; 8 prompts of
+# 64 tokens over 300 14.6 / 9.9, over 1,000 23.5 / 28.
+TILED_TOKENS = 96
+TILED_KEYS = 384
+MAX_TILES = 64                # tiles that they add to a batch at most
 DRAFT_TILE = 64               # draft cuts fall on multiples of the ring stage
 DRAFT_SEGMENT_COST = 512      # balanced draft plans: fixed cost of a segment, in context rows (measured)
 DRAFT_BLOCK_WEIGHT = 0.055    # balanced draft plans: extra cost of a row per block beyond the first (measured)
@@ -305,8 +322,9 @@ def prompt_segments(query_lengths, key_lengths, cuts, n_cu=None, pool=None):
         r = max(prompts, key=lambda x: key_lengths[x] / parts[x])
         need = -(-int(query_lengths[r]) // DECODE_TOKENS) * (2 if parts[r] == 1 else 1)
         used += tiles[r]
-        if (used > RESIDENT_PER_CU * per_head or pool is not None and need > pool
-                or key_lengths[r] < MIN_PROMPT_SEGMENT * (parts[r] + 1)):
+        least = MIN_PROMPT_SEGMENT if used <= per_head else SHARED_PROMPT_SEGMENT
+        if (parts[r] == MAX_PROMPT_SEGMENTS or used > RESIDENT_PER_CU * per_head or pool is not None and need > pool
+                or key_lengths[r] < least * (parts[r] + 1)):
             break
         parts[r], pool, cuts = parts[r] + 1, None if pool is None else pool - need, cuts - 1
     out = []
@@ -383,6 +401,11 @@ def segment_plan(split, query_lengths, key_lengths, starts, groups, chunk, capac
     return padded + out[base + runs + 1:], seg_cap, run_cap
 
 
+def _tile_count(n_req):
+    """Most row tiles that mixed plans add to a batch's requests."""
+    return min(n_req * (TILED_TOKENS // DECODE_TOKENS - 1), MAX_TILES)      # MAX_TILES from 6 requests on
+
+
 def mixed_ints(c):
     """int32 length of a mixed list of capacity c."""
     return WORK_INTS * (c.run_records + c.prompt_records) + c.runs + 1 + REQ_INTS * c.requests + 2 * c.columns
@@ -392,25 +415,59 @@ def mixed_ints(c):
 def mixed_capacity(n_req, query_tokens, key_capacity, max_q, n_cu, limit=None, short=True):
     """The regions of a fixed-capacity mixed list (MixedCapacity) for n_req
     requests of query_tokens query tokens in all, at most max_q > DECODE_TOKENS
-    each (short: some may have up to DECODE_TOKENS), and key_capacity keys in
+    each (short: some may have up to TILED_TOKENS), and key_capacity keys in
     all; limit: the workspace's partial tiles.  List and partials take no more
     bytes than one balanced list of the whole batch would (a record per
     request and run, each of the longest request's tiles): a bucket's workspace
     then fits the memory budget it always did."""
     slots = max(XCDS, RESIDENT_PER_CU * n_cu // 8 // XCDS * XCDS)
-    units = n_req if short else 0
-    runs = run_count(key_capacity, n_cu) if short else XCDS
+    units = n_req + _tile_count(n_req) if short else 0
+    runs = slots if short else XCDS
     longest = -(-max_q // DECODE_TOKENS)
     one_list = run_count(key_capacity, n_cu, longest)
     records = n_req + one_list - 1
     # what plans use at most: a tile per segment of the runs, and four per 32-token
     # workgroup of the prompts, which are cut only while all fit the CUs at once
     tiles = units + runs - 1 + PROMPT_TOKENS // DECODE_TOKENS * slots
-    c = MixedCapacity(units + runs - 1, n_req + slots - 1, runs, n_req,
+    c = MixedCapacity(units + runs - 1, n_req + slots - 1, runs, max(units, n_req),
                       max(slots, query_tokens // PROMPT_TOKENS + n_req), 0)
     grown = 4 * (mixed_ints(c) - (WORK_INTS * records + one_list + 1 + REQ_INTS * n_req))
     tiles = min(tiles, records * longest - -(-grown // PART_TILE_BYTES))
     return c._replace(tiles=tiles if limit is None else min(tiles, limit))
+
+
+def _tiled_requests(query_lengths, key_lengths, n_cu):
+    """Prompts attended as tiles of DECODE_TOKENS in the runs: those of up to
+    TILED_TOKENS, if all of their tiles' keys leave each workgroup slot few."""
+    some = [r for r, q in enumerate(query_lengths) if DECODE_TOKENS < q <= TILED_TOKENS]
+    tiles = [-(-query_lengths[r] // DECODE_TOKENS) for r in some]
+    fits = (sum(tiles) - len(some) <= MAX_TILES
+            and sum(t * key_lengths[r] for t, r in zip(tiles, some)) <= TILED_KEYS * RESIDENT_PER_CU * n_cu // 8)
+    return some if fits else ()
+
+
+def _tile_runs(units, columns):
+    """Runs of row tiles alone (units as in _mixed_plan): a request's tiles are cut
+    at the same keys into equal parts, 8 for every 8 MIN_SEGMENT keys while a part
+    keeps two TILE, at most `columns` segments in all, a run each (a balanced cut would
+    give most runs the end of one tile and the start of another, two segments'
+    fixed work).  The tiles of a part are neighbours on one XCD, whose L2 they
+    share."""
+    share = max(1, columns // len(units))
+    share = share // XCDS * XCDS or share
+    tiles, segs = {}, []
+    for u, unit in enumerate(units):
+        tiles.setdefault(unit[0] & 0xffffff, []).append((u, unit[3]))
+    for group in tiles.values():
+        longest = max(k for _, k in group)
+        parts = min(share, -(-longest // (XCDS * MIN_SEGMENT)) * XCDS, -(-longest // (2 * TILE)))
+        at = [i * longest // parts // TILE * TILE for i in range(parts)] + [longest]
+        for lo, hi in zip(at, at[1:]):
+            segs += [(u, lo, min(hi, k)) for u, k in group if k > lo]
+    depth = -(-len(segs) // XCDS)
+    queues = [segs[x * depth:(x + 1) * depth] for x in range(XCDS)]
+    rounds = min(columns // XCDS, depth)
+    return [queues[x][j::rounds] for j in range(rounds) for x in range(XCDS)]
 
 
 def mixed_plan(query_lengths, key_lengths, starts, n_cu, *, causal=True, capacity=None, xcd_speed=None,
@@ -419,11 +476,31 @@ def mixed_plan(query_lengths, key_lengths, starts, n_cu, *, causal=True, capacit
     DECODE_TOKENS query tokens), as dspark_mixed_attn_fwd takes it: MixedPlan(list,
     records, runs, request records, prompt columns, partial tiles).  The
     requests of up to DECODE_TOKENS are cut into runs by their own keys, as without
-    prompts, and the prompts by prompt_segments.  capacity (mixed_capacity's) lays the list out in regions
+    prompts, with the tiles of _tiled_requests among them; other prompts are cut by
+    prompt_segments.  capacity (mixed_capacity's) lays the list out in regions
     of fixed size, with counts that every transaction shares."""
-    units, prompts, q0 = [], [], 0                # (request, first query row, query length, key length, start)
+    batch = (query_lengths, key_lengths, starts, n_cu, causal, capacity, xcd_speed, slot_balance)
+    tiled = _tiled_requests(query_lengths, key_lengths, n_cu)
+    plan = _mixed_plan(tiled, *batch)
+    if plan is None and tiled:           # the capacity has too few partial tiles for row tiles
+        plan = _mixed_plan((), *batch)
+    if plan is None:
+        raise ValueError('Segment plan exceeds its fixed capacity')
+    return plan
+
+
+def _mixed_plan(tiled, query_lengths, key_lengths, starts, n_cu, causal, capacity, xcd_speed, slot_balance):
+    units, prompts, q0 = [], [], 0                # (first word, first query row, query length, key length, start)
     for r, (q, k) in enumerate(zip(query_lengths, key_lengths)):
-        (prompts if q > DECODE_TOKENS else units).append((r, q0, q, k, starts[r]))
+        if q > DECODE_TOKENS and r not in tiled:
+            prompts.append((r, q0, q, k, starts[r]))
+        elif q <= DECODE_TOKENS:
+            units.append((r, q0, q, k, starts[r]))
+        else:
+            for t in range(-(-q // DECODE_TOKENS)):
+                row = DECODE_TOKENS * t
+                n = min(DECODE_TOKENS, q - row)
+                units.append((r | t << 24, q0 + row, n, k - q + row + n if causal else k, starts[r]))
         q0 += q
     per_head = max(XCDS, n_cu // 8 // XCDS * XCDS)                # CUs per KV head
     cuts, pool = RESIDENT_PER_CU * n_cu, None
@@ -434,6 +511,9 @@ def mixed_plan(query_lengths, key_lengths, starts, n_cu, *, causal=True, capacit
     keys = [u[3] for u in units]
     if not units:
         per_run = [[] for _ in range(XCDS)]
+    elif len(units) == sum(-(-query_lengths[r] // DECODE_TOKENS) for r in tiled):
+        columns = per_head if prompts else RESIDENT_PER_CU * per_head
+        per_run = _tile_runs(units, columns if pool is None else min(columns, max(XCDS, pool // XCDS * XCDS)))
     else:
         # At most one workgroup per CU: the other slot is the prompts'.  63 requests of
         # 7 tokens (157,000 keys) beside 64 tokens over 8,000 keys, 16 / 24 / 32 / 48
@@ -452,7 +532,7 @@ def mixed_plan(query_lengths, key_lengths, starts, n_cu, *, causal=True, capacit
                 held[u] = held.get(u, 0) + 1
         spare = capacity.tiles - sum(c for c in held.values() if c > 1)
         if spare < 0:
-            raise ValueError('Segment plan exceeds its fixed capacity')
+            return None
     loose = prompt_segments([u[2] for u in prompts], [u[3] for u in prompts], cuts, n_cu, spare)
     n, every = len(units), units + prompts
     out, n_seg, groups = _flatten(len(every), per_run,
@@ -468,7 +548,7 @@ def mixed_plan(query_lengths, key_lengths, starts, n_cu, *, causal=True, capacit
     c = capacity
     if (first > c.run_records or len(loose) > c.prompt_records or groups > c.runs or len(every) > c.requests
             or len(columns) > 2 * c.columns):
-        raise ValueError('Segment plan exceeds its fixed capacity')
+        return None
     cut, ranges, n_work = WORK_INTS * first, WORK_INTS * n_seg, c.run_records + c.prompt_records
     padded = np.zeros(mixed_ints(c), dtype=np.int32)
     requests = WORK_INTS * n_work + c.runs + 1

@@ -1,6 +1,7 @@
 """dspark_mixed_attn_fwd: batches of prompts, chunks of prompts and decoding
-requests at the sizes where a plan changes form (prompts alone and beside decoding requests,
-cut and uncut; nothing to merge), packed and from the store, staged by the launch or
+requests at the sizes where a plan changes form (row tiles in the runs, alone
+and among decoding requests; prompts cut and uncut; partials of tiles and of
+prompts; nothing to merge), packed and from the store, staged by the launch or
 before it, against the CPU oracle at the attention tolerance."""
 import pytest
 import torch

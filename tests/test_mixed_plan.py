@@ -3,7 +3,8 @@ these lists, so every row tile's keys are covered exactly once, the merge
 records name the slots that the segments write, and the fixed-capacity form
 always fits its regions, which take no more memory than one balanced list of
 the batch.  And what such a plan must not lose: a prompt leaves the decoding
-requests their workgroups."""
+requests their workgroups, and a few query tokens over a long context are
+spread over the CUs."""
 import numpy as np
 import pytest
 
@@ -117,7 +118,7 @@ def test_random_buckets_fit():
         kl = [q + int(np.exp(rng.uniform(0, np.log(9000)))) - 1 for q in ql]
         bound = sum(kl) + int(rng.integers(0, 5000))
         cap = mixed_capacity(n, sum(ql), bound, max_q, N_CU)
-        if min(ql) > DECODE_TOKENS:
+        if min(ql) > 96:
             exact = mixed_capacity(n, sum(ql), bound, max_q, N_CU, None, False)
             check(ql, kl, list(range(n)), mixed_plan(ql, kl, list(range(n)), N_CU, capacity=exact))
         assert capacity_bytes(cap) <= one_list_bytes(n, bound, max_q)
@@ -136,3 +137,14 @@ def test_a_chunk_leaves_the_decoding_requests_their_workgroups(tokens, fixed):
     cap = mixed_capacity(64, sum(ql), sum(kl), tokens, N_CU) if fixed else None
     busy, _ = check(ql, kl, list(range(64)), mixed_plan(ql, kl, list(range(64)), N_CU, capacity=cap))
     assert busy * 8 >= N_CU
+
+
+@pytest.mark.parametrize('tokens', [9, 16, 32, 64])
+@pytest.mark.parametrize('keys', [2000, 4096, 8000])
+def test_a_short_chunk_over_a_long_context_is_spread(tokens, keys):
+    """At least 14 workgroups per KV head: as 8-token requests over the same keys
+    have (8 to 32), where one list gave a chunk 1 to 7."""
+    ql, kl = [tokens], [keys + tokens]
+    for cap in (None, mixed_capacity(1, tokens, kl[0], tokens, N_CU)):
+        busy, prompts = check(ql, kl, [0], mixed_plan(ql, kl, [0], N_CU, capacity=cap))
+        assert (busy if not prompts else sum(prompts.values())) >= min(14, -(-keys // 256))
