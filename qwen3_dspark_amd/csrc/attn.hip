@@ -1271,15 +1271,15 @@ __device__ __forceinline__ void draft_pair_item(const DraftArgs& a, unsigned cha
   // Only stages that hold context are loaded, so the number of ring loads
   // still in flight behind a given one is known: all but the newest
   // `behind` stages of LPS loads each (PER_WAVE pieces, and with indices
-  // one index load) have landed after wait_stages.
+  // one index load) have landed after stage_barrier, for every wave.
   constexpr int LPS = R::PER_WAVE + (INDEXED ? 1 : 0);
-  auto wait_stages = [](int behind) {
-    if (behind <= 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    else if (behind == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPS) : "memory");
-    else if (behind == 2 || R::STAGES < 4) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LPS) : "memory");
-    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * LPS) : "memory");
+  auto stage_barrier = [](int behind) {
+    if (behind <= 0) ring_barrier<0>();
+    else if (behind == 1) ring_barrier<LPS>();
+    else if (behind == 2 || R::STAGES < 4) ring_barrier<2 * LPS>();
+    else ring_barrier<3 * LPS>();
   };
-  static_assert(R::STAGES <= 4, "wait_stages covers at most three stages in flight");
+  static_assert(R::STAGES <= 4, "stage_barrier covers at most three stages in flight");
   static_assert(R::STAGES == 3 || !INDEXED, "the index prologue loads two stages");
   const int prologue = min(R::STAGES - 1, n_steps);
   if constexpr (INDEXED) {
@@ -1297,8 +1297,7 @@ __device__ __forceinline__ void draft_pair_item(const DraftArgs& a, unsigned cha
     if (p < prologue) issue(p);
   TL_MARK(1);
   if (last) {
-    wait_stages(prologue);   // the Q and own rows, issued first, have landed
-    asm volatile("s_barrier" ::: "memory");
+    stage_barrier(prologue);   // the Q and own rows, issued first, have landed
     TL_MARK(2);
     if (q_lds) read_q();
     if (active && kh == 0) {
@@ -1329,8 +1328,7 @@ __device__ __forceinline__ void draft_pair_item(const DraftArgs& a, unsigned cha
     // the top of step s the stages issued after stage s number
     // min(n_steps - 1 - s, STAGES - 2).
     auto step = [&](int s) {
-      wait_stages(min(n_steps - 1 - s, R::STAGES - 2));
-      asm volatile("s_barrier" ::: "memory");
+      stage_barrier(min(n_steps - 1 - s, R::STAGES - 2));
 #ifdef DSPARK_TIMELINE
       if (s == 0 && !last) TL_MARK(2);
 #endif
@@ -1344,7 +1342,7 @@ __device__ __forceinline__ void draft_pair_item(const DraftArgs& a, unsigned cha
   // overlaps the merge below (a draw inside the stream loop, right after the
   // ring's last stage load, made the compiler spill the loop's registers).
   draw();
-  asm volatile("s_barrier" ::: "memory");   // every wave is done with the ring and the own rows
+  lds_barrier();   // every wave is done with the ring and the own rows
   TL_MARK(3);
 
   // The key halves merge: the kh = 1 wave of each pair leaves its state in
@@ -1937,8 +1935,7 @@ __global__ __launch_bounds__(PF_WAVES * WAVE, 2) void prefill_attn_kernel(Varlen
   auto arrive = [&]() {
     // not before the MFMAs of the step that ends here, which hide the loads
     __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    asm volatile("s_barrier" ::: "memory");
+    ring_barrier<0>();
   };
   auto enter = [&](int s) {
     arrive();

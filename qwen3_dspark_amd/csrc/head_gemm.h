@@ -148,12 +148,12 @@ __device__ __forceinline__ void head_tile_gemm(const bf16* __restrict__ w, const
     if (i < steps) issue(i);
   const int R = L.token();
   for (int s = 0; s < steps; ++s) {
-    // this thread's stage-s loads landed (the STAGES - 2 stages behind it, as
-    // far as there are any, may still be in flight) ...
-    if (Ring::STAGES == 4 && s + 2 < steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * Ring::LOADS) : "memory");
-    else if (s + 1 < steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(Ring::LOADS) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    asm volatile("s_barrier" ::: "memory");            // ... and everyone else's
+    // every wave's stage-s loads landed (the STAGES - 2 stages behind it, as
+    // far as there are any, may still be in flight) and its reads of stage s - 1,
+    // which the next loads overwrite, are done
+    if (Ring::STAGES == 4 && s + 2 < steps) ring_barrier<2 * Ring::LOADS>();
+    else if (s + 1 < steps) ring_barrier<Ring::LOADS>();
+    else ring_barrier<0>();
     if (s + Ring::STAGES - 1 < steps) issue(s + Ring::STAGES - 1);
     const unsigned char* wst = smem + (s % Ring::STAGES) * Ring::STAGE_BYTES + L.kq * Ring::SUB_BYTES;
     const unsigned char* xst = wst + HG_W_BYTES;
@@ -172,7 +172,7 @@ __device__ __forceinline__ void head_tile_gemm(const bf16* __restrict__ w, const
         acc[a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wa, xb, acc[a], 0, 0, 0);
       }
     }
-    if (TG == 1) __builtin_amdgcn_sched_barrier(0);    // no barrier of the next stage above these MFMAs' reads
+    __builtin_amdgcn_sched_barrier(0);    // the next stage's wait not above these MFMAs
   }
   pre_combine();
   __syncthreads();   // every wave is done with the ring: reuse it for the exchange

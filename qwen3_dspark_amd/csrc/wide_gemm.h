@@ -89,8 +89,7 @@ __device__ __forceinline__ void wide_tile_gemm(const bf16* __restrict__ w, const
   for (int s = 0; s < steps; ++s) {
     // stage s has landed for every wave, whose LDS reads of stage s - 1 are done
     __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    asm volatile("s_barrier" ::: "memory");
+    ring_barrier<0>();
     if (s + 1 < steps) issue(s + 1);
     const unsigned char* wst = smem + (s & 1) * WG_STAGE;
     const unsigned char* xst = wst + WG_PART;
