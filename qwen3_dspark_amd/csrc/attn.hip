@@ -348,8 +348,8 @@ struct SegView {
 };
 
 // MIXED: the launch also has requests that prefill workgroups attend; their
-// segments have no live rows here.
-template <bool VERIFY, bool MIXED>
+// segments have no live rows here.  TILED: records may be row tiles of a request.
+template <bool VERIFY, bool MIXED, bool TILED>
 __device__ __forceinline__ SegView seg_view(const VarlenArgs& a, const Segment& sg, int g) {
   SegView v;
   // The segment is wave-uniform; say so, so that its fields and everything
@@ -365,7 +365,7 @@ __device__ __forceinline__ SegView seg_view(const VarlenArgs& a, const Segment& 
   v.ends = k1 == v.kl && (!MIXED || v.live);
   if (VERIFY) {
     // query rows of the request before this tile (kl ends with the tile)
-    const int before = DECODE_TOKENS * (__builtin_amdgcn_readfirstlane(sg.r) >> a.tile_shift);
+    const int before = TILED ? DECODE_TOKENS * (__builtin_amdgcn_readfirstlane(sg.r) >> a.tile_shift) : 0;
     v.a_len = v.kl - v.ql - before;
     const size_t abase = (size_t)start * (size_t)a.slot_stride + (size_t)g * a.a_head_stride;
     v.kA = a.k_a + abase;
@@ -459,7 +459,7 @@ __device__ __forceinline__ void load_q(const VarlenArgs& a, const SegView& s, in
 // k0 + 32w, k0 + 32(w+4), ... of each segment.
 // fetch(n, sg) yields the run's n-th segment (false past the end); every
 // branch on it is uniform across the workgroup.
-template <bool VERIFY, bool MIXED, typename Fetch>
+template <bool VERIFY, bool MIXED, bool TILED, typename Fetch>
 __device__ __forceinline__ void varlen_run(const VarlenArgs& a, unsigned char* smem, int g, Fetch fetch) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -478,7 +478,7 @@ __device__ __forceinline__ void varlen_run(const VarlenArgs& a, unsigned char* s
 
   Segment sg;
   if (!fetch(0, sg)) return;
-  SegView cur = seg_view<VERIFY, MIXED>(a, sg, g);
+  SegView cur = seg_view<VERIFY, MIXED, TILED>(a, sg, g);
   bf16x8 qf[4];
   for (int n = 0;; ++n) {
     load_q(a, cur, g, qf);
@@ -613,7 +613,7 @@ __device__ __forceinline__ void varlen_run(const VarlenArgs& a, unsigned char* s
     }
     __syncthreads();   // the next segment reuses the V tiles and the merge buffer
     if (!more) break;
-    cur = seg_view<VERIFY, MIXED>(a, nsg, g);
+    cur = seg_view<VERIFY, MIXED, TILED>(a, nsg, g);
   }
 }
 
@@ -651,7 +651,7 @@ __device__ __forceinline__ uint64_t tl_now() { return __builtin_amdgcn_s_memreal
 // Without a list, a persistent grid walks the fixed chunks (item, KV head)
 // with a stride of the grid size, so per-workgroup start-up is paid once
 // per CU slot.
-template <bool VERIFY, bool MIXED>
+template <bool VERIFY, bool MIXED, bool TILED>
 __device__ __forceinline__ void varlen_workgroup(const VarlenArgs& a, unsigned char* smem, int wid, int grid) {
   const int slot = wid >> 3;
   const int g = a.work ? (slot & 7) : (wid & 7);
@@ -664,7 +664,7 @@ __device__ __forceinline__ void varlen_workgroup(const VarlenArgs& a, unsigned c
     const uint64_t tl_start = tl_now();
     int tl_keys = 0;
 #endif
-    varlen_run<VERIFY, MIXED>(a, smem, g, [&](int n, Segment& sg) {
+    varlen_run<VERIFY, MIXED, TILED>(a, smem, g, [&](int n, Segment& sg) {
       if (b + n >= e) return false;
       const int32_t* w = a.work + WORK_INTS * (b + n);
       sg = Segment{w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7]};
@@ -688,16 +688,16 @@ __device__ __forceinline__ void varlen_workgroup(const VarlenArgs& a, unsigned c
 #endif
     return;
   }
-  varlen_run<VERIFY, MIXED>(a, smem, g, [&](int n, Segment& sg) {
+  varlen_run<VERIFY, MIXED, TILED>(a, smem, g, [&](int n, Segment& sg) {
     const int idx = wid + n * grid;
     return idx < a.n_slots && chunk_segment(a, VERIFY, idx >> 3, sg);
   });
 }
 
-template <bool VERIFY>
+template <bool VERIFY, bool TILED>
 __global__ __launch_bounds__(256, 2) void varlen_attn_kernel(VarlenArgs a) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[VARLEN_SMEM];
-  varlen_workgroup<VERIFY, false>(a, smem, blockIdx.x, gridDim.x);
+  varlen_workgroup<VERIFY, false, TILED>(a, smem, blockIdx.x, gridDim.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -1271,15 +1271,15 @@ __device__ __forceinline__ void draft_pair_item(const DraftArgs& a, unsigned cha
   // Only stages that hold context are loaded, so the number of ring loads
   // still in flight behind a given one is known: all but the newest
   // `behind` stages of LPS loads each (PER_WAVE pieces, and with indices
-  // one index load) have landed after stage_barrier, for every wave.
+  // one index load) have landed after wait_stages.
   constexpr int LPS = R::PER_WAVE + (INDEXED ? 1 : 0);
-  auto stage_barrier = [](int behind) {
-    if (behind <= 0) ring_barrier<0>();
-    else if (behind == 1) ring_barrier<LPS>();
-    else if (behind == 2 || R::STAGES < 4) ring_barrier<2 * LPS>();
-    else ring_barrier<3 * LPS>();
+  auto wait_stages = [](int behind) {
+    if (behind <= 0) load_wait<0>();
+    else if (behind == 1) load_wait<LPS>();
+    else if (behind == 2 || R::STAGES < 4) load_wait<2 * LPS>();
+    else load_wait<3 * LPS>();
   };
-  static_assert(R::STAGES <= 4, "stage_barrier covers at most three stages in flight");
+  static_assert(R::STAGES <= 4, "wait_stages covers at most three stages in flight");
   static_assert(R::STAGES == 3 || !INDEXED, "the index prologue loads two stages");
   const int prologue = min(R::STAGES - 1, n_steps);
   if constexpr (INDEXED) {
@@ -1287,9 +1287,9 @@ __device__ __forceinline__ void draft_pair_item(const DraftArgs& a, unsigned cha
     // row loads issued after them are in flight.
     if (n_steps > 0) {
       const int after = (q_lds ? R::PER_WAVE : 0) + (last ? R::PER_WAVE : 0);
-      if (after == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      else if (after == R::PER_WAVE) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(R::PER_WAVE) : "memory");
-      else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * R::PER_WAVE) : "memory");
+      if (after == 0) load_wait<0>();
+      else if (after == R::PER_WAVE) load_wait<R::PER_WAVE>();
+      else load_wait<2 * R::PER_WAVE>();
     }
   }
   #pragma unroll
@@ -1297,7 +1297,8 @@ __device__ __forceinline__ void draft_pair_item(const DraftArgs& a, unsigned cha
     if (p < prologue) issue(p);
   TL_MARK(1);
   if (last) {
-    stage_barrier(prologue);   // the Q and own rows, issued first, have landed
+    wait_stages(prologue);   // the Q and own rows, issued first, have landed
+    ring_barrier();
     TL_MARK(2);
     if (q_lds) read_q();
     if (active && kh == 0) {
@@ -1328,7 +1329,8 @@ __device__ __forceinline__ void draft_pair_item(const DraftArgs& a, unsigned cha
     // the top of step s the stages issued after stage s number
     // min(n_steps - 1 - s, STAGES - 2).
     auto step = [&](int s) {
-      stage_barrier(min(n_steps - 1 - s, R::STAGES - 2));
+      wait_stages(min(n_steps - 1 - s, R::STAGES - 2));
+      ring_barrier();
 #ifdef DSPARK_TIMELINE
       if (s == 0 && !last) TL_MARK(2);
 #endif
@@ -1342,7 +1344,7 @@ __device__ __forceinline__ void draft_pair_item(const DraftArgs& a, unsigned cha
   // overlaps the merge below (a draw inside the stream loop, right after the
   // ring's last stage load, made the compiler spill the loop's registers).
   draw();
-  lds_barrier();   // every wave is done with the ring and the own rows
+  ring_barrier();   // every wave is done with the ring and the own rows
   TL_MARK(3);
 
   // The key halves merge: the kh = 1 wave of each pair leaves its state in
@@ -1808,7 +1810,7 @@ __global__ __launch_bounds__(PF_WAVES * WAVE, 2) void prefill_attn_kernel(Varlen
   const int row = blockIdx.y + PF_SEGS_Y * blockIdx.z;
   const int wid = (int)(blockIdx.x + gridDim.x * (unsigned)row);        // keeps the XCD: gridDim.x is a multiple of 8
   if (a.columns ? wid < decode_grid : row < decode_rows) {
-    if (wid < decode_grid) varlen_workgroup<VERIFY, true>(a, smem, wid, decode_grid);
+    if (wid < decode_grid) varlen_workgroup<VERIFY, true, true>(a, smem, wid, decode_grid);
     return;
   }
   const int g = blockIdx.x & 7;
@@ -1935,7 +1937,8 @@ __global__ __launch_bounds__(PF_WAVES * WAVE, 2) void prefill_attn_kernel(Varlen
   auto arrive = [&]() {
     // not before the MFMAs of the step that ends here, which hide the loads
     __builtin_amdgcn_sched_barrier(0);
-    ring_barrier<0>();
+    load_wait<0>();
+    ring_barrier();
   };
   auto enter = [&](int s) {
     arrive();
@@ -2205,7 +2208,7 @@ int varlen_launch(VarlenArgs& a, int64_t key_rows_bound, int max_q, float scale,
   hipStream_t s = static_cast<hipStream_t>(stream);
   const unsigned grid = work ? (unsigned)n_groups * HKV : persistent_grid(a.n_slots);
   if (max_q <= DECODE_TOKENS) {
-    hipLaunchKernelGGL(varlen_attn_kernel<VERIFY>, dim3(grid), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((varlen_attn_kernel<VERIFY, false>), dim3(grid), dim3(256), 0, s, a);
     rc = launch_status(what);
   } else {
     rc = launch_prefill<VERIFY>(a, grid, (unsigned)n_cl, max_q, s);
@@ -2351,7 +2354,7 @@ extern "C" int dspark_mixed_attn_fwd(const void* q, const void* k, const void* v
   const int32_t* requests = work + WORK_INTS * n_work + n_groups + 1;
   const unsigned grid = (unsigned)n_groups * HKV;
   if (n_columns == 0) {
-    hipLaunchKernelGGL(verify ? varlen_attn_kernel<true> : varlen_attn_kernel<false>, dim3(grid), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((verify ? varlen_attn_kernel<true, true> : varlen_attn_kernel<false, false>), dim3(grid), dim3(256), 0, s, a);
     rc = launch_status("varlen_attn_kernel");
   } else {
     a.columns = requests + REQ_INTS * n_req;

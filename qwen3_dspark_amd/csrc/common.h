@@ -133,18 +133,18 @@ __device__ __forceinline__ void lds_dma16_base(const void* base, uint32_t offset
   asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "{m0}"(lds) : "memory");
 }
 
-// The barrier of a ring of direct loads: all but the wave's newest IN_FLIGHT
-// loads have landed, and its LDS reads are done, so that the loads which the other
-// waves issue behind the barrier may overwrite what it read.  One asm statement, because
-// nothing else keeps an LDS read ahead of a barrier that it does not depend on.
+// All but the wave's newest IN_FLIGHT loads have landed.
 template <int IN_FLIGHT>
-__device__ __forceinline__ void ring_barrier() {
+__device__ __forceinline__ void load_wait() {
   static_assert(IN_FLIGHT >= 0 && IN_FLIGHT < 63, "vmcnt holds 6 bits");
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(IN_FLIGHT) : "memory");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(IN_FLIGHT) : "memory");
 }
 
-// The same without a wait for loads.
-__device__ __forceinline__ void lds_barrier() {
+// The barrier of a ring of direct loads, after the load_wait: the wave's LDS reads are
+// done, so that the loads which the other waves issue behind the barrier may
+// overwrite what it read.  One asm statement, because nothing else keeps an LDS read
+// ahead of a barrier that it does not depend on.
+__device__ __forceinline__ void ring_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 

@@ -151,9 +151,10 @@ __device__ __forceinline__ void head_tile_gemm(const bf16* __restrict__ w, const
     // every wave's stage-s loads landed (the STAGES - 2 stages behind it, as
     // far as there are any, may still be in flight) and its reads of stage s - 1,
     // which the next loads overwrite, are done
-    if (Ring::STAGES == 4 && s + 2 < steps) ring_barrier<2 * Ring::LOADS>();
-    else if (s + 1 < steps) ring_barrier<Ring::LOADS>();
-    else ring_barrier<0>();
+    if (Ring::STAGES == 4 && s + 2 < steps) load_wait<2 * Ring::LOADS>();
+    else if (s + 1 < steps) load_wait<Ring::LOADS>();
+    else load_wait<0>();
+    ring_barrier();
     if (s + Ring::STAGES - 1 < steps) issue(s + Ring::STAGES - 1);
     const unsigned char* wst = smem + (s % Ring::STAGES) * Ring::STAGE_BYTES + L.kq * Ring::SUB_BYTES;
     const unsigned char* xst = wst + HG_W_BYTES;

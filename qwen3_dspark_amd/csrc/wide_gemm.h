@@ -89,7 +89,8 @@ __device__ __forceinline__ void wide_tile_gemm(const bf16* __restrict__ w, const
   for (int s = 0; s < steps; ++s) {
     // stage s has landed for every wave, whose LDS reads of stage s - 1 are done
     __builtin_amdgcn_sched_barrier(0);
-    ring_barrier<0>();
+    load_wait<0>();
+    ring_barrier();
     if (s + 1 < steps) issue(s + 1);
     const unsigned char* wst = smem + (s & 1) * WG_STAGE;
     const unsigned char* xst = wst + WG_PART;
