@@ -709,7 +709,7 @@ class DraftKVPool:
             self._lengths[request] += value.shape[1]
         e, H, D = self._elems[0], self.heads, self.dim
         self.last_append_work = dict(requests=len(order), new_context_tokens=first, context_projection_calls=1,
-                                     kv_projection_calls=self.layers, projection_launches=2,
+                                     kv_projection_calls=self.layers, projection_launches=proj.launches(first),
                                      appended_kv_bytes=2 * self.layers * first * H * D * e,
                                      cache_concatenation_kv_elements=0, cache_concatenation_kv_bytes=0)
         return self.last_append_work

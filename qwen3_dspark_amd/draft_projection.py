@@ -19,7 +19,10 @@ dspark_draft_kv_project_rows projects 128-token tiles instead, after one
 launch that computes what depends on the token alone.  path='gemm' runs the
 k/v projection as a library GEMM per GEMM_CHUNK tokens (all layers' folded
 weights as one matrix, bf16 operands, FP32 output) followed by
-dspark_draft_kv_epilogue; no length takes it by default.  All paths keep
+dspark_draft_kv_epilogue: no length takes it by default, since the wide tiles
+are faster at every length measured (see _path); it is there for callers that
+name it, or lower GEMM_MIN_TOKENS, as the matrix-rate probe of bench.py and the
+tests do.  All paths keep
 the projection in FP32 through the norms and RoPE and round every output to
 bf16 once, so the path a given append length takes changes only the
 accumulation order.
@@ -32,7 +35,7 @@ from .kernels import HEAD_DIM, KV_HEADS
 from .prologue import rope_inv_freq
 
 
-GEMM_MIN_TOKENS = float('inf')   # appends at least this long take the library GEMM + epilogue path
+GEMM_MIN_TOKENS = float('inf')   # appends at least this long take the library GEMM + epilogue path (none)
 GEMM_CHUNK = 16384       # tokens per library GEMM (bounds its FP32 output: 640 MiB at 5 layers)
 PATHS = ('fused', 'wide', 'gemm')
 
@@ -107,6 +110,10 @@ class DraftContextProjector:
         if t >= GEMM_MIN_TOKENS:
             return 'gemm'
         return 'wide' if -(-t // 64) * 16 * self.layers > cu_count(self.device) else 'fused'
+
+    def launches(self, t):
+        """Launches that project an append of t tokens: fc, and its path's."""
+        return 1 + {'fused': 1, 'wide': 2, 'gemm': 2 * -(-t // GEMM_CHUNK)}[self._path(t)]
 
     def project_into(self, fc_out, records, n_req, keys, values, *, flag=None, path=None):
         """The projection of fc_out [T, hidden] into pool tensors keys /
