@@ -80,8 +80,9 @@ int64_t dspark_attn_workspace_bytes(int n_req, int64_t key_rows_bound, int row_t
  *       first query row, query length
  * Requests with more than 8 query tokens (in a call whose max_q exceeds 8)
  * are attended by workgroups of their own, one per (record, KV head, 32 query
- * tokens): their records may stand in any run or, after the last run's
- * records, in none (records with query length 0 are skipped).
+ * tokens), or, where few keys make that slower, by a run's workgroups per 8 query
+ * tokens; which one, their own lengths decide.  Their records may stand in any run
+ * or, after the last run's records, in none (records with query length 0 are skipped).
  * The segments of a request must cover its keys exactly once, and a split
  * request's segments must use consecutive partial slots in key order (the
  * merge folds them in slot order).  Cuts at the same key positions give

@@ -40,6 +40,7 @@
 // triples that merge_kernel combines; the kernel boundary makes them visible
 // without any per-workgroup cache flush.
 #include <atomic>
+#include <limits>
 #include <mutex>
 #include <type_traits>
 
@@ -277,7 +278,9 @@ struct VarlenArgs {
   float* part_ml;         // [partial tiles][16][2]
   int n_req;
   int n_work;             // segment records in the work list
-  int tile_shift;         // a record's first word from this bit on: its tile of 8 query tokens
+  int n_groups;           // runs of the work list
+  int planes;             // PLANES launches: row tiles of the requests that plane_form says
+  int64_t plane_keys;
   int n_slots;            // no list: (chunk, KV head) slots, 8 * chunks
   int causal;
   int chunk;
@@ -329,6 +332,27 @@ __device__ __forceinline__ size_t part_tile(int slot, int g, int t, int tmax) {
   return tmax ? ((size_t)slot * 8 + g) * tmax + t : (size_t)(slot + t) * 8 + g;
 }
 
+// What a workgroup of the runs makes of a request's rows.
+//   WHOLE:   requests of up to DECODE_TOKENS alone.
+//   RECORDS: a record may be one row tile of a longer request (a mixed plan's;
+//            its number stands from bit 24 of the first word on, and the key length
+//            ends with its last token).
+//   PLANES:  records hold whole requests; workgroups of plane t attend row tile t of
+//            those that plane_form accepts.
+enum RowTiles { WHOLE, RECORDS, PLANES };
+
+// Requests that the planes attend, by their own lengths (a request-local plan's
+// results do not depend on the batch): over few keys the prompt form's one
+// stage after the other is slower than tiles that read the keys again.  Prompt
+// form / planes in a request-local plan, us: 9 tokens over 300 keys 13.3 / 9.2, over
+// 2,000 26.5 / 18.4; 64 over 300 15.7 / 11.5; 8 prompts of 16 over 1,000 26.2 / 17.1, but
+// over 4,080 30.5 / 45.9.
+constexpr int MAX_PLANES = 8;
+constexpr int64_t PLANE_KEYS = 6144;                 // row tiles x keys
+__device__ __forceinline__ bool plane_form(const VarlenArgs& a, int ql, int kl) {
+  return ql <= DECODE_TOKENS * a.planes && (int64_t)((ql + DECODE_TOKENS - 1) / DECODE_TOKENS) * kl <= a.plane_keys;
+}
+
 // The addressing of one segment for one KV head; every field is
 // wave-uniform.  Key j of the request lives in part A (committed rows) for
 // j < a_len, else in part B (rows new to this call).
@@ -348,9 +372,9 @@ struct SegView {
 };
 
 // MIXED: the launch also has requests that prefill workgroups attend; their
-// segments have no live rows here.  TILED: records may be row tiles of a request.
-template <bool VERIFY, bool MIXED, bool TILED>
-__device__ __forceinline__ SegView seg_view(const VarlenArgs& a, const Segment& sg, int g) {
+// segments have no live rows here.
+template <bool VERIFY, bool MIXED, RowTiles TILES>
+__device__ __forceinline__ SegView seg_view(const VarlenArgs& a, const Segment& sg, int g, int plane) {
   SegView v;
   // The segment is wave-uniform; say so, so that its fields and everything
   // derived from them stay in scalar registers.
@@ -362,10 +386,19 @@ __device__ __forceinline__ SegView seg_view(const VarlenArgs& a, const Segment& 
   const int k1 = __builtin_amdgcn_readfirstlane(sg.k1);
   v.pslot = __builtin_amdgcn_readfirstlane(sg.pslot);
   v.live = v.ql > 0 && (!MIXED || v.ql <= DECODE_TOKENS);
-  v.ends = k1 == v.kl && (!MIXED || v.live);
+  v.ends = k1 == v.kl;
+  int before = 0;                  // query rows of the request before this tile
+  if (TILES == RECORDS) before = DECODE_TOKENS * (__builtin_amdgcn_readfirstlane(sg.r) >> 24);
+  if (TILES == PLANES) {
+    before = DECODE_TOKENS * plane < v.ql ? DECODE_TOKENS * plane : 0;
+    const int rows = DECODE_TOKENS * plane < v.ql ? min(DECODE_TOKENS, v.ql - before) : 0;
+    v.live = rows > 0 && (v.ql <= DECODE_TOKENS || plane_form(a, v.ql, v.kl));
+    v.q0 += before;
+    if (a.causal) v.kl -= v.ql - before - rows;      // what the tile's last token sees
+    v.ql = rows;
+  }
+  v.ends = v.ends && (!MIXED || v.live);
   if (VERIFY) {
-    // query rows of the request before this tile (kl ends with the tile)
-    const int before = TILED ? DECODE_TOKENS * (__builtin_amdgcn_readfirstlane(sg.r) >> a.tile_shift) : 0;
     v.a_len = v.kl - v.ql - before;
     const size_t abase = (size_t)start * (size_t)a.slot_stride + (size_t)g * a.a_head_stride;
     v.kA = a.k_a + abase;
@@ -459,8 +492,8 @@ __device__ __forceinline__ void load_q(const VarlenArgs& a, const SegView& s, in
 // k0 + 32w, k0 + 32(w+4), ... of each segment.
 // fetch(n, sg) yields the run's n-th segment (false past the end); every
 // branch on it is uniform across the workgroup.
-template <bool VERIFY, bool MIXED, bool TILED, typename Fetch>
-__device__ __forceinline__ void varlen_run(const VarlenArgs& a, unsigned char* smem, int g, Fetch fetch) {
+template <bool VERIFY, bool MIXED, RowTiles TILES, typename Fetch>
+__device__ __forceinline__ void varlen_run(const VarlenArgs& a, unsigned char* smem, int g, int plane, Fetch fetch) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int col = lane & 15;
@@ -478,7 +511,7 @@ __device__ __forceinline__ void varlen_run(const VarlenArgs& a, unsigned char* s
 
   Segment sg;
   if (!fetch(0, sg)) return;
-  SegView cur = seg_view<VERIFY, MIXED, TILED>(a, sg, g);
+  SegView cur = seg_view<VERIFY, MIXED, TILES>(a, sg, g, plane);
   bf16x8 qf[4];
   for (int n = 0;; ++n) {
     load_q(a, cur, g, qf);
@@ -588,7 +621,7 @@ __device__ __forceinline__ void varlen_run(const VarlenArgs& a, unsigned char* s
       const int tok_r = row >> 1;
       const int head_r = 2 * g + (row & 1);
       if (cur.pslot >= 0) {
-        const size_t p = part_tile(cur.pslot, g, 0, a.tmax);
+        const size_t p = part_tile(cur.pslot, g, plane, a.tmax);
         float* po = a.part_o + (p * 16 + row) * HD + d0;
         *reinterpret_cast<f32x4*>(po) = f32x4{acc[0], acc[1], acc[2], acc[3]};
         *reinterpret_cast<f32x4*>(po + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]};
@@ -613,7 +646,7 @@ __device__ __forceinline__ void varlen_run(const VarlenArgs& a, unsigned char* s
     }
     __syncthreads();   // the next segment reuses the V tiles and the merge buffer
     if (!more) break;
-    cur = seg_view<VERIFY, MIXED, TILED>(a, nsg, g);
+    cur = seg_view<VERIFY, MIXED, TILES>(a, nsg, g, plane);
   }
 }
 
@@ -651,8 +684,8 @@ __device__ __forceinline__ uint64_t tl_now() { return __builtin_amdgcn_s_memreal
 // Without a list, a persistent grid walks the fixed chunks (item, KV head)
 // with a stride of the grid size, so per-workgroup start-up is paid once
 // per CU slot.
-template <bool VERIFY, bool MIXED, bool TILED>
-__device__ __forceinline__ void varlen_workgroup(const VarlenArgs& a, unsigned char* smem, int wid, int grid) {
+template <bool VERIFY, bool MIXED, RowTiles TILES>
+__device__ __forceinline__ void varlen_workgroup(const VarlenArgs& a, unsigned char* smem, int wid, int grid, int plane) {
   const int slot = wid >> 3;
   const int g = a.work ? (slot & 7) : (wid & 7);
   if (a.work) {
@@ -664,9 +697,25 @@ __device__ __forceinline__ void varlen_workgroup(const VarlenArgs& a, unsigned c
     const uint64_t tl_start = tl_now();
     int tl_keys = 0;
 #endif
-    varlen_run<VERIFY, MIXED, TILED>(a, smem, g, [&](int n, Segment& sg) {
-      if (b + n >= e) return false;
-      const int32_t* w = a.work + WORK_INTS * (b + n);
+    int skipped = 0;
+    varlen_run<VERIFY, MIXED, TILES>(a, smem, g, plane, [&](int n, Segment& sg) {
+      int i = b + n;
+      if (TILES == PLANES) {
+        // the run's records, then those of no run, dealt over the runs; without those
+        // that have no row tile here
+        const int loose = min(max(__builtin_amdgcn_readfirstlane(range[a.n_groups - run]), 0), a.n_work) + run;
+        for (;; ++skipped) {
+          i = b + n + skipped;
+          if (i >= e) i = loose + (i - e) * a.n_groups;
+          if (i >= a.n_work) return false;
+          const int32_t* w = a.work + WORK_INTS * i;
+          const int ql = __builtin_amdgcn_readfirstlane(w[5]), kl = __builtin_amdgcn_readfirstlane(w[6]);
+          if (ql > DECODE_TOKENS * plane && (ql <= DECODE_TOKENS || plane_form(a, ql, kl))) break;
+        }
+      } else if (i >= e) {
+        return false;
+      }
+      const int32_t* w = a.work + WORK_INTS * i;
       sg = Segment{w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7]};
 #ifdef DSPARK_TIMELINE
       tl_keys += sg.k1 - sg.k0;
@@ -688,16 +737,16 @@ __device__ __forceinline__ void varlen_workgroup(const VarlenArgs& a, unsigned c
 #endif
     return;
   }
-  varlen_run<VERIFY, MIXED, TILED>(a, smem, g, [&](int n, Segment& sg) {
+  varlen_run<VERIFY, MIXED, TILES>(a, smem, g, plane, [&](int n, Segment& sg) {
     const int idx = wid + n * grid;
     return idx < a.n_slots && chunk_segment(a, VERIFY, idx >> 3, sg);
   });
 }
 
-template <bool VERIFY, bool TILED>
+template <bool VERIFY, RowTiles TILES>
 __global__ __launch_bounds__(256, 2) void varlen_attn_kernel(VarlenArgs a) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[VARLEN_SMEM];
-  varlen_workgroup<VERIFY, false, TILED>(a, smem, blockIdx.x, gridDim.x);
+  varlen_workgroup<VERIFY, false, TILES>(a, smem, blockIdx.x, gridDim.x, TILES == PLANES ? blockIdx.y : 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1796,27 +1845,31 @@ __device__ __forceinline__ void prefill_merge(const VarlenArgs& a, const float* 
 }
 
 // A call whose max_q exceeds DECODE_TOKENS is one launch: first the workgroups that
-// walk the runs for the requests of up to DECODE_TOKENS, then the prompts'.  With
-// `columns` (a mixed plan) those are the listed (record, tile) pairs, in the
-// order of the list, which starts with the longest; else the grid is
-// gridDim.x = 8 x the tiles of max_q wide, its first `decode_rows` rows walk
-// the runs, and one row follows per record: each request is then attended by one
-// of the two forms by its own query count.
-template <bool VERIFY>
+// walk the runs, then the prompts'.  With COLUMNS (a mixed plan) those are the listed
+// (record, tile) pairs, in the order of the list, which starts with the longest; else
+// the grid is gridDim.x = 8 x the tiles of max_q wide, its first `decode_rows` rows
+// walk the runs (or fixed chunks), a plane after the other, and one row follows per
+// record: each request is then attended by one of the two forms by its own lengths.
+template <bool VERIFY, bool COLUMNS>
 __global__ __launch_bounds__(PF_WAVES * WAVE, 2) void prefill_attn_kernel(VarlenArgs a, int decode_grid, int decode_rows) {
   // 1 KiB alignment: tile offsets are XORed into LDS addresses.
   __shared__ __attribute__((aligned(1024))) unsigned char smem[PF_SMEM];
   static_assert(PF_SMEM >= VARLEN_SMEM && PF_WAVES * WAVE == 256, "one launch shape for both forms");
   const int row = blockIdx.y + PF_SEGS_Y * blockIdx.z;
   const int wid = (int)(blockIdx.x + gridDim.x * (unsigned)row);        // keeps the XCD: gridDim.x is a multiple of 8
-  if (a.columns ? wid < decode_grid : row < decode_rows) {
-    if (wid < decode_grid) varlen_workgroup<VERIFY, true, true>(a, smem, wid, decode_grid);
+  if (COLUMNS ? wid < decode_grid : row < decode_rows) {
+    if (COLUMNS) {
+      varlen_workgroup<VERIFY, true, RECORDS>(a, smem, wid, decode_grid, 0);
+    } else {
+      const int plane = wid / decode_grid;
+      if (plane < a.planes) varlen_workgroup<VERIFY, true, PLANES>(a, smem, wid - plane * decode_grid, decode_grid, plane);
+    }
     return;
   }
   const int g = blockIdx.x & 7;
   int t = (gridDim.x >> 3) - 1 - (blockIdx.x >> 3);
   int seg = row - decode_rows;
-  if (a.columns) {
+  if (COLUMNS) {
     const int32_t* column = a.columns + 2 * ((wid - decode_grid) >> 3);
     seg = min(__builtin_amdgcn_readfirstlane(column[0]), a.n_work) - 1;
     t = max(__builtin_amdgcn_readfirstlane(column[1]), 0);
@@ -1824,16 +1877,17 @@ __global__ __launch_bounds__(PF_WAVES * WAVE, 2) void prefill_attn_kernel(Varlen
     seg = a.n_work - 1 - seg;        // a plan puts its prompts after the runs, longest last
   }
   Segment sg;
-  if (a.work) {
+  if (COLUMNS || a.work) {
     const int32_t* w = a.work + WORK_INTS * max(seg, 0);        // no record: no query tokens
     sg = Segment{w[0], w[1], w[2], w[3], w[4], seg < 0 ? 0 : w[5], w[6], w[7]};
   } else if (!chunk_segment(a, VERIFY, seg, sg)) {
     return;
   }
-  const int ql = __builtin_amdgcn_readfirstlane(sg.ql);
+  const int kl = __builtin_amdgcn_readfirstlane(sg.kl);
+  int ql = __builtin_amdgcn_readfirstlane(sg.ql);
+  if (!COLUMNS && plane_form(a, ql, kl)) ql = 0;               // the planes attend it
   if (ql <= DECODE_TOKENS || PF_TOKENS * t >= ql) return;      // uniform across the workgroup
   const int q0 = __builtin_amdgcn_readfirstlane(sg.q0);
-  const int kl = __builtin_amdgcn_readfirstlane(sg.kl);
   const int k0 = __builtin_amdgcn_readfirstlane(sg.k0);
   const int k1 = __builtin_amdgcn_readfirstlane(sg.k1);
   const int start = __builtin_amdgcn_readfirstlane(sg.start);
@@ -2101,15 +2155,15 @@ using namespace dspark;
 constexpr float LOG2E = 1.4426950408889634f;
 
 // Workgroups resident at once for the varlen/verify kernel (2 per CU at its
-// register budget).
-unsigned persistent_grid(int n_slots) {
+// register budget), over the planes of a launch.
+unsigned persistent_grid(int n_slots, int planes) {
   static int cus = 0;
   if (!cus) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
       cus = 256;
   }
-  const int64_t resident = std::max<int64_t>(8, (int64_t)cus * 2 / 8 * 8);
+  const int64_t resident = std::max<int64_t>(8, (int64_t)cus * 2 / planes / 8 * 8);
   return (unsigned)std::min<int64_t>(n_slots, resident);
 }
 
@@ -2166,13 +2220,21 @@ extern "C" int64_t dspark_attn_workspace_bytes(int n_req, int64_t key_rows_bound
 
 namespace {
 
-// `grid` workgroups over the runs (or fixed chunks), then `prompts` rows of the prompt form.
+// A launch without a work list attends every request by row tiles if the longest
+// has at most MAX_PLANES of them and tiles x the bound of the key rows is at most
+// this (the bucket alone decides).  Prompt form / row tiles, us: 9 tokens over 2,000
+// keys 27.5 / 15.7, over 8,000 28.1 / 19.7; 64 over 300 16.7 / 9.8, over 2,000 24.7 / 16.7; 8
+// prompts of 16 over 1,000 27.1 / 17.5.
+constexpr int64_t CHUNK_PLANE_KEYS = 24576;
+
+// `grid` workgroups over the runs (or fixed chunks) per plane, then `prompts` rows
+// of the prompt form.
 template <bool VERIFY>
 int launch_prefill(const VarlenArgs& a, unsigned grid, unsigned prompts, int max_q, hipStream_t s) {
   const unsigned gx = HKV * ((max_q + PF_TOKENS - 1) / PF_TOKENS);
-  const unsigned decode_rows = (grid + gx - 1) / gx;
+  const unsigned decode_rows = (grid * a.planes + gx - 1) / gx;
   const unsigned rows = decode_rows + prompts;
-  hipLaunchKernelGGL(prefill_attn_kernel<VERIFY>, dim3(gx, std::min(rows, (unsigned)PF_SEGS_Y), (rows + PF_SEGS_Y - 1) / PF_SEGS_Y),
+  hipLaunchKernelGGL((prefill_attn_kernel<VERIFY, false>), dim3(gx, std::min(rows, (unsigned)PF_SEGS_Y), (rows + PF_SEGS_Y - 1) / PF_SEGS_Y),
                      dim3(256), 0, s, a, (int)grid, (int)decode_rows);
   return launch_status("prefill_attn_kernel");
 }
@@ -2202,13 +2264,19 @@ int varlen_launch(VarlenArgs& a, int64_t key_rows_bound, int max_q, float scale,
   a.part_ml = a.part_o + n_cl * HKV * tiles * 16 * HD;
   a.chunk = chunk;
   a.tmax = tiles;
-  a.tile_shift = 31;
+  a.n_groups = n_groups;
+  const bool all_planes = !work && tiles <= MAX_PLANES && tiles * key_rows_bound <= CHUNK_PLANE_KEYS;
+  a.planes = work ? std::min(tiles, MAX_PLANES) : (all_planes ? tiles : 1);
+  a.plane_keys = work ? PLANE_KEYS : (all_planes ? std::numeric_limits<int64_t>::max() : 0);
   a.scale_log2 = scale * LOG2E;
   a.n_slots = (int)(n_cl * HKV);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const unsigned grid = work ? (unsigned)n_groups * HKV : persistent_grid(a.n_slots);
+  const unsigned grid = work ? (unsigned)n_groups * HKV : persistent_grid(a.n_slots, all_planes ? tiles : 1);
   if (max_q <= DECODE_TOKENS) {
-    hipLaunchKernelGGL((varlen_attn_kernel<VERIFY, false>), dim3(grid), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((varlen_attn_kernel<VERIFY, WHOLE>), dim3(grid), dim3(256), 0, s, a);
+    rc = launch_status(what);
+  } else if (all_planes) {
+    hipLaunchKernelGGL((varlen_attn_kernel<VERIFY, PLANES>), dim3(grid, tiles), dim3(256), 0, s, a);
     rc = launch_status(what);
   } else {
     rc = launch_prefill<VERIFY>(a, grid, (unsigned)n_cl, max_q, s);
@@ -2348,17 +2416,16 @@ extern "C" int dspark_mixed_attn_fwd(const void* q, const void* k, const void* v
   a.n_work = n_work;
   a.causal = causal ? 1 : 0;
   a.tmax = 0;
-  a.tile_shift = 24;
   a.scale_log2 = scale * LOG2E;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int32_t* requests = work + WORK_INTS * n_work + n_groups + 1;
   const unsigned grid = (unsigned)n_groups * HKV;
   if (n_columns == 0) {
-    hipLaunchKernelGGL((verify ? varlen_attn_kernel<true, true> : varlen_attn_kernel<false, false>), dim3(grid), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((verify ? varlen_attn_kernel<true, RECORDS> : varlen_attn_kernel<false, RECORDS>), dim3(grid), dim3(256), 0, s, a);
     rc = launch_status("varlen_attn_kernel");
   } else {
     a.columns = requests + REQ_INTS * n_req;
-    hipLaunchKernelGGL(verify ? prefill_attn_kernel<true> : prefill_attn_kernel<false>,
+    hipLaunchKernelGGL((verify ? prefill_attn_kernel<true, true> : prefill_attn_kernel<false, true>),
                        dim3(grid + (unsigned)n_columns * HKV), dim3(256), 0, s, a, (int)grid, 0);
     rc = launch_status("prefill_attn_kernel");
   }
