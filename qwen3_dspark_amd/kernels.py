@@ -122,9 +122,9 @@ class HipVarlenKernel:
         if len(listed) > 3:
             work, n_work, runs, records, columns, tiles = listed
             ws = self._workspace.get(PART_TILE_BYTES * tiles)
-            _native.call('dspark_mixed_attn_fwd', _native.ptr(query), _native.ptr(key), _native.ptr(value), None, None,
-                         None, None, records, 0, 0, 0, max_q, int(self.causal), float(SCALE), _native.ptr(work), n_work,
-                         runs, columns, tiles, _native.ptr(out), _native.ptr(ws), ws.numel(),
+            _native.call('dspark_mixed_attn_fwd', query.data_ptr(), key.data_ptr(), value.data_ptr(), None, None, None,
+                         None, records, 0, 0, 0, max_q, int(self.causal), SCALE, work.data_ptr(), n_work, runs,
+                         columns, tiles, out.data_ptr(), ws.data_ptr(), ws.numel(),
                          _native.stream_handle(self.device))
             return out
         work, n_work, runs = listed

@@ -85,7 +85,7 @@ class Workspace:
         for name, t in tensors.items():
             setattr(self, name, t)
         self._names = tuple(tensors)
-        self.mixed = None        # counts of the bucket's mixed plans (MixedPlan without its list), from the first on
+        self.counts = None       # of the bucket's work lists (HipKVDevice.list_counts)
 
     def tensors(self):
         return {name: getattr(self, name) for name in self._names}
@@ -150,6 +150,16 @@ class HipKVDevice:
         """(record capacity, runs) of a bucket's fixed-capacity work list."""
         return _list_shape(shape, self.device, self.chunk, self.split)
 
+    def list_counts(self, ws, shape):
+        """(capacity, counts) of the bucket's work lists in ws: a mixed plan's
+        MixedCapacity and MixedPlan without its list, or None and (records,
+        runs).  They depend on the bucket and its buffers alone."""
+        if ws.counts is None:
+            c = _mixed_shape(shape, self.device, self.split, ws.attn.numel() // PART_TILE_BYTES)
+            ws.counts = (c, self.launch_shape(shape) if c is None else
+                         (c.run_records + c.prompt_records, c.runs, c.requests, c.columns, c.tiles))
+        return ws.counts
+
     # -- workspaces -----------------------------------------------------------
     def workspace(self, shape):
         """Allocate the buffers of a bucket, or of a family arena whose shape
@@ -202,16 +212,14 @@ class HipKVDevice:
         published if the list does not fit or a launch fails."""
         key_lengths = [c + q for c, q in zip(contexts, query_lengths)]
         n_cu = cu_count(self.device)
-        capacity = _mixed_shape(shape, self.device, self.split, ws.attn.numel() // PART_TILE_BYTES)
+        capacity, counts = self.list_counts(ws, shape)
         if capacity is not None:
-            plan = mixed_plan(query_lengths, key_lengths, slots, n_cu, capacity=capacity, xcd_speed=self.xcd_speed,
-                              slot_balance=self.slot_balance)
-            records, ws.mixed = plan.records, plan[1:]
+            records = mixed_plan(query_lengths, key_lengths, slots, n_cu, capacity=capacity, xcd_speed=self.xcd_speed,
+                                 slot_balance=self.slot_balance).records
         else:
             runs = run_count(sum(key_lengths), n_cu, (shape.maximum_query_length + 7) // 8)
-            records, _, _ = segment_plan(self.split, query_lengths, key_lengths, slots, runs, self.chunk,
-                                         self.launch_shape(shape), xcd_speed=self.xcd_speed,
-                                         n_cu=n_cu if self.slot_balance else None)
+            records, _, _ = segment_plan(self.split, query_lengths, key_lengths, slots, runs, self.chunk, counts,
+                                         xcd_speed=self.xcd_speed, n_cu=n_cu if self.slot_balance else None)
         if len(records) > ws.work.numel():
             raise ValueError('Work list exceeds the bucket workspace')
         r = len(slots)
@@ -247,8 +255,9 @@ class HipKVDevice:
         time."""
         C = self.capacity
         k, v, sk, sv = self.layer_pointers[layer]
-        if ws.mixed is not None:
-            n_work, runs, requests, columns, tiles = ws.mixed
+        capacity, counts = self.list_counts(ws, shape)
+        if capacity is not None:
+            n_work, runs, requests, columns, tiles = counts
             new = (sk, sv, None, None) if keys is None else (keys, values, sk, sv)
             _native.call('dspark_mixed_attn_fwd', query, k, v, *new, requests, KV_HEADS * C * HEAD_DIM, HEAD_DIM,
                          C * HEAD_DIM, shape.maximum_query_length, 1, SCALE, ws.work.data_ptr(), n_work, runs,
@@ -258,7 +267,7 @@ class HipKVDevice:
         tail = (ws.cu_query.data_ptr(), ws.cu_key.data_ptr(), ws.req.data_ptr(),
                 shape.request_count, KV_HEADS * C * HEAD_DIM, HEAD_DIM, C * HEAD_DIM,
                 shape.key_capacity, shape.maximum_query_length, SCALE, self.chunk,
-                ws.work.data_ptr(), *self.launch_shape(shape), out, ws.attn.data_ptr(), ws.attn.numel(),
+                ws.work.data_ptr(), *counts, out, ws.attn.data_ptr(), ws.attn.numel(),
                 _native.stream_handle(self.device))
         if keys is not None:
             _native.call('dspark_verify_attn_staged_fwd', query, k, v, keys, values, sk, sv, *tail)

@@ -132,13 +132,12 @@ def run_count(total_keys, n_cu, row_tiles=1):
     return -(-runs // XCDS) * XCDS
 
 
-def _flatten(n, per_run, record, request, loose=(), width=None):
+def _flatten(n, per_run, record, request, loose=()):
     """Flatten per-run [(request, k0, k1)] segment lists into the int32 list
     format, giving split requests consecutive request-major partial slots in
     key order.  record(r, k0, k1, slot) and request(r, first, count) give the
     8 and 4 ints of a segment and a request.  loose: segments of no run, after
-    the runs' records.  width(r): slots that a segment of request r takes (one
-    without).  Returns (list, segment count, run count)."""
+    the runs' records.  Returns (list, segment count, run count)."""
     loose = list(loose)
     keyed = [[] for _ in range(n)]               # first keys of each request's segments
     for run in [*per_run, loose]:
@@ -149,11 +148,10 @@ def _flatten(n, per_run, record, request, loose=(), width=None):
         if len(keys) <= 1:
             first.append(-1)
             continue
-        # partial slot of a segment = first slot of its request + its key-order rank (in units of width)
-        w = 1 if width is None else width(r)
+        # partial slot of a segment = first slot of its request + its key-order rank
         first.append(slot)
-        rank[r] = {k0: slot + w * i for i, k0 in enumerate(sorted(keys))}
-        slot += len(keys) * w
+        rank[r] = {k0: slot + i for i, k0 in enumerate(sorted(keys))}
+        slot += len(keys)
     out, ranges = [], [0]
     for run in per_run:
         for r, k0, k1 in run:
@@ -208,13 +206,16 @@ def _balanced_runs(key_lengths, groups, tile, seg_cost=0, weights=None, shares=N
         vbegin.append(vtotal)
         total += int(k)
         vtotal += seg_cost + w * int(k)
-    cuts, r = [0], 0
+    cuts, r, last = [0], 0, 0
     for w in range(1, groups):
         x = bound[w] * vtotal                         # cut in cost space
         while r + 1 < n and vbegin[r + 1] <= x:
             r += 1
-        into = int(max(0.0, (x - vbegin[r] - seg_cost) / wt[r]))   # keys of request r before the cut
-        cuts.append(max(cuts[-1], begin[r] + (min(into, int(key_lengths[r])) // tile) * tile))
+        into = int((x - vbegin[r] - seg_cost) / wt[r])             # keys of request r before the cut
+        at = begin[r] + (min(into, int(key_lengths[r])) // tile * tile if into > 0 else 0)
+        if at > last:
+            last = at
+        cuts.append(last)
     cuts.append(total)
     per_run = [[] for _ in range(groups)]
     w = 0
@@ -225,12 +226,14 @@ def _balanced_runs(key_lengths, groups, tile, seg_cost=0, weights=None, shares=N
         if kl == 0:
             per_run[w].append((r, 0, 0))
             continue
-        v = w
+        v, lo, end = w, a, a + kl
         while True:
-            lo, hi = max(cuts[v], a), min(cuts[v + 1], a + kl)
+            cut = cuts[v + 1]
+            hi = cut if cut < end else end
             if hi > lo:
                 per_run[v].append((r, lo - a, hi - a))
-            if cuts[v + 1] >= a + kl or v + 1 == groups:
+                lo = hi
+            if cut >= end or v + 1 == groups:
                 break
             v += 1
     return per_run
@@ -518,8 +521,10 @@ def _mixed_plan(tiled, query_lengths, key_lengths, starts, n_cu, causal, capacit
         # At most one workgroup per CU: the other slot is the prompts'.  63 requests of
         # 7 tokens (157,000 keys) beside 64 tokens over 8,000 keys, 16 / 24 / 32 / 48
         # / 64 runs: 168, 138, 131, 139, 136 us; beside 4 prompts of 1,500
-        # 184, 157, 169, 172, 181; alone 159, 123, 116, 127, 118.
-        groups = min(run_count(sum(keys), n_cu), per_head)
+        # 184, 157, 169, 172, 181; alone 159, 123, 116, 127, 118.  And runs of twice
+        # MIN_SEGMENT beside prompts: 6 requests with 4,700 keys beside 300 and 800
+        # tokens, 8 / 16 / 24 / 32 runs: 24.9, 23.8, 24.3, 26.3.
+        groups = min(run_count(sum(keys) // (2 if prompts else 1), n_cu), per_head)
         while pool is not None and groups > XCDS and min(len(units) + groups - 1, 2 * (groups - 1)) > pool:
             groups -= XCDS
         per_run = _balanced_runs(keys, groups, TILE, SEGMENT_COST,
@@ -535,26 +540,48 @@ def _mixed_plan(tiled, query_lengths, key_lengths, starts, n_cu, causal, capacit
             return None
     loose = prompt_segments([u[2] for u in prompts], [u[3] for u in prompts], cuts, n_cu, spare)
     n, every = len(units), units + prompts
-    out, n_seg, groups = _flatten(len(every), per_run,
-                                  lambda u, k0, k1, slot: (every[u][0], k0, k1, slot, *every[u][1:]),
-                                  lambda u, first, count: (first, count, *every[u][1:3]),
-                                  [(n + p, k0, k1) for p, k0, k1 in loose], lambda u: -(-every[u][2] // DECODE_TOKENS))
-    first = n_seg - len(loose)
+    segs = [x for run in per_run for x in run] + [(n + p, k0, k1) for p, k0, k1 in loose]
+    count = [0] * len(every)
+    for u, _, _ in segs:
+        count[u] += 1
+    width, first_slot, tiles = [-(-u[2] // DECODE_TOKENS) for u in every], [], 0
+    for c, w in zip(count, width):
+        first_slot.append(tiles if c > 1 else -1)
+        tiles += c * w if c > 1 else 0
+    out, requests, ranges, nxt = [], [], [0], list(first_slot)
+    if tiled:                            # a request's slots in key order, which balanced runs and prompts have
+        slot = {}
+        for seg in sorted(segs):
+            slot[seg] = nxt[seg[0]]
+            nxt[seg[0]] += width[seg[0]]
+    for seg in segs:
+        u, k0, k1 = seg
+        word, row, q, k, start = every[u]
+        if first_slot[u] < 0:
+            out += (word, k0, k1, -1, row, q, k, start)
+        elif tiled:
+            out += (word, k0, k1, slot[seg], row, q, k, start)
+        else:
+            out += (word, k0, k1, nxt[u], row, q, k, start)
+            nxt[u] += width[u]
+    for (_, row, q, _, _), f, c in zip(every, first_slot, count):
+        requests += (f if c > 1 else 0, c, row, q)
+    for run in per_run:
+        ranges.append(ranges[-1] + len(run))
+    groups, first = len(per_run), ranges[-1]
     columns = _prompt_columns(prompts, loose, first if capacity is None else capacity.run_records, causal)
     if capacity is None:
-        counts = out[-REQ_INTS * len(every) + 1::REQ_INTS]
-        tiles = sum(c * -(-u[2] // DECODE_TOKENS) for c, u in zip(counts, every) if c > 1)
-        return MixedPlan(out + columns, n_seg, groups, len(every), len(columns) // 2, tiles)
+        return MixedPlan(out + ranges + requests + columns, len(segs), groups, len(every), len(columns) // 2, tiles)
     c = capacity
     if (first > c.run_records or len(loose) > c.prompt_records or groups > c.runs or len(every) > c.requests
             or len(columns) > 2 * c.columns):
         return None
-    cut, ranges, n_work = WORK_INTS * first, WORK_INTS * n_seg, c.run_records + c.prompt_records
+    cut, n_work = WORK_INTS * first, c.run_records + c.prompt_records
     padded = np.zeros(mixed_ints(c), dtype=np.int32)
-    requests = WORK_INTS * n_work + c.runs + 1
-    for at, part in ((0, out[:cut]), (WORK_INTS * c.run_records, out[cut:ranges]),
-                     (WORK_INTS * n_work, out[ranges:ranges + groups + 1] + [first] * (c.runs - groups)),
-                     (requests, out[ranges + groups + 1:]), (requests + REQ_INTS * c.requests, columns)):
+    after = WORK_INTS * n_work + c.runs + 1
+    for at, part in ((0, out[:cut]), (WORK_INTS * c.run_records, out[cut:]),
+                     (WORK_INTS * n_work, ranges + [first] * (c.runs - groups)), (after, requests),
+                     (after + REQ_INTS * c.requests, columns)):
         padded[at:at + len(part)] = part
     return MixedPlan(padded, n_work, c.runs, c.requests, c.columns, c.tiles)
 
