@@ -534,7 +534,7 @@ def main():
             'bound': 'hbm', 'achieved': round(v_gbs, 1), 'peak': HBM_PEAK_GBS, 'unit': 'GB/s',
             'frac': round(v_gbs / HBM_PEAK_GBS, 4), 'traffic': traffic, 'traffic_per_algorithmic_byte': traffic_ratio,
             'traffic_round_algorithmic_bytes': traffic_round,
-            'kernel': 'fused verification attention: varlen_attn_kernel<true> + merge_kernel',
+            'kernel': 'fused verification attention: varlen_attn_kernel + merge_kernel',
             'avg_launch_ms': round(v_avg_ms, 5), 'algorithmic_bytes_per_launch': int(v_avg_bytes),
             'profiled': profiled,
         },
@@ -1628,7 +1628,8 @@ def mfma_probe(args):
          8192-row contexts, 8 blocks each, anchors evenly spread up to 8192;
       2. draft attention of the bench workload (1..8 blocks per request);
       3. the 9,840-row draft context projection of 5 layers: the fused
-         kernel, then the hipBLASLt GEMM + epilogue path.
+         kernel, the 128-token tiles (the path that length takes), then the
+         hipBLASLt GEMM + epilogue path.
     Pool and input contents are zero: MFMA work does not depend on them."""
     import numpy as np
     import torch
@@ -1670,7 +1671,7 @@ def mfma_probe(args):
         first += n
     records = upload(dev, rec)
     fc_out = torch.zeros(first, h, dtype=torch.bfloat16, device=dev)
-    for path in ('fused', 'gemm'):
+    for path in ('fused', 'wide', 'gemm'):
         for _ in range(3):
             proj.project_into(fc_out, records, n_req, keys, values, path=path)
         torch.cuda.synchronize()

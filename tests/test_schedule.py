@@ -289,7 +289,7 @@ def test_prompt_segments_follow_the_runs(ql, kl, split):
     """Requests with more than 8 query tokens: every key covered once by
     records of no run, after the runs' records, within the list's bound; the
     other requests stay in the runs; prompts are cut at whole 64-key stages
-    into parts of at least 1,024 keys (balanced), or at the chunk (request)."""
+    into parts of at least MIN_PROMPT_SEGMENT keys (balanced), or at the chunk (request)."""
     from qwen3_dspark_amd.schedule import MIN_PROMPT_SEGMENT, PROMPT_TOKENS, segment_plan
     n = len(ql)
     groups = run_count(sum(kl), 256, (max(ql) + 7) // 8)
