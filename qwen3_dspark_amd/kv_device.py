@@ -25,8 +25,8 @@ import torch
 from . import _native
 from ._device import KV_PAIR_SKEW, cu_count, kv_pair, require_gfx950, upload
 from .kernels import HEAD_DIM, KV_HEADS, SCALE
-from .schedule import (DECODE_TOKENS, PART_TILE_BYTES, REQ_INTS, TILED_TOKENS, WORK_INTS, mixed_capacity, mixed_ints, mixed_plan, run_count,
-                       segment_plan, varlen_list_bound)
+from .schedule import (DECODE_TOKENS, PART_TILE_BYTES, REQ_INTS, TILED_TOKENS, WORK_INTS, XCDS, mixed_capacity,
+                       mixed_ints, mixed_plan, run_count, segment_plan, varlen_list_bound)
 
 MAX_BUCKET_REQUESTS = 4096      # requests per transaction (one metadata workgroup scans them in LDS)
 
@@ -56,6 +56,20 @@ def _list_shape(shape, device, chunk, split):
         return c.run_records + c.prompt_records, c.runs
     return _list_counts(shape.request_count, shape.key_capacity, (shape.maximum_query_length + 7) // 8,
                         cu_count(device), None if split == 'balanced' else chunk)
+
+
+def _fitting_shape(shape, device, chunk, split, ints, tiles):
+    """_list_shape of a shape without mixed plans, with as many runs as a list of
+    `ints` int32 and `tiles` partial tiles hold: an arena is sized for its
+    families' longest request, whose lists have fewer runs than those of a
+    decoding family."""
+    records, runs = _list_shape(shape, device, chunk, split)
+    row_tiles = (shape.maximum_query_length + 7) // 8
+    while runs > XCDS and (WORK_INTS * records + runs + 1 + REQ_INTS * shape.request_count > ints
+                           or records * row_tiles > tiles):
+        runs -= XCDS
+        records = varlen_list_bound(shape.request_count, runs, shape.key_capacity, None if split == 'balanced' else chunk)
+    return records, runs
 
 
 def _list_ints(shape, device, chunk, split):
@@ -155,9 +169,10 @@ class HipKVDevice:
         MixedCapacity and MixedPlan without its list, or None and (records,
         runs).  They depend on the bucket and its buffers alone."""
         if ws.counts is None:
-            c = _mixed_shape(shape, self.device, self.split, ws.attn.numel() // PART_TILE_BYTES)
-            ws.counts = (c, self.launch_shape(shape) if c is None else
-                         (c.run_records + c.prompt_records, c.runs, c.requests, c.columns, c.tiles))
+            tiles = ws.attn.numel() // PART_TILE_BYTES
+            c = _mixed_shape(shape, self.device, self.split, tiles)
+            ws.counts = (c, _fitting_shape(shape, self.device, self.chunk, self.split, ws.work.numel(), tiles)
+                         if c is None else (c.run_records + c.prompt_records, c.runs, c.requests, c.columns, c.tiles))
         return ws.counts
 
     # -- workspaces -----------------------------------------------------------
@@ -217,7 +232,7 @@ class HipKVDevice:
             records = mixed_plan(query_lengths, key_lengths, slots, n_cu, capacity=capacity, xcd_speed=self.xcd_speed,
                                  slot_balance=self.slot_balance).records
         else:
-            runs = run_count(sum(key_lengths), n_cu, (shape.maximum_query_length + 7) // 8)
+            runs = min(run_count(sum(key_lengths), n_cu, (shape.maximum_query_length + 7) // 8), counts[1])
             records, _, _ = segment_plan(self.split, query_lengths, key_lengths, slots, runs, self.chunk, counts,
                                          xcd_speed=self.xcd_speed, n_cu=n_cu if self.slot_balance else None)
         if len(records) > ws.work.numel():

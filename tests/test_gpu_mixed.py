@@ -95,3 +95,31 @@ def test_families_of_one_arena():
                                     [h.index for h in handles], ctx, cu_q, scale=SCALE)
         attention_gate(f64(out), ref, segments(cu_q))
         store.abort(tx)
+
+
+@pytest.mark.parametrize('split', ['balanced', 'request'])
+def test_a_decoding_family_in_an_arena_of_fewer_partials(split):
+    """Four decoding requests beside a family of 40 tokens at most: a list of
+    their own would have more runs than the arena's partials hold."""
+    from qwen3_dspark_amd.persistent_kv import PersistentTargetKV, QueryFamily
+    gen = torch.Generator().manual_seed(SEED)
+    store = PersistentTargetKV(layers=1, slots=4, context_capacity=6000, max_query_tokens=78, heads=8, dim=128,
+                               device=DEV, split=split)
+    handles = [store.add_request(f'r{i}') for i in range(4)]
+    ctx = [5900, 5800, 5700, 5500]
+    for h, c in zip(handles, ctx):
+        kv = randn_bf16(gen, 2, 1, c, 8, 128).to(DEV)
+        store.load_prefix(h, kv[0], kv[1])
+    small = QueryFamily(4, 19, 8, 22958, 6000, 'decoding')
+    large = QueryFamily(4, 78, 40, 22978, 6000, 'with prompts')
+    store.register_families((small, large))
+    for family, ql in ((small, (7, 1, 8, 3)), (large, (7, 40, 9, 22)), (small, (4, 5, 5, 5))):
+        rows = sum(ql)
+        q, nk, nv = (randn_bf16(gen, rows, h, 128).to(DEV) for h in (16, 8, 8))
+        tx = store.begin(handles, family, query_lengths=ql)
+        out = store.attend(tx, 0, q, keys=nk, values=nv)
+        cu_q = [sum(ql[:i]) for i in range(5)]
+        ref = cref.verify_attention(bits(q), bits(store.keys[0]), bits(store.values[0]), bits(nk), bits(nv),
+                                    [h.index for h in handles], ctx, cu_q, scale=SCALE)
+        attention_gate(f64(out), ref, segments(cu_q))
+        store.abort(tx)

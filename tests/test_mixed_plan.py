@@ -148,3 +148,44 @@ def test_a_short_chunk_over_a_long_context_is_spread(tokens, keys):
     for cap in (None, mixed_capacity(1, tokens, kl[0], tokens, N_CU)):
         busy, prompts = check(ql, kl, [0], mixed_plan(ql, kl, [0], N_CU, capacity=cap))
         assert (busy if not prompts else sum(prompts.values())) >= min(14, -(-keys // 256))
+
+
+@pytest.mark.parametrize('split', ['balanced', 'request'])
+def test_lists_of_the_families_of_one_arena(split, monkeypatch):
+    """An arena takes the elementwise maximum of its families' shapes, whose lists
+    have fewer runs where a request is long: every family's lists and partials
+    still fit, with as many runs as a list of its own wherever those do."""
+    from types import SimpleNamespace
+    from qwen3_dspark_amd import kv_device as kd
+    monkeypatch.setattr(kd, 'cu_count', lambda device: N_CU)
+    rng = np.random.default_rng(3)
+    fields = ('request_count', 'query_tokens', 'key_capacity', 'maximum_query_length')
+    first = [[(4, 19, 22958, 8), (4, 78, 22958, 40)], [(3, 19, 11732, 8), (3, 40, 11732, 40)],
+             [(1, 7, 16000, 7), (1, 9, 16000, 9)], [(128, 128, 1 << 20, 1), (1, 17, 17, 17)]]
+    for i in range(3000):
+        if i < len(first):
+            arena = first[i]
+        else:
+            arena = []
+            for _ in range(int(rng.integers(1, 4))):
+                n, longest = int(rng.choice([1, 2, 3, 8, 33, 128])), int(rng.choice([1, 7, 8, 9, 17, 40, 97, 1000]))
+                q = int(rng.integers(max(n, longest), n * longest + 1)) if n * longest > n + longest else n * longest
+                arena.append((n, q, q + int(rng.integers(0, n * 8000)), longest))
+        arena = [SimpleNamespace(**dict(zip(fields, f))) for f in arena]
+        top = SimpleNamespace(**{name: max(getattr(f, name) for f in arena) for name in fields})
+        mixed = kd._mixed_shape(top, None, split)
+        tiles = (mixed.tiles if mixed is not None else
+                 kd._list_shape(top, None, 512, split)[0] * -(-top.maximum_query_length // 8))
+        ints = kd._list_ints(top, None, 512, split)
+        for f in arena:
+            c = kd._mixed_shape(f, None, split, tiles)
+            if c is not None:
+                assert mixed_ints(c) <= ints and c.tiles <= tiles
+                continue
+            records, runs = kd._fitting_shape(f, None, 512, split, ints, tiles)
+            assert runs >= 8 and runs % 8 == 0
+            size = 8 * records + runs + 1 + 4 * f.request_count
+            width = -(-f.maximum_query_length // 8)
+            assert size <= ints and records * width <= tiles
+            own = kd._list_shape(f, None, 512, split)
+            assert (records, runs) == own or 8 * own[0] + own[1] + 1 + 4 * f.request_count > ints or own[0] * width > tiles
