@@ -16,8 +16,8 @@ import torch
 
 from . import _native, backends
 from ._device import Workspace, cu_count, require_gfx950
-from .schedule import (DECODE_TOKENS, DEFAULT_CHUNK, PART_TILE_BYTES, SPLITS, mixed_plan, run_count, segment_plan,
-                       upload_work)
+from .schedule import (DECODE_TOKENS, DEFAULT_CHUNK, PART_TILE_BYTES, SPLITS, check_chunk, mixed_plan, run_count,
+                       segment_plan, upload_work)
 
 Q_HEADS, KV_HEADS, HEAD_DIM = 16, 8, 128
 SCALE = 128 ** -0.5
@@ -121,6 +121,7 @@ class HipVarlenKernel:
         listed = self._work_list(layout, tiles) or (None, 0, 0)
         if len(listed) > 3:
             work, n_work, runs, records, columns, tiles = listed
+            check_chunk(self.chunk)
             ws = self._workspace.get(PART_TILE_BYTES * tiles)
             _native.call('dspark_mixed_attn_fwd', query.data_ptr(), key.data_ptr(), value.data_ptr(), None, None, None,
                          None, records, 0, 0, 0, max_q, int(self.causal), SCALE, work.data_ptr(), n_work, runs,

@@ -25,8 +25,8 @@ import torch
 from . import _native
 from ._device import KV_PAIR_SKEW, cu_count, kv_pair, require_gfx950, upload
 from .kernels import HEAD_DIM, KV_HEADS, SCALE
-from .schedule import (DECODE_TOKENS, PART_TILE_BYTES, REQ_INTS, TILED_TOKENS, WORK_INTS, XCDS, mixed_capacity,
-                       mixed_ints, mixed_plan, run_count, segment_plan, varlen_list_bound)
+from .schedule import (DECODE_TOKENS, PART_TILE_BYTES, REQ_INTS, TILED_TOKENS, WORK_INTS, XCDS, check_chunk,
+                       mixed_capacity, mixed_ints, mixed_plan, run_count, segment_plan, varlen_list_bound)
 
 MAX_BUCKET_REQUESTS = 4096      # requests per transaction (one metadata workgroup scans them in LDS)
 
@@ -68,7 +68,8 @@ def _fitting_shape(shape, device, chunk, split, ints, tiles):
     while runs > XCDS and (WORK_INTS * records + runs + 1 + REQ_INTS * shape.request_count > ints
                            or records * row_tiles > tiles):
         runs -= XCDS
-        records = varlen_list_bound(shape.request_count, runs, shape.key_capacity, None if split == 'balanced' else chunk)
+        records = varlen_list_bound(shape.request_count, runs, shape.key_capacity,
+                                    None if split == 'balanced' else chunk)
     return records, runs
 
 
@@ -272,6 +273,7 @@ class HipKVDevice:
         k, v, sk, sv = self.layer_pointers[layer]
         capacity, counts = self.list_counts(ws, shape)
         if capacity is not None:
+            check_chunk(self.chunk)
             n_work, runs, requests, columns, tiles = counts
             new = (sk, sv, None, None) if keys is None else (keys, values, sk, sv)
             _native.call('dspark_mixed_attn_fwd', query, k, v, *new, requests, KV_HEADS * C * HEAD_DIM, HEAD_DIM,

@@ -94,6 +94,12 @@ MixedCapacity = namedtuple('MixedCapacity', 'run_records prompt_records runs req
 MixedPlan = namedtuple('MixedPlan', 'records n_work runs requests columns tiles')
 
 
+def check_chunk(chunk):
+    """Refuses what the attention entry points refuse: the mixed one takes no chunk."""
+    if chunk < TILE or chunk % TILE or chunk > 1 << 20:
+        raise ValueError(f'chunk must be a multiple of {TILE} in [{TILE}, 2^20] (got {chunk})')
+
+
 def n_chunks(n, chunk):
     return max(1, -(-int(n) // chunk))
 

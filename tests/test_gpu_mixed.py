@@ -123,3 +123,21 @@ def test_a_decoding_family_in_an_arena_of_fewer_partials(split):
                                     [h.index for h in handles], ctx, cu_q, scale=SCALE)
         attention_gate(f64(out), ref, segments(cu_q))
         store.abort(tx)
+
+
+@pytest.mark.parametrize('chunk', [0, 33, 1 << 21])
+@pytest.mark.parametrize('tokens', [5, 40])
+def test_a_chunk_that_the_other_calls_refuse(chunk, tokens):
+    """Refused on the host whatever the plan, packed and from the store."""
+    from qwen3_dspark_amd.kernels import HipVarlenKernel
+    from qwen3_dspark_amd.persistent_kv import Bucket, PersistentTargetKV
+    layout, q, k, v = layout_of([tokens], [tokens])
+    with pytest.raises((ValueError, RuntimeError)):
+        HipVarlenKernel(DEV, chunk=chunk)(q.to(DEV), k.to(DEV), v.to(DEV), layout, scale=SCALE)
+    store = PersistentTargetKV(layers=1, slots=1, context_capacity=128, max_query_tokens=64, heads=8, dim=128,
+                               device=DEV, chunk=chunk)
+    bucket = Bucket((tokens,), (64,), 'chunk')
+    store.register_bucket(bucket)
+    tx = store.begin([store.add_request('r')], bucket, query_lengths=(tokens,))
+    with pytest.raises((ValueError, RuntimeError)):
+        store.attend(tx, 0, q.to(DEV), keys=k.to(DEV), values=v.to(DEV))

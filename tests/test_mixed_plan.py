@@ -8,8 +8,8 @@ spread over the CUs."""
 import numpy as np
 import pytest
 
-from qwen3_dspark_amd.schedule import (DECODE_TOKENS, PART_TILE_BYTES, REQ_INTS, WORK_INTS, mixed_capacity, mixed_ints, mixed_plan,
-                                       run_count)
+from qwen3_dspark_amd.schedule import (DECODE_TOKENS, PART_TILE_BYTES, REQ_INTS, WORK_INTS, mixed_capacity,
+                                       mixed_ints, mixed_plan, run_count)
 
 N_CU = 256
 
@@ -188,4 +188,5 @@ def test_lists_of_the_families_of_one_arena(split, monkeypatch):
             width = -(-f.maximum_query_length // 8)
             assert size <= ints and records * width <= tiles
             own = kd._list_shape(f, None, 512, split)
-            assert (records, runs) == own or 8 * own[0] + own[1] + 1 + 4 * f.request_count > ints or own[0] * width > tiles
+            own_size = 8 * own[0] + own[1] + 1 + 4 * f.request_count
+            assert (records, runs) == own or own_size > ints or own[0] * width > tiles
