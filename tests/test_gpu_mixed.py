@@ -141,3 +141,46 @@ def test_a_chunk_that_the_other_calls_refuse(chunk, tokens):
     tx = store.begin([store.add_request('r')], bucket, query_lengths=(tokens,))
     with pytest.raises((ValueError, RuntimeError)):
         store.attend(tx, 0, q.to(DEV), keys=k.to(DEV), values=v.to(DEV))
+
+
+@pytest.mark.parametrize('split', ['balanced', 'request'])
+def test_captured_rounds_with_prompts(split):
+    """One captured program for a bucket of prompts and short requests, replayed
+    over contexts that change which of them are cut or attended by row tiles: every
+    replay equals the eager call."""
+    from qwen3_dspark_amd.graph import VerificationGraph
+    from qwen3_dspark_amd.persistent_kv import Bucket, PersistentTargetKV
+    gen = torch.Generator().manual_seed(SEED)
+    ql, ceiling = (7, 64, 9, 200), 6000
+    rows = sum(ql)
+    store = PersistentTargetKV(layers=2, slots=8, context_capacity=6400, max_query_tokens=rows, heads=8, dim=128,
+                               device=DEV, split=split)
+    contexts = (0, 300, 20, 5900, 700, 2500, 64, 4000)
+    handles = [store.add_request(f'r{i}') for i in range(8)]
+    for h, c in zip(handles, contexts):
+        if c:
+            kv = randn_bf16(gen, 2, 2, c, 8, 128).to(DEV)
+            store.load_prefix(h, kv[0], kv[1])
+    bucket = Bucket(ql, (ceiling,) * 4, 'captured prompts')
+    store.register_bucket(bucket)
+    graph = VerificationGraph(store, bucket).capture()
+    cu_q = [sum(ql[:i]) for i in range(5)]
+    for chosen in ((0, 1, 2, 6), (3, 5, 7, 4), (1, 0, 3, 6), (7, 2, 5, 3), (0, 1, 2, 6)):
+        some = [handles[i] for i in chosen]
+        ctx = [store.length(h) for h in some]
+        print(f'[mixed] captured split={split} ctx={ctx}', flush=True)
+        q, nk, nv = (randn_bf16(gen, 2, rows, h, 128).to(DEV) for h in (16, 8, 8))
+        tx = store.begin(some, bucket)
+        eager = [store.attend(tx, l, q[l], keys=nk[l], values=nv[l]) for l in range(2)]
+        store.abort(tx)
+        torch.cuda.synchronize()
+        tx = store.begin(some, bucket)
+        graph.query.copy_(q)
+        graph.keys.copy_(nk)
+        graph.values.copy_(nv)
+        out = graph.wait(graph.submit(tx))
+        assert all(torch.equal(out[l], eager[l]) for l in range(2))
+        ref = cref.verify_attention(bits(q[1]), bits(store.keys[1]), bits(store.values[1]), bits(nk[1]), bits(nv[1]),
+                                    [h.index for h in some], ctx, cu_q, scale=SCALE)
+        attention_gate(f64(out[1]), ref, segments(cu_q))
+        store.commit(tx, {h: min(n, 5) for h, n in zip(some, ql)})
